@@ -239,7 +239,7 @@ int svo_march_beam(svo_ctx *ctx, const svo_octree *oct, const svo_camera *cam, u
  * same kernels, with the beam image kept in a static device array of 2^20 cells (4 MiB per device,
  * held until the process ends) instead of pool memory: frames need (ceil(W/8)+1)*(ceil(H/8)+1) <=
  * 1048576 beam cells (up to 7680x4320, for example); larger frames return SVO_ERR_INVALID_ARGUMENT.
- * The launch schedule is fixed (svo_march_mode's, else one ray per lane in 16x16 tiles; the autotuner
+ * The launch schedule is fixed (svo_march_mode's, else one ray per lane in 8x8 tiles; the autotuner
  * is not consulted) and no stage timer runs.  With the profiler off (svo_prof_enable) it calls no
  * allocating routine.  Every call on one device shares the array, which keeps the last call's beam
  * image: calls that overlap on one GPU, from any context, race; serialise them. */
@@ -274,7 +274,7 @@ int svo_march_plan_create(svo_ctx *ctx, const svo_octree *const *octs, const svo
 int svo_march_plan_set_cameras(svo_ctx *ctx, svo_march_plan *plan, const svo_camera *cams);
 int svo_march_plan_use_graph(svo_march_plan *plan, int on);
 /* Workgroup tile of the march launch: 0 = 16x16 pixels (4 waves), 1 = 8x8 (1 wave), 2 = 16x8,
- * 3 = 32x8; -1 = the default, or the autotuner's choice when svo_autotune is on. */
+ * 3 = 32x8; -1 = the default (8x8), or the autotuner's choice when svo_autotune is on. */
 int svo_march_plan_set_shape(svo_march_plan *plan, int shape);
 int svo_march_plan_run(svo_ctx *ctx, svo_march_plan *plan, svo_hit *hits_dev);
 int svo_march_plan_destroy(svo_march_plan *plan);
@@ -290,8 +290,8 @@ int svo_autotune(svo_ctx *ctx, int on);
  * 1 = a fixed grid of waves whose lanes take a new ray as soon as theirs has ended (rays dealt to
  * the waves in 64-ray chunks; wins when ray lengths diverge); 0 = one ray per lane (wins
  * for coherent rays), frames in 16x16-pixel blocks; 2 = as 0 with one-wave 8x8-pixel blocks for
- * frames; -1 (default) = chosen per shape class by the autotuner when svo_autotune is on, else 0.
- * Results are identical. */
+ * frames; -1 (default) = chosen per shape class by the autotuner when svo_autotune is on, else 2 for
+ * frames and 0 for rays.  Results are identical. */
 int svo_march_mode(svo_ctx *ctx, int mode);
 int svo_autotune_report(svo_ctx *ctx, char *buf, uint64_t cap, uint64_t *len);
 

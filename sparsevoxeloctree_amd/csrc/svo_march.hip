@@ -394,8 +394,19 @@ __device__ __forceinline__ f3 gen_ray(const CamArgs &c, float cx, float cy) {
 	return normalize3(v);
 }
 
-// Linear block id -> tile so that the blocks one XCD receives (ids b, b+8, b+16, ...) cover one
-// contiguous band of the frame and share its octree working set in that XCD's L2.
+// Linear block id b of n -> item (a tile of a frame, a chunk of rays).  The hardware deals blocks to the
+// 8 XCDs in turn; here groups of kGroup consecutive items go to the XCDs in turn.  The blocks of a
+// group share one XCD's L2, and every XCD works on all parts of the range.
+template <uint32_t kGroup> __device__ __forceinline__ uint32_t xcd_stripes(uint32_t b, uint32_t n) {
+	if (b >= n / (8u * kGroup) * (8u * kGroup))
+		return b; // the last, partial round
+	const uint32_t k = b >> 3;
+	return (k / kGroup * 8u + (b & 7u)) * kGroup + k % kGroup;
+}
+// The same with one contiguous band of the range per XCD: less of the octree is read by two XCDs, but
+// XCDs with a cheap band idle.  8x8-tile marches, bands -> stripes of 64 tiles: 3840x2160 over slivers at
+// 2^12 3950 -> 2890 us, 1920x1080 over spheres at 2^10 157 -> 133 us, 2560x1440 in the room at 2^11
+// 196 -> 111 us, but 1920x1080 in the room at 2^10 127 -> 137 us (stripes of 1..64 tiles within 3%).
 __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nblocks) {
 	const uint32_t per = (nblocks + 7u) / 8u;
 	const uint32_t full = nblocks - (per - 1u) * 8u; // XCDs that get `per` blocks
@@ -503,15 +514,16 @@ __global__ void __launch_bounds__(64)
 		atomicOr(err_out, err);
 }
 
-// (8 WX) x (8 WY)-pixel tile per block, one 8x8 quad per wave, XCD-banded tile order.
-template <uint32_t WX, uint32_t WY>
+// (8 WX) x (8 WY)-pixel tile per block, one 8x8 quad per wave.
+template <uint32_t WX, uint32_t WY, bool kBands>
 __global__ void __launch_bounds__(64 * WX * WY)
     march_frame_kernel(const uint32_t *__restrict__ oct, uint64_t W, CamArgs cam, uint32_t width, uint32_t height,
                        const float *__restrict__ beam, uint32_t bw, uint32_t tiles_x, uint4 *__restrict__ hits,
                        uint32_t *err_out) {
 	constexpr uint32_t kT = 64 * WX * WY;
 	__shared__ uint32_t s_stack[kStackSlots * kT];
-	const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+	const uint32_t tile =
+	    kBands ? xcd_tile(blockIdx.x, gridDim.x) : xcd_stripes<64u / (WX * WY)>(blockIdx.x, gridDim.x);
 	const uint32_t tx = tile % tiles_x, ty = tile / tiles_x;
 	const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
 	const uint32_t px = tx * (8u * WX) + (wave % WX) * 8u + (lane & 7u);
@@ -546,8 +558,9 @@ __global__ void __launch_bounds__(kBlock)
 		atomicOr(err_out, err);
 }
 
-// Frames of S scenes: (8 WX) x (8 WY)-pixel tiles, one 8x8 quad per wave; the tiles of all scenes
-// form one XCD-banded sequence, so an XCD works on few scenes at a time.
+// Frames of S scenes: (8 WX) x (8 WY)-pixel tiles, one 8x8 quad per wave; the tiles of all scenes form
+// one sequence, dealt to the XCDs in stripes (bands gave each XCD whole scenes, of different cost: 32
+// 256x256 frames 255 -> 234 us in 16x16 tiles, 241 -> 208 us in 8x8 tiles).
 template <uint32_t WX, uint32_t WY>
 __global__ void __launch_bounds__(64 * WX * WY)
     march_frame_batch(const MarchSeg *__restrict__ segs, uint32_t width, uint32_t height,
@@ -555,7 +568,7 @@ __global__ void __launch_bounds__(64 * WX * WY)
                       uint32_t tiles_per_scene, uint4 *__restrict__ hits, uint32_t *err_out) {
 	constexpr uint32_t kT = 64 * WX * WY;
 	__shared__ uint32_t s_stack[kStackSlots * kT];
-	const uint32_t tile_g = xcd_tile(blockIdx.x, gridDim.x);
+	const uint32_t tile_g = xcd_stripes<64u / (WX * WY)>(blockIdx.x, gridDim.x);
 	const uint32_t s = tile_g / tiles_per_scene, tile = tile_g % tiles_per_scene;
 	const uint32_t tx = tile % tiles_x, ty = tile / tiles_x;
 	const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
@@ -1527,7 +1540,8 @@ int tune(svo_ctx *ctx, const std::string &key, int nshapes, const char *const *n
 	return SVO_OK;
 }
 
-const char *const kScheduleName[3] = {"one-ray-per-lane", "persistent-refill", "one-ray-per-lane-8x8"};
+const char *const kScheduleName[4] = {"one-ray-per-lane", "persistent-refill", "one-ray-per-lane-8x8",
+                                      "one-ray-per-lane-8x8-bands"};
 
 // Persistent march of n rays from src; name is the profiler's name of the march.
 template <int kVariant, class Src>
@@ -1574,7 +1588,7 @@ namespace {
 
 // The primary march of a frame (and its beam pre-pass when beam_img is not null, written there).
 // may_tune: the autotuner may time the candidate schedules of a new shape class; without it the
-// schedule is the context's fixed one, or one ray per lane in 16x16 tiles.  timed: bracket the
+// schedule is the context's fixed one, or one ray per lane in 8x8 tiles.  timed: bracket the
 // passes with the context's stage timers.
 int march_frame_into(svo_ctx *ctx, const svo_octree *oct, const svo_camera *cam, uint32_t w, uint32_t h,
                      float *beam_img, svo_hit *hits, bool may_tune, bool timed = true) {
@@ -1587,8 +1601,8 @@ int march_frame_into(svo_ctx *ctx, const svo_octree *oct, const svo_camera *cam,
 		if (rc)
 			return rc;
 	}
-	// schedules: 0 = one ray per lane in 16x16 tiles, 1 = persistent refill, 2 = one ray per lane in
-	// one-wave 8x8 tiles
+	// schedules: 0 = one ray per lane in 16x16 tiles, 1 = persistent refill, 2 = one ray per lane in one-wave
+	// 8x8 tiles, 3 = as 2 with one band of the frame per XCD (the autotuner's only)
 	auto run = [&](int mode) -> hipError_t {
 		if (mode == 1) {
 			const uint32_t tx8 = (w + 7u) / 8u, ty8 = (h + 7u) / 8u;
@@ -1596,23 +1610,24 @@ int march_frame_into(svo_ctx *ctx, const svo_octree *oct, const svo_camera *cam,
 			              reinterpret_cast<uint4 *>(hits)};
 			return launch_persist<0>(ctx, "march_frame", src, (uint64_t)tx8 * ty8 * 64u);
 		}
-		const uint32_t WX = mode == 0 ? 2u : 1u, WY = mode == 0 ? 2u : 1u; // 16x16 or 8x8 tiles
-		const uint32_t tiles_x = (w + 8u * WX - 1u) / (8u * WX), tiles_y = (h + 8u * WY - 1u) / (8u * WY);
-		if (mode == 0)
-			return launch(ctx, "march_frame", march_frame_kernel<2, 2>, dim3(tiles_x * tiles_y), dim3(256), 0,
-			              (const uint32_t *)oct->words, oct->W, ca, w, h, (const float *)beam_img, bw, tiles_x,
-			              reinterpret_cast<uint4 *>(hits), ctx->d_err);
-		return launch(ctx, "march_frame", march_frame_kernel<1, 1>, dim3(tiles_x * tiles_y), dim3(64), 0,
-		              (const uint32_t *)oct->words, oct->W, ca, w, h, (const float *)beam_img, bw, tiles_x,
-		              reinterpret_cast<uint4 *>(hits), ctx->d_err);
+		const uint32_t edge = mode == 0 ? 16u : 8u; // pixels
+		const uint32_t tiles_x = (w + edge - 1u) / edge, tiles_y = (h + edge - 1u) / edge;
+		return launch(ctx, "march_frame",
+		              mode == 0   ? march_frame_kernel<2, 2, false>
+		              : mode == 2 ? march_frame_kernel<1, 1, false>
+		                          : march_frame_kernel<1, 1, true>,
+		              dim3(tiles_x * tiles_y), dim3(mode == 0 ? 256 : 64), 0, (const uint32_t *)oct->words, oct->W, ca,
+		              w, h, (const float *)beam_img, bw, tiles_x, reinterpret_cast<uint4 *>(hits), ctx->d_err);
 	};
 	int mode = ctx->march_mode;
 	if (mode < 0) {
-		mode = 0;
+		// one-wave tiles: a tile's wave ends with its own longest ray (512x512 57 -> 49 us, 3840x2160 over
+		// slivers 2960 -> 2890 us against 16x16 tiles, at no size slower)
+		mode = 2;
 		if (ctx->autotune && may_tune) {
 			char key[96];
 			std::snprintf(key, sizeof key, "march_frame %ux%u level=%u beam=%d", w, h, oct->level, beam ? 1 : 0);
-			const int rc = tune(ctx, key, 3, kScheduleName, run, mode);
+			const int rc = tune(ctx, key, 4, kScheduleName, run, mode);
 			if (rc)
 				return rc;
 		}
@@ -1952,7 +1967,7 @@ int march_plan_run(svo_ctx *ctx, MarchPlan *p, svo_hit *hits) {
 	if (p->S == 0 || p->width == 0 || p->height == 0)
 		return SVO_OK;
 	if (p->shape < 0) {
-		p->shape = 0;
+		p->shape = 1;
 		if (ctx->autotune) {
 			char key[96];
 			std::snprintf(key, sizeof key, "march_frame_batch S=%u %ux%u beam=%d", p->S, p->width, p->height, p->beam);

@@ -3,7 +3,6 @@ octrees at the line between the two, against the oracle, on every schedule.
 
 Reference: shader/octree.glsl:47-177,179-340,342-629.  Records are bit-exact, so no tolerance.
 """
-import ctypes as C
 import math
 
 import numpy as np
@@ -150,3 +149,41 @@ def test_malformed_octrees_raise_error_bits(ctx, words, bit):
     for other in got[1:]:
         ok, msg = hits_equal(other, got[0])
         assert ok, msg
+
+
+@pytest.mark.parametrize("W,H", [(8, 8), (176, 184), (184, 184), (256, 128), (203, 331), (520, 505)])
+def test_frame_tiles_cover_every_pixel(ctx, no_device_errors, W, H):
+    # tile counts below, at and above whole rounds of the dealing to the XCDs (512 one-wave tiles,
+    # 128 16x16 tiles), with partial tiles, in every one-ray-per-lane schedule
+    import sparsevoxeloctree_amd as S
+    from sparsevoxeloctree_amd._capi import lib, ptr
+
+    blank = np.zeros(3 * W * H * 8, np.uint32)
+    words = scene_words(ctx)
+    octree = S.Octree.FromWords(ctx, words, 6)
+    cam = S.camera_look_at((2.3, 2.0, 0.8), (1.5, 1.5, 1.5), aspect=W / H)
+    beam, _ = oracle.beam(words, 6, cam.uniform_array(), W, H)
+    ref = oracle.march_frame(words, 6, cam.uniform_array(), W, H, beam)
+    print("frame tiles", W, H, flush=True)
+    for mode in (0, 1, 2):
+        ctx.check(lib.svo_march_mode(ctx.h, mode))
+        try:
+            t = S.OctreeTracer.Create(octree, cam)
+            t.Resize(W, H)
+            t._ensure()
+            ctx.check(lib.svo_upload(ctx.h, t.hits.ptr, ptr(blank), W * H * 32))
+            t.CmdDrawPipeline()
+            ok, msg = hits_equal(t.GetHits(), ref)
+        finally:
+            ctx.check(lib.svo_march_mode(ctx.h, -1))
+        assert ok, "mode %d: %s" % (mode, msg)
+    for shape in (0, 1, 2, 3):
+        plan = S.MarchPlan([octree] * 3, [cam] * 3, W, H)
+        plan.set_shape(shape)
+        hits = plan.alloc_hits()
+        ctx.check(lib.svo_upload(ctx.h, hits.ptr, ptr(blank), 3 * W * H * 32))
+        plan.run(hits)
+        got = hits.download(S.HIT_DTYPE, 3 * W * H).reshape(3, H, W)
+        for k in range(3):
+            ok, msg = hits_equal(got[k], ref)
+            assert ok, "shape %d frame %d: %s" % (shape, k, msg)
