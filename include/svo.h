@@ -287,8 +287,8 @@ int svo_march_rays_batch(svo_ctx *ctx, const svo_octree *const *octs, uint32_t n
  * candidate workgroup/tile shape once and keeps the fastest; the report lists the decisions. */
 int svo_autotune(svo_ctx *ctx, int on);
 /* Schedule of svo_march, svo_march_rays, svo_march_rays_batch and the server's ray batches:
- * 1 = a fixed grid of waves whose lanes take a new ray as soon as theirs has ended (rays dealt to
- * the waves in 64-ray chunks; wins when ray lengths diverge); 0 = one ray per lane (wins
+ * 1 = refill: lanes take a new ray from their block's pool when theirs has ended (wins when ray
+ * lengths diverge); 0 = one ray per lane (wins
  * for coherent rays), frames in 16x16-pixel blocks; 2 = as 0 with one-wave 8x8-pixel blocks for
  * frames; -1 (default) = chosen per shape class by the autotuner when svo_autotune is on, else 2 for
  * frames and 0 for rays.  Results are identical. */

@@ -631,61 +631,76 @@ __global__ void __launch_bounds__(kBlock)
 		atomicOr(err_out, err);
 }
 
-// ---- persistent march with per-lane ray refill ------------------------------------------------
+// ---- marches with per-lane ray refill --------------------------------------------------------------
 // Rays of one march diverge: a wave lasts as long as its longest ray while finished lanes idle.
-// Here a fixed grid of waves marches all rays; a lane whose ray has ended writes its record and,
-// once kRefill lanes of the wave are idle, they take the next rays of the wave's pool.  The rays
-// are dealt to the waves in chunks of 64 (an 8x8-pixel tile of a frame), chunk c to wave
-// c mod (number of waves), so costly image regions spread over all waves and no atomics are
-// needed.  Every ray runs the same per-ray arithmetic as the one-ray-per-lane kernels, so the
-// records are identical; only which lane marches which ray changes.
-// A refill costs a ray set-up for the whole wave, so checks are spaced: 16 idle lanes and 16 trips
-// between checks measured best (4 or 8 trips: 4-8% slower; 32 trips or 32 lanes: slower again).
+// Here a block of 4 waves owns a pool of kPool rays; a lane whose ray has ended writes its record and,
+// once kRefill lanes of its wave are idle (looked at every kTrips trips), they take the next rays of
+// the block's pool (one LDS atomic).  The hardware deals the blocks, so no CU waits for another's
+// share.  What the record needs of the ray waits in LDS, and rays for the general loop are marked and
+// marched one per lane after the pool: 52 VGPRs, 8 waves per SIMD.  Every ray runs the same per-ray
+// arithmetic as the one-ray-per-lane kernels, so the records are identical.
+// 2M bounce rays in the room at 2^10: 250 us, against 380 one ray per lane and 283 with a grid that just
+// fills the GPU and a fixed share of the rays per wave (80 VGPRs); pools of 512 / 2048 rays 302 / 278,
+// 8 / 32 trips 265 / 280, 8 / 32 idle lanes 252 / 264.  Frames gain nothing from refills (a bigger pool
+// only lowers the number of waves): 256 rays, i.e. a 16x16 tile, 1920x1080 150 us.
 constexpr uint32_t kRefill = 16; // idle lanes that trigger a refill
-constexpr uint32_t kTrips = 16;  // loop trips between refill checks
-constexpr uint32_t kChunk = 64;  // rays per chunk
 
-// Ray sources: ray(k, ...) sets up ray k (false: no ray, e.g. a pixel outside the frame) and the
-// address of its 32-byte record.
-struct FrameRays { // primary rays of one frame, numbered in 8x8-pixel tiles
+// Ray sources: ray(k, ...) sets up ray k (false: no ray, e.g. a pixel outside the frame), out(k) is
+// the address of its 32-byte record.
+struct FrameRays { // primary rays of one frame, numbered in 32x32-pixel regions of 8x8 tiles in Z order
+	static constexpr bool kOneOctree = true;
+	static constexpr uint32_t kPool = 256, kTrips = 32;
 	const uint32_t *oct;
 	uint64_t W;
 	CamArgs cam;
-	uint32_t width, height, bw, tiles_x;
+	uint32_t width, height, bw, regions_x;
 	const float *beam;
 	uint4 *hits;
-	__device__ bool ray(uint64_t k, f3 &o, f3 &d, const uint32_t *&oc, uint64_t &w, uint4 *&out) const {
-		const uint32_t tile = (uint32_t)(k >> 6), q = (uint32_t)k & 63u;
-		const uint32_t px = (tile % tiles_x) * 8u + (q & 7u), py = (tile / tiles_x) * 8u + (q >> 3);
+	__device__ void pixel(uint64_t k, uint32_t &px, uint32_t &py) const {
+		const uint32_t region = (uint32_t)(k >> 10), t = (uint32_t)(k >> 6) & 15u, q = (uint32_t)k & 63u;
+		px = (region % regions_x) * 32u + ((t & 1u) | (t >> 1 & 2u)) * 8u + (q & 7u);
+		py = (region / regions_x) * 32u + ((t >> 1 & 1u) | (t >> 2 & 2u)) * 8u + (q >> 3);
+	}
+	__device__ bool ray(uint64_t k, f3 &o, f3 &d, const uint32_t *&oc, uint64_t &w) const {
+		uint32_t px, py;
+		pixel(k, px, py);
 		if (px >= width || py >= height)
 			return false;
 		frame_ray(cam, width, height, beam, bw, px, py, o, d);
 		oc = oct;
 		w = W;
-		out = hits + 2 * ((uint64_t)py * width + px);
 		return true;
+	}
+	__device__ uint4 *out(uint64_t k) const {
+		uint32_t px, py;
+		pixel(k, px, py);
+		return hits + 2 * ((uint64_t)py * width + px);
 	}
 };
 struct ExplicitRays { // R x {o, d} against one octree
+	static constexpr bool kOneOctree = true;
+	static constexpr uint32_t kPool = 1024, kTrips = 16;
 	const uint32_t *oct;
 	uint64_t W;
 	const float *rays;
 	uint4 *hits;
-	__device__ bool ray(uint64_t k, f3 &o, f3 &d, const uint32_t *&oc, uint64_t &w, uint4 *&out) const {
+	__device__ bool ray(uint64_t k, f3 &o, f3 &d, const uint32_t *&oc, uint64_t &w) const {
 		const float *r = rays + 6 * k;
 		o = f3{r[0], r[1], r[2]};
 		d = f3{r[3], r[4], r[5]};
 		oc = oct;
 		w = W;
-		out = hits + 2 * k;
 		return true;
 	}
+	__device__ uint4 *out(uint64_t k) const { return hits + 2 * k; }
 };
 struct SegmentRays { // rays [rbeg[s], rbeg[s+1]) against octree s, per-segment buffers
+	static constexpr bool kOneOctree = false;
+	static constexpr uint32_t kPool = 1024, kTrips = 16;
 	const MarchSeg *segs;
 	const uint64_t *rbeg;
 	uint32_t S;
-	__device__ bool ray(uint64_t k, f3 &o, f3 &d, const uint32_t *&oc, uint64_t &w, uint4 *&out) const {
+	__device__ bool ray(uint64_t k, f3 &o, f3 &d, const uint32_t *&oc, uint64_t &w) const {
 		const uint32_t s = S == 1u ? 0u : seg_find(rbeg, S, k);
 		const MarchSeg &g = segs[s];
 		const uint64_t local = k - rbeg[s];
@@ -694,10 +709,123 @@ struct SegmentRays { // rays [rbeg[s], rbeg[s+1]) against octree s, per-segment 
 		d = f3{r[3], r[4], r[5]};
 		oc = g.oct;
 		w = g.W;
-		out = g.hits + 2 * local;
 		return true;
 	}
+	__device__ uint4 *out(uint64_t k) const {
+		const uint32_t s = S == 1u ? 0u : seg_find(rbeg, S, k);
+		return segs[s].hits + 2 * (k - rbeg[s]);
+	}
 };
+
+template <int kVariant, uint32_t kT, class Src>
+__global__ void __launch_bounds__(kT) march_pool(Src src, uint64_t n, uint32_t *err_out) {
+	constexpr uint32_t kPool = Src::kPool;
+	__shared__ uint32_t s_stack[kStackSlots * kT];
+	__shared__ float s_ray[6 * kT]; // origin and direction of the lane's ray, for its record
+	__shared__ uint32_t s_general[kPool / 32u];
+	__shared__ uint32_t s_next;
+	uint32_t *stk = s_stack + threadIdx.x;
+	float *park = s_ray + threadIdx.x;
+	const uint32_t lane = threadIdx.x & 63u;
+	const uint64_t below = (1ull << lane) - 1ull;
+	const uint64_t base = (uint64_t)xcd_stripes<8>(blockIdx.x, gridDim.x) * kPool;
+	const uint32_t total = (uint32_t)(n - base < kPool ? n - base : kPool);
+	for (uint32_t i = threadIdx.x; i < kPool / 32u; i += kT)
+		s_general[i] = 0u;
+	if (threadIdx.x == 0u)
+		s_next = 0u;
+	__syncthreads();
+	March m;
+	LeanOctree tree{nullptr, 0, 0u, false};
+	if constexpr (Src::kOneOctree)
+		tree = lean_octree(src.oct, src.W);
+	uint32_t k = 0u, iter = 0u, err = 0u;
+	bool active = false, dry = false;
+	for (;;) {
+		const uint64_t idle = __ballot(!active);
+		const uint32_t nidle = (uint32_t)__popcll(idle);
+		if (nidle >= kRefill && !dry) {
+			uint32_t got = 0u;
+			if (lane == 0u)
+				got = atomicAdd(&s_next, nidle);
+			got = (uint32_t)__builtin_amdgcn_readfirstlane(got);
+			dry = got + nidle >= total;
+			k = active ? k : got + (uint32_t)__popcll(idle & below);
+			if (!active && k < total) {
+				f3 o, d;
+				const uint32_t *oct;
+				uint64_t W;
+				if (src.ray(base + k, o, d, oct, W)) {
+					march_init<kVariant != 0>(o, d, m);
+					if constexpr (!Src::kOneOctree)
+						tree = lean_octree(oct, W);
+					iter = 0u;
+					active = lean_ray(tree, m);
+					if (active) {
+						park[0] = o.x, park[kT] = o.y, park[2 * kT] = o.z;
+						park[3 * kT] = d.x, park[4 * kT] = d.y, park[5 * kT] = d.z;
+					} else {
+						atomicOr(&s_general[k >> 5], 1u << (k & 31u));
+					}
+				}
+			}
+		}
+		if (__ballot(active) == 0ull) {
+			if (dry)
+				break;
+			continue;
+		}
+		// a lane whose ray ends writes its record after the trips, together with the other lanes
+		// that ended in them
+		if (active) {
+			uint32_t t = 0;
+			bool marching;
+#pragma unroll 1
+			do
+				marching = lean_trip<false, kT>(tree, m, stk, iter, 0.0f, 0.0f);
+			while (marching && ++t < Src::kTrips);
+			if (!marching) {
+				active = false;
+				if (lean_odd(tree, m, iter)) {
+					atomicOr(&s_general[k >> 5], 1u << (k & 31u));
+				} else {
+					const f3 o{park[0], park[kT], park[2 * kT]}, d{park[3 * kT], park[4 * kT], park[5 * kT]};
+					uint4 r0, r1;
+					march_finish<kVariant>(m, o, d, iter, iter, r0, r1);
+					uint4 *out = src.out(base + k);
+					out[0] = r0;
+					out[1] = r1;
+				}
+			}
+		}
+	}
+	// the block's other rays, one per lane
+	__syncthreads();
+	for (uint32_t q = threadIdx.x; q < total; q += kT) {
+		if (!(s_general[q >> 5] >> (q & 31u) & 1u))
+			continue;
+		f3 o, d;
+		const uint32_t *oct;
+		uint64_t W;
+		(void)src.ray(base + q, o, d, oct, W);
+		March g;
+		uint32_t it, nfetch;
+		march_general<kVariant != 0, kT>(oct, W, o, d, g, stk, it, nfetch, err);
+		uint4 r0, r1;
+		march_finish<kVariant>(g, o, d, it, nfetch, r0, r1);
+		uint4 *out = src.out(base + q);
+		out[0] = r0;
+		out[1] = r1;
+	}
+	if (err)
+		atomicOr(err_out, err);
+}
+
+// ---- the persistent path tracers' refill (path_persist, path_persist_env) ---------------------------
+// A refill costs a ray set-up for the whole wave, so checks are spaced: 16 idle lanes and 16 trips
+// between checks measured best (4 or 8 trips: 4-8% slower; 32 trips or 32 lanes: slower again).
+constexpr uint32_t kTrips = 16;  // loop trips between refill checks
+constexpr uint32_t kChunk = 64;  // rays per chunk
 
 // Up to kTrips trips of the lane's ray, by lean_trip or (lean = false) march_trip; marching turns
 // false when its loop has ended, with iter and nfetch final.  A ray that lean_odd finds starts again
@@ -725,73 +853,6 @@ __device__ __forceinline__ void march_trips(const uint32_t *__restrict__ oct, ui
 		for (uint32_t t = 0; t < kTrips && marching; ++t)
 			marching = march_trip<kT>(oct, W, m, stk, iter, nfetch, err);
 	}
-}
-
-template <int kVariant, uint32_t kT, class Src>
-__global__ void __launch_bounds__(kT)
-    march_persist(Src src, uint64_t n, uint32_t *err_out) {
-	__shared__ uint32_t s_stack[kStackSlots * kT];
-	uint32_t *stk = s_stack + threadIdx.x;
-	const uint32_t lane = threadIdx.x & 63u;
-	const uint64_t wave = (uint64_t)blockIdx.x * (kT / 64u) + (threadIdx.x >> 6);
-	const uint64_t nwaves = (uint64_t)gridDim.x * (kT / 64u);
-	const uint64_t below = (1ull << lane) - 1ull;
-	March m;
-	f3 o{0.0f, 0.0f, 0.0f}, d{0.0f, 0.0f, 0.0f};
-	const uint32_t *oct = nullptr;
-	uint64_t W = 0;
-	uint4 *out = nullptr;
-	uint32_t iter = 0u, nfetch = 0u, err = 0u;
-	bool active = false, lean = false;
-	// wave-uniform: the pool [pool_next, pool_end) and the wave's next chunk
-	uint64_t pool_next = 0, pool_end = 0, chunk = wave;
-	bool exhausted = false;
-	for (;;) {
-		const uint64_t idle = __ballot(!active);
-		const uint32_t nidle = (uint32_t)__popcll(idle);
-		if (nidle >= kRefill && (!exhausted || pool_next < pool_end)) {
-			if (pool_next == pool_end) {
-				const uint64_t lo = chunk * kChunk;
-				if (lo < n) {
-					pool_next = lo;
-					pool_end = lo + kChunk < n ? lo + kChunk : n;
-					chunk += nwaves;
-				} else {
-					exhausted = true;
-				}
-			}
-			if (pool_next < pool_end) {
-				if (!active) {
-					const uint64_t k = pool_next + (uint32_t)__popcll(idle & below);
-					if (k < pool_end && src.ray(k, o, d, oct, W, out)) {
-						march_init<kVariant != 0>(o, d, m);
-						lean = lean_ray(lean_octree(oct, W), m);
-						iter = nfetch = 0u;
-						active = true;
-					}
-				}
-				pool_next = pool_next + nidle < pool_end ? pool_next + nidle : pool_end;
-			}
-		}
-		if (__ballot(active) == 0ull) {
-			if (exhausted && pool_next == pool_end)
-				break;
-			continue;
-		}
-		// kTrips trips; a lane whose ray ends stops stepping and writes its record after the trips,
-		// together with the other lanes that ended in them
-		bool marching = active;
-		march_trips<kVariant != 0, kT>(oct, W, o, d, m, stk, lean, iter, nfetch, err, marching);
-		if (active && !marching) {
-			uint4 r0, r1;
-			march_finish<kVariant>(m, o, d, iter, nfetch, r0, r1);
-			out[0] = r0;
-			out[1] = r1;
-			active = false;
-		}
-	}
-	if (err)
-		atomicOr(err_out, err);
 }
 
 // ---- the path tracer's sampler (shader/path_tracer.comp:42,72,113-117, shader/sobol.glsl:9-10) ----
@@ -1540,17 +1601,14 @@ int tune(svo_ctx *ctx, const std::string &key, int nshapes, const char *const *n
 	return SVO_OK;
 }
 
-const char *const kScheduleName[4] = {"one-ray-per-lane", "persistent-refill", "one-ray-per-lane-8x8",
+const char *const kScheduleName[4] = {"one-ray-per-lane", "refill", "one-ray-per-lane-8x8",
                                       "one-ray-per-lane-8x8-bands"};
 
-// Persistent march of n rays from src; name is the profiler's name of the march.
+// Refill march of n rays from src; name is the profiler's name of the march.
 template <int kVariant, class Src>
-hipError_t launch_persist(svo_ctx *ctx, const char *name, const Src &src, uint64_t n) {
-	uint64_t grid = (n + kBlock - 1) / kBlock;
-	const uint64_t cap = (uint64_t)ctx->cu_count * 6u; // 6 blocks of 4 waves per CU: the occupancy limit
-	grid = grid < cap ? grid : cap;
-	return launch(ctx, name, march_persist<kVariant, kBlock, Src>, dim3((uint32_t)(grid ? grid : 1)), dim3(kBlock), 0,
-	              src, n, ctx->d_err);
+hipError_t launch_pool(svo_ctx *ctx, const char *name, const Src &src, uint64_t n) {
+	return launch(ctx, name, march_pool<kVariant, kBlock, Src>, dim3(div_up(n, Src::kPool)), dim3(kBlock), 0, src, n,
+	              ctx->d_err);
 }
 
 } // namespace
@@ -1588,7 +1646,7 @@ namespace {
 
 // The primary march of a frame (and its beam pre-pass when beam_img is not null, written there).
 // may_tune: the autotuner may time the candidate schedules of a new shape class; without it the
-// schedule is the context's fixed one, or one ray per lane in 8x8 tiles.  timed: bracket the
+// schedule is the context's fixed one, or one ray per lane in 16x16 tiles.  timed: bracket the
 // passes with the context's stage timers.
 int march_frame_into(svo_ctx *ctx, const svo_octree *oct, const svo_camera *cam, uint32_t w, uint32_t h,
                      float *beam_img, svo_hit *hits, bool may_tune, bool timed = true) {
@@ -1601,14 +1659,14 @@ int march_frame_into(svo_ctx *ctx, const svo_octree *oct, const svo_camera *cam,
 		if (rc)
 			return rc;
 	}
-	// schedules: 0 = one ray per lane in 16x16 tiles, 1 = persistent refill, 2 = one ray per lane in one-wave
-	// 8x8 tiles, 3 = as 2 with one band of the frame per XCD (the autotuner's only)
+	// schedules: 0 = one ray per lane in 16x16 tiles, 1 = refill, 2 = one ray per lane in one-wave 8x8
+	// tiles, 3 = as 2 with one band of the frame per XCD (the autotuner's only)
 	auto run = [&](int mode) -> hipError_t {
 		if (mode == 1) {
-			const uint32_t tx8 = (w + 7u) / 8u, ty8 = (h + 7u) / 8u;
-			FrameRays src{(const uint32_t *)oct->words, oct->W, ca, w, h, bw, tx8, beam_img,
+			const uint32_t rx = (w + 31u) / 32u, ry = (h + 31u) / 32u;
+			FrameRays src{(const uint32_t *)oct->words, oct->W, ca, w, h, bw, rx, beam_img,
 			              reinterpret_cast<uint4 *>(hits)};
-			return launch_persist<0>(ctx, "march_frame", src, (uint64_t)tx8 * ty8 * 64u);
+			return launch_pool<0>(ctx, "march_frame", src, (uint64_t)rx * ry * 1024u);
 		}
 		const uint32_t edge = mode == 0 ? 16u : 8u; // pixels
 		const uint32_t tiles_x = (w + edge - 1u) / edge, tiles_y = (h + edge - 1u) / edge;
@@ -1707,9 +1765,9 @@ int march_rays(svo_ctx *ctx, const svo_octree *oct, const float *rays, uint64_t 
 	const ExplicitRays src{(const uint32_t *)oct->words, oct->W, rays, out};
 	auto run = [&](int mode) -> hipError_t {
 		if (mode == 1)
-			return variant == SVO_MARCH_LEAF_ITER ? launch_persist<0>(ctx, "march_rays6", src, R)
-			       : variant == SVO_MARCH_LEAF    ? launch_persist<1>(ctx, "march_rays5", src, R)
-			                                      : launch_persist<2>(ctx, "march_occlude", src, R);
+			return variant == SVO_MARCH_LEAF_ITER ? launch_pool<0>(ctx, "march_rays6", src, R)
+			       : variant == SVO_MARCH_LEAF    ? launch_pool<1>(ctx, "march_rays5", src, R)
+			                                      : launch_pool<2>(ctx, "march_occlude", src, R);
 		if (variant == SVO_MARCH_LEAF_ITER)
 			return launch(ctx, "march_rays6", march_rays_kernel<0>, grid, dim3(kBlock), 0,
 			              (const uint32_t *)oct->words, oct->W, rays, R, out, ctx->d_err);
@@ -2047,9 +2105,9 @@ int march_rays_segments(svo_ctx *ctx, const svo_octree *const *octs, const float
 	auto run = [&](int sh) -> hipError_t {
 		if (sh == 3) {
 			const SegmentRays src{(const MarchSeg *)segs, (const uint64_t *)rbeg, S};
-			return variant == SVO_MARCH_LEAF_ITER ? launch_persist<0>(ctx, "march_rays_batch", src, R)
-			       : variant == SVO_MARCH_LEAF    ? launch_persist<1>(ctx, "march_rays_batch", src, R)
-			                                      : launch_persist<2>(ctx, "march_rays_batch", src, R);
+			return variant == SVO_MARCH_LEAF_ITER ? launch_pool<0>(ctx, "march_rays_batch", src, R)
+			       : variant == SVO_MARCH_LEAF    ? launch_pool<1>(ctx, "march_rays_batch", src, R)
+			                                      : launch_pool<2>(ctx, "march_rays_batch", src, R);
 		}
 		const uint32_t bs = kRayBlock[sh];
 		const dim3 grid(div_up(R, bs)), block(bs);

@@ -80,7 +80,7 @@ def march_all(ctx, octree, rays, variant):
         ctx.check(lib.svo_march_mode(ctx.h, mode))
         try:
             out.append(S.march_rays(ctx, octree, rays, variant))
-            cut = len(rays) // 3 + 5
+            cut = len(rays) // 3
             out.append(np.concatenate(S.march_rays_batch([octree, octree], [rays[:cut], rays[cut:]], variant)))
         finally:
             ctx.check(lib.svo_march_mode(ctx.h, -1))
@@ -187,3 +187,18 @@ def test_frame_tiles_cover_every_pixel(ctx, no_device_errors, W, H):
         for k in range(3):
             ok, msg = hits_equal(got[k], ref)
             assert ok, "shape %d frame %d: %s" % (shape, k, msg)
+
+
+@pytest.mark.parametrize("R", [1, 65, 1023, 1025, 66567])
+def test_ray_pool_sizes_match_oracle(ctx, no_device_errors, R):
+    # whole and partial pools of the refill schedule (1024 rays), around its dealing to the XCDs (64 pools)
+    import sparsevoxeloctree_amd as S
+
+    words = scene_words(ctx)
+    octree = S.Octree.FromWords(ctx, words, 6)
+    rays = odd_rays(R, max(R, 8))[:R]
+    ref = oracle.march_rays(words, 6, rays, 0)
+    print("ray pool", R, flush=True)
+    for k, got in enumerate(march_all(ctx, octree, rays, 0)):
+        ok, msg = hits_equal(got, ref)
+        assert ok, "form %d: %s" % (k, msg)
