@@ -110,6 +110,8 @@ struct BuildSeg {
 	uint64_t nbins;      // leaf blocks = nodes of depth L-1 (the root when L = 1)
 	uint32_t L;
 	uint32_t overflow;   // W > 2^30
+	uint32_t raw;        // keys are fragment indices: a raw coordinate above 2^L (structure phase)
+	uint32_t pad;
 	uint64_t off[14];    // word offset of B[d] relative to bm, d = 1..L; off[L] = the scene's bitmap words
 	uint32_t fb[16];     // first block of every depth: fb[0] = 0 (root block), fb[1] = 1
 };
@@ -133,7 +135,7 @@ struct BuildBatch {
 	uint32_t maxL = 0;
 	uint64_t Ftot = 0, TW = 0, nbins = 0;
 	std::vector<BuildSeg> h_segs;
-	// begin tables, S + 1 entries each: fbeg (fragments), bbeg (leaf blocks), dw[d] at 2 + d (words of
+	// begin tables, S + 1 entries each: tbeg (fragment tiles), bbeg (leaf blocks), dw[d] at 2 + d (words of
 	// B[d] of the scenes with L > d), dr[d] at 3 + kMaxLevel + d (same, scenes with L > d + 1); then
 	// pw (pw_at): the block writer's segments
 	std::vector<uint64_t> h_index;
@@ -141,10 +143,15 @@ struct BuildBatch {
 	uint64_t *index = nullptr;
 	uint32_t *bm = nullptr, *rk = nullptr; // bitmaps (TW words), ranks of 8-word chunks (TW / 8 + 1)
 	uint32_t *cnt = nullptr, *aux = nullptr; // per leaf block (nbins)
-	uint32_t *node = nullptr;   // 2 * Ftot: {leaf block, place in its bucket}
-	uint32_t *bucket = nullptr; // 2 * Ftot
-	uint32_t *list = nullptr;   // 2 + 2 * cap: large leaf blocks
-	const uint64_t *fbeg() const { return index; }
+	uint32_t *raw = nullptr;    // per scene: raw flag of the structure phase (after rk)
+	// per fragment tile (tiles = h_index[S]), in one allocation at runs: runs, heads, keys, run counts
+	uint64_t tiles = 0;
+	uint2 *runs = nullptr;
+	uint64_t *heads = nullptr;
+	uint32_t *keys = nullptr, *nrun = nullptr;
+	uint32_t *bucket = nullptr; // Ftot keys, by leaf block
+	uint32_t *list = nullptr;   // 3 + 3 * cap: large leaf blocks
+	const uint64_t *tbeg() const { return index; }
 	const uint64_t *bbeg() const { return index + (S + 1); }
 	const uint64_t *dw(uint32_t d) const { return index + (2 + d) * (uint64_t)(S + 1); }
 	uint64_t h_dw(uint32_t d, uint32_t s) const { return h_index[(2 + d) * (uint64_t)(S + 1) + s]; }

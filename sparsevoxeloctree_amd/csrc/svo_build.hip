@@ -8,9 +8,10 @@
 // fragment pass per level:
 //
 // Reference pass              -> here
-//   octree_tag_node.comp      -> bm_mark: each fragment sets the bit of its depth-(L-1) node in
-//   (levels 1..L-1)              bitmap B[L-1]; bm_reduce ORs each byte of B[d+1] (8 children) into
-//                                one bit of B[d], d = L-2..1
+//   octree_tag_node.comp      -> bm_group: each tile of consecutive fragments is grouped by depth-(L-1)
+//   (levels 1..L-1)              node ("runs"), and every run's node is marked in bitmap B[L-1];
+//                                bm_reduce ORs each byte of B[d+1] (8 children) into one bit of B[d],
+//                                d = L-2..1
 //   octree_alloc_node.comp    -> one exclusive scan over the set-bit counts of all bitmaps' 8-word
 //                                chunks (stored by bm_reduce while it reads them)
 //                                (rank of every occupied node among its depth = its block among
@@ -19,15 +20,15 @@
 //   octree_modify_arg.comp    -> bm_levels: per-depth counts -> first block of every depth, the
 //                                leaf blocks and W = (counter + 1) * 8
 //   octree_init_node.comp     -> bm_write_blocks writes every block whole (pointers and zeros)
-//   octree_tag_node.comp      -> build_tag_leaf: leaf block ("bin") of each fragment = rank of its
-//   (level L) + leaf CAS fold    depth-(L-1) node; count per bin, scan, scatter into per-bin buckets;
-//                                build_fold{,_mid,_big} sort each bucket by the 64-bit fragment and
+//   octree_tag_node.comp      -> tag_runs: leaf block ("bin") of each run = rank of its depth-(L-1)
+//   (level L) + leaf CAS fold    node; count per bin, scan, scatter_runs into per-bin buckets;
+//                                build_fold and build_fold_lists sort each bucket in fragment order and
 //                                fold the 8 leaves of the block in that order (the reference's order
 //                                is whatever its atomics produce), writing the leaf block whole.
 // The node words are identical to the reference's pass structure run with a serial allocator.
 //
-// Batch layout: the scenes' fragments, bitmap words and leaf blocks each form one index space
-// (begin tables fbeg, dw/dr per depth, bbeg).  Every depth's bitmap starts on an 8-word boundary;
+// Batch layout: the scenes' fragment tiles, bitmap words and leaf blocks each form one index space
+// (begin tables tbeg, dw/dr per depth, bbeg).  Every depth's bitmap starts on an 8-word boundary;
 // the rank array R holds one entry per 8-word chunk (set bits of all bitmaps before the chunk), so
 // it is 1/8 of the bitmaps' size, and a node's rank is its chunk's entry plus the popcounts of the
 // chunk's words before it.  Every rank is a difference of two R-based counts of the same scene,
@@ -77,12 +78,6 @@ __device__ __forceinline__ uint64_t morton(uint32_t x, uint32_t y, uint32_t z) {
 	return spread3(x) | (spread3(y) << 1) | (spread3(z) << 2);
 }
 
-__device__ __forceinline__ void cmp_swap(uint64_t &x, uint64_t &y) {
-	const uint64_t lo = y < x ? y : x, hi = y < x ? x : y;
-	x = lo;
-	y = hi;
-}
-
 __device__ __forceinline__ uint64_t frag_key(uint2 f) { return ((uint64_t)f.x << 32) | f.y; }
 
 // Set bits of the words of an 8-word chunk before word j (< 8), and word j (one 32-byte load).
@@ -107,118 +102,227 @@ __device__ __forceinline__ uint32_t bits_before(const uint32_t *__restrict__ B, 
 	return R[w >> 3] + chunk_before(B + (w & ~7ull), (uint32_t)(w & 7u), word);
 }
 
-__global__ void __launch_bounds__(kThreads) bm_zero(uint32_t *B, uint64_t n) {
+// Clears the bitmaps and the scenes' raw flags.
+__global__ void __launch_bounds__(kThreads) bm_zero(uint32_t *B, uint64_t n, uint32_t *raw, uint32_t S) {
 	const uint64_t stride = (uint64_t)gridDim.x * kThreads;
 	for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride)
 		B[i] = 0u;
+	if (blockIdx.x == 0u)
+		for (uint32_t s = threadIdx.x; s < S; s += kThreads)
+			raw[s] = 0u;
 }
 
-// Fragments per thread and loop trip in the per-fragment passes: their loads are issued together,
-// so a wave waits on one chain of dependent memory round trips for kU fragments.
-constexpr uint32_t kU = 4;
+// Order of a leaf block's fragments in 32 bits: child slot | raw-coordinate flags | rgb.  The fold goes
+// leaf by leaf in ascending fragment order, and the fragments of one leaf differ in their raw
+// coordinates only where the descent saturates (res and above meet res - 1): at most one step above
+// for a voxelized scene, so a flag per axis orders them as the packed words do (z's low byte, y, x;
+// the low byte of res is below that of res - 1 from 2^8 on).  A raw coordinate above res (a list from
+// the host, or a scene reaching out of the cube) does not fit: kRawKey, and its scene's keys become
+// fragment indices (BuildSeg::raw), compared by the fragments they name.
+constexpr uint32_t kRawKey = 0xFFFFFFFFu;
 
-// Where a fragment's scene keeps what the per-fragment passes read: the fragment itself, the first
-// word of the scene's B[L-1] (and of its ranks), the level and the scene's first bin.
-struct FragSrc {
-	const uint2 *frag;
-	uint64_t w0;
-	uint32_t L, bin_begin;
-};
+__device__ __forceinline__ uint32_t leaf_key(uint2 f, uint32_t res) {
+	const uint32_t x = f.x & 0xfffu, y = (f.x >> 12u) & 0xfffu, z = (f.x >> 24u) | ((f.y >> 28u) << 8u);
+	const uint32_t sx = x >= res ? 1u : 0u, sy = y >= res ? 1u : 0u, sz = z >= res ? 1u : 0u;
+	const uint32_t slot = ((x - sx) & 1u) | ((y - sy) & 1u) << 1u | ((z - sz) & 1u) << 2u;
+	const uint32_t fz = sz ^ (res >= 256u ? 1u : 0u);
+	const uint32_t key = slot << 27u | fz << 26u | sy << 25u | sx << 24u | (f.y & 0xffffffu);
+	return umax32(umax32(x, y), z) > res ? kRawKey : key;
+}
 
-// Descriptor lookups for the kU fragments base + u * kThreads + threadIdx.x of one loop trip
-// (no fragment loads); frag = nullptr past the end.
-__device__ __forceinline__ void frag_sources(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ fbeg,
-                                             uint32_t S, uint64_t Ftot, uint64_t base, uint32_t &hint,
-                                             FragSrc (&src)[kU]) {
+// ---- tiles and runs ------------------------------------------------------------------------------
+// Fragments come in raster order, so consecutive ones lie in few leaf blocks: a tile of kTile = 1024
+// holds about 270 distinct ones (a room at 2^10; 160 for spheres at 2^9, 400 with random slivers at
+// 2^12).  So a tile's fragments are grouped by leaf block once, into "runs", and everything that is
+// random access happens per run: marking, rank lookups, bin counts, bucket places.  Per fragment only
+// a 4-byte key moves, in tile order (whole lines) and from there to its bucket (a run at a time).
+// Against marking, tagging and scattering whole fragments one by one (same order: room at 2^10 / slivers
+// at 2^12 / 32 mixed scenes): 752 / 4688 / 2573 us -> 454 / 3804 / 1190 us for the three passes.  Larger
+// tiles have hardly fewer runs (4096: -4%), and groups of tiles per XCD measured no different.
+//   keys[t * kTile ..]   leaf_keys of tile t (or fragment indices), run after run
+//   heads[t * 16 ..]     bit i: key i starts a run
+//   runs[t * kTile ..]   per run {node P low, P's bit 32 << 31 | first key}, then {bin, place - first key}
+//   nrun[t]              its runs
+constexpr uint32_t kTile = 1024;
+constexpr uint32_t kU = kTile / kThreads;
+constexpr uint32_t kHeads = kTile / 64u;
+constexpr uint32_t kLines = 256;    // LDS table: groups of 16 neighbouring nodes (2 bits of x, one of y and z)
+constexpr uint32_t kLineStride = 9; // words of two counters per group, padded against bank conflicts
+constexpr uint32_t kProbes = 32;
+constexpr uint32_t kEmpty = 0xFFFFFFFFu;
+static_assert(kLines == kThreads, "one thread per group in the scan");
+
+// One block per tile.  Every fragment finds its group of 16 nodes in an LDS hash table and takes a
+// place in its node's counter; a scan over the counters turns them into offsets, so the runs come out
+// group by group in Morton order inside (neighbouring lanes of tag_runs then count in one 64-byte
+// line).  A fragment that finds no group in kProbes probes becomes a run of its own at the tile's end
+// (random slivers at 2^12 touch 152 groups on average, 288 at most).  Each group marks its nodes with
+// one load and, only if bits are missing, one atomic.  Bound by VALU (0.6 busy) and the latency of its
+// phases, at 8 waves per SIMD: 193 us for 35M fragments in a room.  kIndex: a second pass that only rewrites the
+// keys (and their order) of the raw scenes' tiles as fragment indices.
+template <bool kIndex>
+__global__ void __launch_bounds__(kThreads)
+    bm_group(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ tbeg, uint32_t S, uint32_t *B,
+             uint32_t *__restrict__ keys, uint64_t *__restrict__ heads, uint2 *__restrict__ runs,
+             uint32_t *__restrict__ nrun, uint32_t *raw) {
+	__shared__ uint32_t s_line[kLines], s_node[kLines]; // group key, Morton index of the group
+	__shared__ uint32_t s_n[kLines * kLineStride];      // per node 16 bits: fragments, then the first key
+	__shared__ uint32_t s_key[kTile];
+	__shared__ uint32_t s_head[kTile / 32u], s_before[kTile / 32u];
+	__shared__ uint32_t s_wave[kThreads / 64u], s_over;
+	const uint64_t tile = blockIdx.x;
+	if (tile >= tbeg[S])
+		return;
+	const uint32_t sc = S == 1u ? 0u : seg_find(tbeg, S, tile);
+	const BuildSeg &g = segs[sc];
+	if (kIndex && !g.raw)
+		return; // block-uniform
+	const uint32_t L = g.L, res = 1u << L;
+	const uint64_t first = (tile - tbeg[sc]) * kTile;
+	const uint32_t n = g.F - first < kTile ? (uint32_t)(g.F - first) : kTile;
+	const uint2 *frags = g.frags + first;
+	for (uint32_t i = threadIdx.x; i < kLines * kLineStride; i += kThreads)
+		s_n[i] = 0u;
+	s_line[threadIdx.x] = kEmpty;
+	if (threadIdx.x < kTile / 32u)
+		s_head[threadIdx.x] = 0u;
+	if (threadIdx.x == 0u)
+		s_over = 0u;
+	uint2 fr[kU];
 #pragma unroll
 	for (uint32_t u = 0; u < kU; ++u) {
-		const uint64_t b = base + (uint64_t)u * kThreads, f = b + threadIdx.x;
-		src[u] = FragSrc{nullptr, 0u, 1u, 0u};
-		if (f < Ftot)
-			with_seg<kThreads>(fbeg, S, hint, b, f, [&](uint32_t s) {
-				const BuildSeg &g = segs[s];
-				const uint32_t L = g.L;
-				src[u] = FragSrc{g.frags + (f - fbeg[s]), g.bm + (L > 1u ? g.off[L - 1u] : 0u), L,
-				                 (uint32_t)g.bin_begin};
-			});
-	}
-}
-
-// Depth-(L-1) node of a fragment (its leaf block's parent), as a Morton index.
-__device__ __forceinline__ uint64_t frag_parent(uint2 fr, uint32_t L) {
-	uint32_t x, y, z;
-	decode_frag(fr, 1u << L, x, y, z);
-	return morton(x, y, z) >> 3;
-}
-
-// Open-addressing tables in LDS that merge the kU * kThreads fragments of one loop trip by key
-// before anything touches global memory: fragments come in raster order, so lanes next to each
-// other alternate between leaf blocks and a wave's runs of equal keys are short, while a trip's
-// 1024 fragments hold few distinct keys.
-constexpr uint32_t kHash = 2048; // slots, twice the fragments of a trip
-constexpr uint32_t kEmpty = 0xFFFFFFFFu;
-
-__device__ __forceinline__ uint32_t hash_slot(uint64_t key) {
-	return (uint32_t)((key * 0x9E3779B97F4A7C15ull) >> (64 - 11)); // 11 bits = kHash
-}
-
-// Each fragment marks its depth-(L-1) node.  The trip's bits are ORed per bitmap word in LDS, then
-// each distinct word costs one load and, only when that load does not already show all of its
-// bits, one atomic.
-__global__ void __launch_bounds__(kThreads)
-    bm_mark(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ fbeg, uint32_t S, uint32_t *B) {
-	const uint64_t Ftot = fbeg[S];
-	static_assert(kHash == 2048u && kHash >= 2u * kU * kThreads, "hash_slot returns 11 bits");
-	__shared__ unsigned long long s_word[kHash];
-	__shared__ uint32_t s_bits[kHash];
-	for (uint32_t h = threadIdx.x; h < kHash; h += kThreads) {
-		s_word[h] = ~0ull;
-		s_bits[h] = 0u;
+		const uint32_t i = threadIdx.x + u * kThreads;
+		fr[u] = i < n ? frags[i] : make_uint2(0u, 0u);
 	}
 	__syncthreads();
-	const uint64_t stride = (uint64_t)gridDim.x * kThreads * kU;
-	uint32_t hint = 0;
-	for (uint64_t base = (uint64_t)blockIdx.x * kThreads * kU; base < Ftot; base += stride) {
-		FragSrc src[kU];
-		frag_sources(segs, fbeg, S, Ftot, base, hint, src);
-		uint2 fr[kU];
+	// counter of the fragment's node (group * 16 + node; kEmpty: a run of its own) and place in its run
+	uint32_t at[kU], place[kU], key[kU];
+	bool wide = false;
 #pragma unroll
-		for (uint32_t u = 0; u < kU; ++u)
-			fr[u] = src[u].frag ? *src[u].frag : make_uint2(0u, 0u);
-#pragma unroll
-		for (uint32_t u = 0; u < kU; ++u) {
-			if (src[u].frag && src[u].L > 1u) {
-				const uint64_t P = frag_parent(fr[u], src[u].L);
-				const unsigned long long word = src[u].w0 + (P >> 5); // global bitmap word
-				uint32_t h = hash_slot(word);
-				for (;;) { // at most kU * kThreads keys in kHash slots: a free or equal slot exists
-					const unsigned long long old = atomicCAS(&s_word[h], ~0ull, word);
-					if (old == ~0ull || old == word)
-						break;
-					h = (h + 1u) & (kHash - 1u);
-				}
-				atomicOr(&s_bits[h], 1u << (uint32_t)(P & 31u));
+	for (uint32_t u = 0; u < kU; ++u) {
+		at[u] = kEmpty;
+		place[u] = 0u;
+		if (threadIdx.x + u * kThreads >= n)
+			continue;
+		key[u] = leaf_key(fr[u], res);
+		wide |= key[u] == kRawKey;
+		uint32_t x, y, z;
+		decode_frag(fr[u], res, x, y, z);
+		const uint32_t line = (x >> 3u) | (y >> 2u) << 9u | (z >> 2u) << 19u;
+		const uint32_t sub = (x >> 1u & 1u) | (y & 2u) | (z << 1u & 4u) | (x << 1u & 8u);
+		uint32_t h = (line * 2654435761u) >> 24u;
+		for (uint32_t probe = 0; probe < kProbes; ++probe) {
+			const uint32_t old = atomicCAS(&s_line[h], kEmpty, line);
+			if (old == kEmpty || old == line) {
+				at[u] = h * 16u + sub;
+				break;
 			}
+			h = (h + 1u) & (kLines - 1u);
 		}
-		__syncthreads();
-		uint64_t word[kHash / kThreads];
-		uint32_t bits[kHash / kThreads], have[kHash / kThreads];
+		const uint32_t sh = (sub & 1u) * 16u;
+		place[u] = at[u] != kEmpty ? atomicAdd(&s_n[h * kLineStride + (sub >> 1u)], 1u << sh) >> sh & 0xffffu
+		                           : atomicAdd(&s_over, 1u);
+	}
+	if (!kIndex && __any(wide) && (threadIdx.x & 63u) == 0u)
+		atomicOr(&raw[sc], 1u);
+	__syncthreads();
+	// first keys of the groups' nodes (thread h owns group h), marking
+	uint32_t v[8], sum = 0u, mask = 0u;
 #pragma unroll
-		for (uint32_t k = 0; k < kHash / kThreads; ++k) {
-			const uint32_t h = threadIdx.x + k * kThreads;
-			word[k] = s_word[h];
-			bits[k] = s_bits[h];
-			s_word[h] = ~0ull;
-			s_bits[h] = 0u;
+	for (uint32_t c = 0; c < 8u; ++c) {
+		v[c] = s_n[threadIdx.x * kLineStride + c];
+		sum += (v[c] & 0xffffu) + (v[c] >> 16u);
+		mask |= (v[c] & 0xffffu ? 1u << (2u * c) : 0u) | (v[c] >> 16u ? 2u << (2u * c) : 0u);
+	}
+	if (mask) {
+		const uint32_t line = s_line[threadIdx.x];
+		// the group's Morton index: the node's bits above the 4 of its place in the group
+		const uint32_t gn = (uint32_t)(morton((line & 0x1ffu) << 2u, (line >> 9u & 0x3ffu) << 1u,
+		                                      (line >> 19u & 0x3ffu) << 1u) >> 4);
+		s_node[threadIdx.x] = gn;
+		if (!kIndex && L > 1u) {
+			uint32_t *word = B + g.bm + g.off[L - 1u] + (gn >> 1u);
+			const uint32_t bits = mask << (16u * (gn & 1u));
+			if ((*word & bits) != bits) // a stale cached word only costs a redundant atomic
+				atomicOr(word, bits);
 		}
+	}
+	uint32_t incl = sum;
 #pragma unroll
-		for (uint32_t k = 0; k < kHash / kThreads; ++k)
-			have[k] = word[k] != ~0ull ? B[word[k]] : ~0u;
+	for (uint32_t d = 1; d < 64u; d <<= 1) {
+		const uint32_t o = __shfl_up(incl, d, 64);
+		incl += (threadIdx.x & 63u) >= d ? o : 0u;
+	}
+	if ((threadIdx.x & 63u) == 63u)
+		s_wave[threadIdx.x >> 6] = incl;
+	__syncthreads();
+	uint32_t run = incl - sum, grouped = 0u;
 #pragma unroll
-		for (uint32_t k = 0; k < kHash / kThreads; ++k)
-			if ((have[k] & bits[k]) != bits[k]) // a stale cached word only costs a redundant atomic
-				atomicOr(B + word[k], bits[k]);
-		__syncthreads();
+	for (uint32_t w = 0; w < kThreads / 64u; ++w) {
+		run += w < (threadIdx.x >> 6) ? s_wave[w] : 0u;
+		grouped += s_wave[w];
+	}
+	if (mask) {
+#pragma unroll
+		for (uint32_t c = 0; c < 8u; ++c) {
+			const uint32_t next = run + (v[c] & 0xffffu);
+			s_n[threadIdx.x * kLineStride + c] = run | next << 16u;
+			run = next + (v[c] >> 16u);
+		}
+	}
+	__syncthreads();
+	// keys to their places, run heads
+#pragma unroll
+	for (uint32_t u = 0; u < kU; ++u) {
+		const uint32_t i = threadIdx.x + u * kThreads;
+		if (i >= n)
+			continue;
+		uint32_t p = grouped;
+		if (at[u] != kEmpty)
+			p = s_n[(at[u] >> 4u) * kLineStride + (at[u] >> 1u & 7u)] >> (at[u] & 1u) * 16u & 0xffffu;
+		const bool head = at[u] == kEmpty || place[u] == 0u;
+		p += place[u];
+		s_key[p] = kIndex ? (uint32_t)(first + i) : key[u];
+		if (head)
+			atomicOr(&s_head[p >> 5u], 1u << (p & 31u));
+		place[u] = head ? p : kEmpty; // from here on: the run's first key, at its head
+	}
+	__syncthreads();
+	if (threadIdx.x < 64u) { // run heads before each 32 keys
+		const uint32_t c = threadIdx.x < kTile / 32u ? (uint32_t)__popc(s_head[threadIdx.x]) : 0u;
+		uint32_t p = c;
+#pragma unroll
+		for (uint32_t d = 1; d < kTile / 32u; d <<= 1) {
+			const uint32_t o = __shfl_up(p, d, 64);
+			p += threadIdx.x >= d ? o : 0u;
+		}
+		if (threadIdx.x < kTile / 32u)
+			s_before[threadIdx.x] = p - c;
+		if (threadIdx.x == kTile / 32u - 1u)
+			nrun[tile] = p;
+	}
+	for (uint32_t i = threadIdx.x; i < n; i += kThreads)
+		keys[tile * kTile + i] = s_key[i];
+	if (threadIdx.x < kHeads)
+		heads[tile * kHeads + threadIdx.x] = (uint64_t)s_head[2u * threadIdx.x + 1u] << 32 | s_head[2u * threadIdx.x];
+	__syncthreads();
+#pragma unroll
+	for (uint32_t u = 0; u < kU; ++u) {
+		const uint32_t i = threadIdx.x + u * kThreads, p = place[u];
+		if (i >= n || p == kEmpty)
+			continue;
+		const uint32_t r = s_before[p >> 5u] + (uint32_t)__popc(s_head[p >> 5u] & ((1u << (p & 31u)) - 1u));
+		uint64_t P;
+		if (at[u] != kEmpty) {
+			P = (uint64_t)s_node[at[u] >> 4u] << 4 | (at[u] & 15u);
+		} else {
+			uint32_t x, y, z;
+			decode_frag(frags[i], res, x, y, z);
+			P = morton(x, y, z) >> 3;
+			if (!kIndex && L > 1u)
+				atomicOr(B + g.bm + g.off[L - 1u] + (P >> 5), 1u << (uint32_t)(P & 31u));
+		}
+		runs[tile * kTile + r] = make_uint2((uint32_t)P, (uint32_t)(P >> 32) << 31u | p);
 	}
 }
 
@@ -334,7 +438,8 @@ struct RankDst {
 
 // One thread per scene: per-depth node counts -> first block of every depth (fb[0] = 0 is the root
 // block, fb[1] = 1), the leaf blocks and W (src/OctreeBuilder.cpp:212-214: W = (counter + 1) * 8).
-__global__ void bm_levels(BuildSeg *segs, uint32_t S, const uint32_t *__restrict__ R, uint64_t cap) {
+__global__ void bm_levels(BuildSeg *segs, uint32_t S, const uint32_t *__restrict__ R, const uint32_t *__restrict__ raw,
+                          uint64_t cap) {
 	const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
 	if (s >= S)
 		return;
@@ -354,6 +459,7 @@ __global__ void bm_levels(BuildSeg *segs, uint32_t S, const uint32_t *__restrict
 	g.W = 8u * first;
 	g.overflow = g.W > cap ? 1u : 0u;
 	g.nbins = nlast;
+	g.raw = raw[s];
 }
 
 // The 8 words of the block of one depth-(d-1) parent: pointers to the blocks of its occupied
@@ -396,7 +502,7 @@ __device__ __forceinline__ uint32_t nth_bit(uint32_t v, uint32_t n) {
 // are contiguous.  A wave across a segment boundary walks each word's set bits in its own lane.
 // Block 0 also writes the root block of every scene with L > 1 (its 8 words point to the depth-1
 // blocks of the occupied children, the bits of B[1]).  The same launch clears the nb leaf-block
-// counters of build_tag_leaf and the three counts of the fold's work lists.
+// counters of tag_runs and the three counts of the fold's work lists.
 __global__ void __launch_bounds__(kThreads)
     bm_write_blocks(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ pw, uint32_t M, uint32_t S,
                     const uint32_t *__restrict__ B, const uint32_t *__restrict__ R, uint32_t *cnt,
@@ -506,176 +612,111 @@ __global__ void __launch_bounds__(kThreads)
 	}
 }
 
-// Leaf block ("bin") of every fragment: the rank of its depth-(L-1) node, offset by the scene's
-// first bin; node[f] = {bin, place}, where place is unique inside the bin, so the scatter needs no
-// atomics.  Places come from per-bin counters in global memory whose atomics the L2 cannot perform
-// (they are device-coherent, so they go to memory), and each such request stalls the L2 for the
-// reads behind it.  So a loop trip first counts its kU * kThreads fragments in LDS, per 64-byte line
-// of 16 counters (a line table with linear probing; the count's old value is the fragment's place
-// among the trip's fragments of its bin), and then adds each line's counts with 16 neighbouring
-// lanes, which the L1 merges into one request per line: a trip of 1024 fragments touches about
-// 40 lines (a room scene at 2^10) to 150 (random slivers at 2^12) instead of 200+; kLines line slots
-// (128 up to level 11, 256 at level 12).  A fragment that finds the table full takes its place with
-// its own atomic.
-constexpr uint32_t kLineBins = 16; // 4-byte counters per 64-byte line
-
-template <uint32_t kLines>
+// Leaf block ("bin") of every run: the rank of its depth-(L-1) node, offset by the scene's first bin, and
+// the run's place in the bin's bucket, from per-bin counters.  A wave takes a tile's runs 64 at a time;
+// neighbouring lanes hold neighbouring nodes, so their counters share 64-byte lines and the L1 sends
+// one request per line (device-coherent atomics are done at the memory side, and each request stalls
+// the L2 for the reads behind it).  Bound by those requests: 2.7M in 134 us for the 9.4M runs of a room.
 __global__ void __launch_bounds__(kThreads)
-    build_tag_leaf(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ fbeg, uint32_t S,
-                   const uint32_t *__restrict__ B, const uint32_t *__restrict__ R, uint2 *__restrict__ node,
-                   uint32_t *cnt) {
-	const uint64_t Ftot = fbeg[S];
-	__shared__ uint32_t line[kLines];
-	__shared__ uint32_t n[kLines * kLineBins];
-	for (uint32_t i = threadIdx.x; i < kLines; i += kThreads)
-		line[i] = kEmpty;
-	for (uint32_t i = threadIdx.x; i < kLines * kLineBins; i += kThreads)
-		n[i] = 0u;
-	__syncthreads();
-	const uint64_t stride = (uint64_t)gridDim.x * kThreads * kU;
-	uint32_t hint = 0;
-	for (uint64_t base = (uint64_t)blockIdx.x * kThreads * kU; base < Ftot; base += stride) {
-		FragSrc src[kU];
-		frag_sources(segs, fbeg, S, Ftot, base, hint, src);
-		uint2 fr[kU];
+    tag_runs(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ tbeg, uint32_t S,
+             const uint32_t *__restrict__ B, const uint32_t *__restrict__ R, uint2 *__restrict__ runs,
+             const uint32_t *__restrict__ nrun, uint32_t *cnt) {
+	constexpr uint32_t kPer = kThreads / 64u, kV = 4; // tiles per block, runs per lane and trip
+	const uint32_t lane = threadIdx.x & 63u;
+	const uint64_t tile = (uint64_t)blockIdx.x * kPer + (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	if (tile >= tbeg[S])
+		return;
+	const uint32_t sc = S == 1u ? 0u : seg_find(tbeg, S, tile);
+	const BuildSeg &g = segs[sc];
+	const uint64_t w0 = g.bm + (g.L > 1u ? g.off[g.L - 1u] : 0u); // the depth's first word starts a chunk
+	const uint32_t bin0 = (uint32_t)g.bin_begin - (g.L > 1u ? R[w0 >> 3] : 0u);
+	const uint64_t first = (tile - tbeg[sc]) * kTile;
+	const uint32_t keys = g.F - first < kTile ? (uint32_t)(g.F - first) : kTile, n = nrun[tile];
+	uint2 *rt = runs + tile * kTile;
+	for (uint32_t i0 = 0; i0 < n; i0 += 64u * kV) {
+		uint32_t bin[kV], len[kV];
+		uint2 r[kV];
+		uint32_t end[kV];
 #pragma unroll
-		for (uint32_t u = 0; u < kU; ++u)
-			fr[u] = src[u].frag ? *src[u].frag : make_uint2(0u, 0u);
-		// rank of the fragment's depth-(L-1) node among its scene's occupied nodes of that depth
-		// (w0, the depth's first word, starts a chunk)
-		uint32_t below[kU], r[kU], r0[kU], bin[kU];
+		for (uint32_t v = 0; v < kV; ++v) {
+			const uint32_t i = i0 + v * 64u + lane;
+			r[v] = i < n ? rt[i] : make_uint2(0u, 0u);
+			end[v] = i + 1u < n ? rt[i + 1u].y : keys;
+		}
 #pragma unroll
-		for (uint32_t u = 0; u < kU; ++u) {
-			r[u] = r0[u] = below[u] = 0u;
-			if (src[u].frag && src[u].L > 1u) {
-				const uint64_t P = frag_parent(fr[u], src[u].L);
+		for (uint32_t v = 0; v < kV; ++v) {
+			bin[v] = bin0;
+			len[v] = (end[v] & 0x7fffffffu) - (r[v].y & 0x7fffffffu);
+			if (g.L > 1u && i0 + v * 64u + lane < n) {
+				const uint64_t P = (uint64_t)(r[v].y >> 31u) << 32 | r[v].x;
 				uint32_t word;
-				r[u] = bits_before(B, R, src[u].w0 + (P >> 5), word);
-				r0[u] = R[src[u].w0 >> 3];
-				below[u] = word & ((1u << (uint32_t)(P & 31u)) - 1u);
+				bin[v] += bits_before(B, R, w0 + (P >> 5), word);
+				bin[v] += (uint32_t)__popc(word & ((1u << (uint32_t)(P & 31u)) - 1u));
 			}
 		}
-		uint32_t slot[kU], local[kU];
 #pragma unroll
-		for (uint32_t u = 0; u < kU; ++u) {
-			bin[u] = src[u].frag ? src[u].bin_begin + (r[u] - r0[u]) + (uint32_t)__popc(below[u]) : kEmpty;
-			slot[u] = kEmpty;
-			local[u] = 0u;
-			if (bin[u] != kEmpty) {
-				const uint32_t key = bin[u] / kLineBins;
-				static_assert(kLines == 128u || kLines == 256u, "kLines: 7 or 8 hash bits");
-				uint32_t h = (key * 2654435761u) >> (kLines == 256u ? 24 : 25), probes = 0;
-				for (;;) {
-					const uint32_t old = atomicCAS(&line[h], kEmpty, key);
-					if (old == kEmpty || old == key) {
-						slot[u] = h * kLineBins + bin[u] % kLineBins;
-						break;
-					}
-					if (++probes == kLines)
-						break; // table full
-					h = (h + 1u) & (kLines - 1u);
-				}
-				local[u] = slot[u] != kEmpty ? atomicAdd(&n[slot[u]], 1u) : atomicAdd(&cnt[bin[u]], 1u);
-			}
-		}
-		__syncthreads();
-		// one atomic per counter with fragments; lanes 16k..16k+15 hold the 16 counters of one line
-		constexpr uint32_t kPer = kLines * kLineBins / kThreads, kGroup = 8; // counters per thread, per batch
-		static_assert(kPer % kGroup == 0u, "whole batches");
-#pragma unroll 1
-		for (uint32_t k0 = 0; k0 < kPer; k0 += kGroup) {
-			uint32_t key[kGroup], c[kGroup];
+		for (uint32_t v = 0; v < kV; ++v)
+			if (i0 + v * 64u + lane < n)
+				r[v] = make_uint2(bin[v], atomicAdd(&cnt[bin[v]], len[v]) - (r[v].y & 0x7fffffffu));
 #pragma unroll
-			for (uint32_t k = 0; k < kGroup; ++k) {
-				const uint32_t p = threadIdx.x + (k0 + k) * kThreads;
-				key[k] = line[p / kLineBins];
-				c[k] = n[p];
-			}
-#pragma unroll
-			for (uint32_t k = 0; k < kGroup; ++k) {
-				const uint32_t p = threadIdx.x + (k0 + k) * kThreads;
-				if (key[k] != kEmpty && c[k] != 0u)
-					n[p] = atomicAdd(&cnt[key[k] * kLineBins + p % kLineBins], c[k]);
-			}
-		}
-		__syncthreads();
-#pragma unroll
-		for (uint32_t u = 0; u < kU; ++u) {
-			const uint64_t f = base + (uint64_t)u * kThreads + threadIdx.x;
-			if (bin[u] != kEmpty)
-				node[f] = make_uint2(bin[u], slot[u] != kEmpty ? n[slot[u]] + local[u] : local[u]);
-		}
-		__syncthreads();
-		for (uint32_t i = threadIdx.x; i < kLines; i += kThreads)
-			line[i] = kEmpty;
-		for (uint32_t i = threadIdx.x; i < kLines * kLineBins; i += kThreads)
-			n[i] = 0u;
-		__syncthreads();
+		for (uint32_t v = 0; v < kV; ++v)
+			if (i0 + v * 64u + lane < n)
+				rt[i0 + v * 64u + lane] = r[v];
 	}
 }
 
-// Scatter every fragment to its place in its bin's bucket (aux[j] = first slot of bin j).
+// Every key to its place in its bin's bucket (aux[j] = first slot of bin j), a wave per tile.  The wave
+// first turns the tile's runs into slots in LDS, with the keys already on their way, so a tile costs
+// three dependent loads; then lane i finds key i's run by the heads at or below it, and the lanes of a
+// run write neighbouring slots.  Bound by latency and part-line writes: 35M keys in 127 us (190 us with
+// every lane loading its key's run and bin offset itself).
 __global__ void __launch_bounds__(kThreads)
-    build_scatter(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ fbeg, uint32_t S,
-                  const uint2 *__restrict__ node, const uint32_t *__restrict__ aux, uint2 *__restrict__ bucket) {
-	const uint64_t Ftot = fbeg[S];
-	const uint64_t stride = (uint64_t)gridDim.x * kThreads * kU;
-	uint32_t hint = 0;
-	for (uint64_t base = (uint64_t)blockIdx.x * kThreads * kU; base < Ftot; base += stride) {
-		FragSrc src[kU];
-		frag_sources(segs, fbeg, S, Ftot, base, hint, src);
-		uint2 fr[kU], np[kU];
+    scatter_runs(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ tbeg, uint32_t S,
+                 const uint32_t *__restrict__ keys, const uint64_t *__restrict__ heads,
+                 const uint2 *__restrict__ runs, const uint32_t *__restrict__ nrun, const uint32_t *__restrict__ aux,
+                 uint32_t *__restrict__ bucket) {
+	constexpr uint32_t kPer = kThreads / 64u, kV = 4; // tiles per block, runs per lane and trip
+	__shared__ uint32_t s_slot[kPer][kTile];          // run r: slot of key i of the run, less i
+	const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const uint64_t upto = (2ull << lane) - 1ull; // heads at or below the lane
+	const uint64_t tile = (uint64_t)blockIdx.x * kPer + wave;
+	if (tile >= tbeg[S])
+		return; // no block barrier follows
+	const uint32_t sc = S == 1u ? 0u : seg_find(tbeg, S, tile);
+	const uint64_t first = (tile - tbeg[sc]) * kTile, F = segs[sc].F;
+	const uint32_t n = F - first < kTile ? (uint32_t)(F - first) : kTile, nr = nrun[tile];
+	const uint2 *rt = runs + tile * kTile;
+	const uint64_t *ht = heads + tile * kHeads;
+	uint32_t *slot = s_slot[wave];
+	uint32_t key[kHeads];
 #pragma unroll
-		for (uint32_t u = 0; u < kU; ++u) {
-			const uint64_t f = base + (uint64_t)u * kThreads + threadIdx.x;
-			fr[u] = np[u] = make_uint2(0u, 0u);
-			if (src[u].frag) {
-				fr[u] = *src[u].frag;
-				np[u] = node[f];
-			}
-		}
-		uint32_t first[kU];
+	for (uint32_t v = 0; v < kHeads; ++v)
+		key[v] = v * 64u + lane < n ? keys[tile * kTile + v * 64u + lane] : 0u;
+	for (uint32_t i0 = 0; i0 < nr; i0 += 64u * kV) {
+		uint2 r[kV];
+		uint32_t a[kV];
 #pragma unroll
-		for (uint32_t u = 0; u < kU; ++u)
-			first[u] = src[u].frag ? aux[np[u].x] : 0u;
+		for (uint32_t v = 0; v < kV; ++v)
+			r[v] = i0 + v * 64u + lane < nr ? rt[i0 + v * 64u + lane] : make_uint2(0u, 0u);
 #pragma unroll
-		for (uint32_t u = 0; u < kU; ++u)
-			if (src[u].frag)
-				bucket[first[u] + np[u].y] = fr[u];
+		for (uint32_t v = 0; v < kV; ++v)
+			a[v] = i0 + v * 64u + lane < nr ? aux[r[v].x] : 0u;
+#pragma unroll
+		for (uint32_t v = 0; v < kV; ++v)
+			if (i0 + v * 64u + lane < nr)
+				slot[i0 + v * 64u + lane] = a[v] + r[v].y;
 	}
-}
-
-// ceil(2^32 / w): floor(a / w) = umulhi(a, kDivMagic[w]) for a < 2^14 and 2 <= w <= 64 (checked
-// exhaustively), the only divisions the colour fold needs.
-__constant__ uint32_t kDivMagic[65] = {
-    0u,         0u,         2147483648u, 1431655766u, 1073741824u, 858993460u, 715827883u, 613566757u, 536870912u,
-    477218589u, 429496730u, 390451573u,  357913942u,  330382100u,  306783379u, 286331154u, 268435456u, 252645136u,
-    238609295u, 226050911u, 214748365u,  204522253u,  195225787u,  186737709u, 178956971u, 171798692u, 165191050u,
-    159072863u, 153391690u, 148102321u,  143165577u,  138547333u,  134217728u, 130150525u, 126322568u, 122713352u,
-    119304648u, 116080198u, 113025456u,  110127367u,  107374183u,  104755300u, 102261127u, 99882961u,  97612894u,
-    95443718u,  93368855u,  91382283u,   89478486u,   87652394u,   85899346u,  84215046u,  82595525u,  81037119u,
-    79536432u,  78090315u,  76695845u,   75350304u,   74051161u,   72796056u,  71582789u,  70409300u,  69273667u,
-    68174085u,  67108864u};
-
-// Running average of the reference's CAS loop (octree_tag_node.comp:43-57): fold colour c into
-// leaf word prev (0 = empty leaf).  The word's 6-bit count n = min(a, 63) after a fragments is the
-// weight the next fragment meets: avg' = (avg * n + c) / (n + 1) per channel, count' = min(n + 1, 63).
-// magic = kDivMagic staged in LDS (a per-lane index into __constant__ memory would be a global load).
-__device__ __forceinline__ uint32_t fold_word(uint32_t prev, uint32_t c, const uint32_t *magic) {
-	if (prev == 0u)
-		return 0xC1000000u | c;
-	const uint32_t n = (prev >> 24u) & 0x3fu, w = n + 1u, m = magic[w];
-	const uint32_t r = __umulhi((prev & 0xffu) * n + (c & 0xffu), m);
-	const uint32_t g = __umulhi(((prev >> 8u) & 0xffu) * n + ((c >> 8u) & 0xffu), m);
-	const uint32_t b = __umulhi(((prev >> 16u) & 0xffu) * n + ((c >> 16u) & 0xffu), m);
-	return (umin32(w, 0x3fu) << 24u) | (r & 0xffu) | ((g & 0xffu) << 8u) | ((b & 0xffu) << 16u) | 0xC0000000u;
-}
-
-// Stages the division table in LDS; every thread of the block must call it.
-__device__ __forceinline__ void stage_magic(uint32_t *s_magic) {
-	for (uint32_t i = threadIdx.x; i < 65u; i += blockDim.x)
-		s_magic[i] = kDivMagic[i];
-	__syncthreads();
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+	uint32_t before = 0u; // runs that start before these 64 keys
+#pragma unroll
+	for (uint32_t v = 0; v < kHeads; ++v) {
+		const uint32_t i = v * 64u + lane;
+		const uint64_t h = ht[v]; // the last tile's heads are zero past its end
+		if (i < n)
+			bucket[slot[before + (uint32_t)__popcll(h & upto) - 1u] + i] = key[v];
+		before += (uint32_t)__popcll(h);
+	}
 }
 
 // The leaf a fragment key belongs to inside its block (child slot at depth L).
@@ -683,20 +724,6 @@ __device__ __forceinline__ uint32_t key_slot(uint64_t key, uint32_t res) {
 	uint32_t x, y, z;
 	decode_frag(make_uint2((uint32_t)(key >> 32), (uint32_t)key), res, x, y, z);
 	return (x & 1u) | ((y & 1u) << 1u) | ((z & 1u) << 2u);
-}
-
-// Folds one key (in ascending key order) into the 8 leaf words of a block.  The slot is selected
-// without dynamic register indexing.
-__device__ __forceinline__ void slot_push(uint32_t (&w)[8], uint64_t key, uint32_t res, const uint32_t *magic) {
-	const uint32_t s = key_slot(key, res);
-	uint32_t cw = w[0];
-#pragma unroll
-	for (uint32_t t = 1; t < 8u; ++t)
-		cw = s == t ? w[t] : cw;
-	const uint32_t nw = fold_word(cw, (uint32_t)key & 0xffffffu, magic);
-#pragma unroll
-	for (uint32_t t = 0; t < 8u; ++t)
-		w[t] = s == t ? nw : w[t];
 }
 
 __device__ __forceinline__ void store_block(uint32_t *oct, uint64_t block, const uint32_t (&w)[8]) {
@@ -724,76 +751,159 @@ struct LeafTarget {
 	uint32_t *oct;
 	uint64_t block;
 	uint32_t res;
+	const uint2 *raw; // a raw scene's fragments, else null
 };
 __device__ __forceinline__ LeafTarget leaf_target(const BuildSeg &g, const uint64_t *bbeg, uint32_t s, uint32_t j) {
 	const uint32_t L = g.L;
-	return LeafTarget{g.words, (uint64_t)(L == 1u ? 0u : g.fb[L - 1u]) + (j - bbeg[s]), 1u << L};
+	return LeafTarget{g.words, (uint64_t)(L == 1u ? 0u : g.fb[L - 1u]) + (j - bbeg[s]), 1u << L, g.raw ? g.frags : nullptr};
 }
 
-// One thread per leaf block with at most 16 fragments: sorted by the 64-bit fragment in registers
-// (5-, 19- or 63-comparator networks, +inf padding), then folded in that order into the 8 leaves;
-// the whole block is written, empty leaves as 0.  Each block of threads first orders its 256 leaf
-// blocks by size class in LDS, so that most waves run a single network.
-template <uint32_t kN>
-__device__ __forceinline__ void fold_small(const uint2 *__restrict__ b, uint32_t n, uint32_t res, const uint32_t *magic,
-                                           uint32_t (&w)[8]) {
-	uint64_t k[kN];
-#pragma unroll
-	for (uint32_t a = 0; a < kN; ++a)
-		k[a] = a < n ? frag_key(b[a]) : ~0ull;
-	if (kN == 4) {
-		cmp_swap(k[0], k[1]), cmp_swap(k[2], k[3]), cmp_swap(k[0], k[2]), cmp_swap(k[1], k[3]), cmp_swap(k[1], k[2]);
-	} else if (kN == 8) {
-		cmp_swap(k[0], k[1]), cmp_swap(k[2], k[3]), cmp_swap(k[4], k[5]), cmp_swap(k[6], k[7]);
-		cmp_swap(k[0], k[2]), cmp_swap(k[1], k[3]), cmp_swap(k[4], k[6]), cmp_swap(k[5], k[7]);
-		cmp_swap(k[1], k[2]), cmp_swap(k[5], k[6]), cmp_swap(k[0], k[4]), cmp_swap(k[3], k[7]);
-		cmp_swap(k[1], k[5]), cmp_swap(k[2], k[6]);
-		cmp_swap(k[1], k[4]), cmp_swap(k[3], k[6]);
-		cmp_swap(k[2], k[4]), cmp_swap(k[3], k[5]);
-		cmp_swap(k[3], k[4]);
-	} else { // Batcher odd-even merge sort of 16
-		cmp_swap(k[0], k[1]), cmp_swap(k[2], k[3]), cmp_swap(k[0], k[2]), cmp_swap(k[1], k[3]);
-		cmp_swap(k[1], k[2]), cmp_swap(k[4], k[5]), cmp_swap(k[6], k[7]), cmp_swap(k[4], k[6]);
-		cmp_swap(k[5], k[7]), cmp_swap(k[5], k[6]), cmp_swap(k[0], k[4]), cmp_swap(k[2], k[6]);
-		cmp_swap(k[2], k[4]), cmp_swap(k[1], k[5]), cmp_swap(k[3], k[7]), cmp_swap(k[3], k[5]);
-		cmp_swap(k[1], k[2]), cmp_swap(k[3], k[4]), cmp_swap(k[5], k[6]), cmp_swap(k[8], k[9]);
-		cmp_swap(k[10], k[11]), cmp_swap(k[8], k[10]), cmp_swap(k[9], k[11]), cmp_swap(k[9], k[10]);
-		cmp_swap(k[12], k[13]), cmp_swap(k[14], k[15]), cmp_swap(k[12], k[14]), cmp_swap(k[13], k[15]);
-		cmp_swap(k[13], k[14]), cmp_swap(k[8], k[12]), cmp_swap(k[10], k[14]), cmp_swap(k[10], k[12]);
-		cmp_swap(k[9], k[13]), cmp_swap(k[11], k[15]), cmp_swap(k[11], k[13]), cmp_swap(k[9], k[10]);
-		cmp_swap(k[11], k[12]), cmp_swap(k[13], k[14]), cmp_swap(k[0], k[8]), cmp_swap(k[4], k[12]);
-		cmp_swap(k[4], k[8]), cmp_swap(k[2], k[10]), cmp_swap(k[6], k[14]), cmp_swap(k[6], k[10]);
-		cmp_swap(k[2], k[4]), cmp_swap(k[6], k[8]), cmp_swap(k[10], k[12]), cmp_swap(k[1], k[9]);
-		cmp_swap(k[5], k[13]), cmp_swap(k[5], k[9]), cmp_swap(k[3], k[11]), cmp_swap(k[7], k[15]);
-		cmp_swap(k[7], k[11]), cmp_swap(k[3], k[5]), cmp_swap(k[7], k[9]), cmp_swap(k[11], k[13]);
-		cmp_swap(k[1], k[2]), cmp_swap(k[3], k[4]), cmp_swap(k[5], k[6]), cmp_swap(k[7], k[8]);
-		cmp_swap(k[9], k[10]), cmp_swap(k[11], k[12]), cmp_swap(k[13], k[14]);
+__device__ __forceinline__ void cmp_swap32(uint32_t &x, uint32_t &y) {
+	const uint32_t lo = umin32(x, y), hi = umax32(x, y);
+	x = lo;
+	y = hi;
+}
+
+// The reference's running average of one leaf (octree_tag_node.comp:43-57), channels as floats: the
+// n-th fragment (from 0, weight min(n, 63)) gives floor((avg * n + c) / (n + 1)).  The numerator is below
+// 2^14 and the divisor at most 64, so (numerator + 1/2) / divisor is at least 1/128 away from an
+// integer, and a reciprocal off by a few ulp gives the exact floor.
+struct LeafMean {
+	float r, g, b, n;
+	__device__ __forceinline__ void clear() { r = g = b = n = 0.0f; }
+	__device__ __forceinline__ void add(uint32_t rgb) {
+		const float w = n + 1.0f, inv = __builtin_amdgcn_rcpf(w), half = 0.5f * inv;
+		r = __builtin_floorf(__builtin_fmaf(__builtin_fmaf(r, n, (float)(rgb & 0xffu)), inv, half));
+		g = __builtin_floorf(__builtin_fmaf(__builtin_fmaf(g, n, (float)(rgb >> 8u & 0xffu)), inv, half));
+		b = __builtin_floorf(__builtin_fmaf(__builtin_fmaf(b, n, (float)(rgb >> 16u & 0xffu)), inv, half));
+		n = __builtin_fminf(w, 63.0f);
 	}
+	__device__ __forceinline__ uint32_t word() const {
+		uint32_t v = __builtin_amdgcn_cvt_pk_u8_f32(r, 0u, 0u);
+		v = __builtin_amdgcn_cvt_pk_u8_f32(g, 1u, v);
+		v = __builtin_amdgcn_cvt_pk_u8_f32(b, 2u, v);
+		return __builtin_amdgcn_cvt_pk_u8_f32(n + 192.0f, 3u, v); // 0xC0 | n
+	}
+};
+
+// A leaf block of a raw scene (keys = fragment indices): leaf by leaf, by repeated minimum over the
+// whole fragments (equal fragments are folded together).  w: the block's leaf words, one per child
+// slot, stride kThreads.
+__device__ void fold_raw(const uint32_t *b, const uint2 *frags, uint32_t n, uint32_t res, uint32_t *w) {
+#pragma unroll 1
+	for (uint32_t slot = 0; slot < 8u; ++slot) {
+		LeafMean leaf;
+		leaf.clear();
+		uint64_t last = 0;
+		bool any = false;
+		for (;;) {
+			uint64_t best = ~0ull;
+			uint32_t same = 0u;
+#pragma unroll 1
+			for (uint32_t i = 0; i < n; ++i) {
+				const uint64_t k = frag_key(frags[b[i]]);
+				if (key_slot(k, res) != slot || (any && k <= last) || k > best)
+					continue;
+				same = k == best ? same + 1u : 1u;
+				best = k;
+			}
+			if (!same)
+				break;
+			for (uint32_t i = 0; i < same; ++i)
+				leaf.add((uint32_t)best);
+			last = best;
+			any = true;
+		}
+		if (any)
+			w[slot * kThreads] = leaf.word();
+	}
+}
+
+// One thread per leaf block with at most 16 fragments: leaf_keys sorted in registers (5-, 19- or
+// 63-comparator networks of v_min / v_max, +inf padding), then folded in that order, each leaf's word
+// going to the thread's LDS column; the whole block is written, empty leaves as 0.  Each block of
+// threads first orders its 256 leaf blocks by size class in LDS, so that most waves run a single
+// network; the next 256 sizes and bucket positions are loaded a step ahead.  Bound by the latency of its
+// loads (7 waves per SIMD): 7.2M leaf blocks of a room at 2^10 279 -> 133 us, 62M with slivers at 2^12
+// 1578 -> 825 us, against whole fragments, 64-bit comparators, leaf words in registers and integer
+// division.  Staging the buckets in LDS instead of each thread reading its own: 192 and 1211 us.
+template <uint32_t kN> __device__ __forceinline__ void fold_small(const uint32_t *b, uint32_t n, uint32_t *w) {
+	uint32_t k[kN];
 #pragma unroll
 	for (uint32_t a = 0; a < kN; ++a)
-		if (a < n)
-			slot_push(w, k[a], res, magic);
+		k[a] = a < n ? b[a] : kRawKey;
+	if (kN == 4) {
+		cmp_swap32(k[0], k[1]), cmp_swap32(k[2], k[3]), cmp_swap32(k[0], k[2]), cmp_swap32(k[1], k[3]);
+		cmp_swap32(k[1], k[2]);
+	} else if (kN == 8) {
+		cmp_swap32(k[0], k[1]), cmp_swap32(k[2], k[3]), cmp_swap32(k[4], k[5]), cmp_swap32(k[6], k[7]);
+		cmp_swap32(k[0], k[2]), cmp_swap32(k[1], k[3]), cmp_swap32(k[4], k[6]), cmp_swap32(k[5], k[7]);
+		cmp_swap32(k[1], k[2]), cmp_swap32(k[5], k[6]), cmp_swap32(k[0], k[4]), cmp_swap32(k[3], k[7]);
+		cmp_swap32(k[1], k[5]), cmp_swap32(k[2], k[6]);
+		cmp_swap32(k[1], k[4]), cmp_swap32(k[3], k[6]);
+		cmp_swap32(k[2], k[4]), cmp_swap32(k[3], k[5]);
+		cmp_swap32(k[3], k[4]);
+	} else { // Batcher odd-even merge sort of 16
+		cmp_swap32(k[0], k[1]), cmp_swap32(k[2], k[3]), cmp_swap32(k[0], k[2]), cmp_swap32(k[1], k[3]);
+		cmp_swap32(k[1], k[2]), cmp_swap32(k[4], k[5]), cmp_swap32(k[6], k[7]), cmp_swap32(k[4], k[6]);
+		cmp_swap32(k[5], k[7]), cmp_swap32(k[5], k[6]), cmp_swap32(k[0], k[4]), cmp_swap32(k[2], k[6]);
+		cmp_swap32(k[2], k[4]), cmp_swap32(k[1], k[5]), cmp_swap32(k[3], k[7]), cmp_swap32(k[3], k[5]);
+		cmp_swap32(k[1], k[2]), cmp_swap32(k[3], k[4]), cmp_swap32(k[5], k[6]), cmp_swap32(k[8], k[9]);
+		cmp_swap32(k[10], k[11]), cmp_swap32(k[8], k[10]), cmp_swap32(k[9], k[11]), cmp_swap32(k[9], k[10]);
+		cmp_swap32(k[12], k[13]), cmp_swap32(k[14], k[15]), cmp_swap32(k[12], k[14]), cmp_swap32(k[13], k[15]);
+		cmp_swap32(k[13], k[14]), cmp_swap32(k[8], k[12]), cmp_swap32(k[10], k[14]), cmp_swap32(k[10], k[12]);
+		cmp_swap32(k[9], k[13]), cmp_swap32(k[11], k[15]), cmp_swap32(k[11], k[13]), cmp_swap32(k[9], k[10]);
+		cmp_swap32(k[11], k[12]), cmp_swap32(k[13], k[14]), cmp_swap32(k[0], k[8]), cmp_swap32(k[4], k[12]);
+		cmp_swap32(k[4], k[8]), cmp_swap32(k[2], k[10]), cmp_swap32(k[6], k[14]), cmp_swap32(k[6], k[10]);
+		cmp_swap32(k[2], k[4]), cmp_swap32(k[6], k[8]), cmp_swap32(k[10], k[12]), cmp_swap32(k[1], k[9]);
+		cmp_swap32(k[5], k[13]), cmp_swap32(k[5], k[9]), cmp_swap32(k[3], k[11]), cmp_swap32(k[7], k[15]);
+		cmp_swap32(k[7], k[11]), cmp_swap32(k[3], k[5]), cmp_swap32(k[7], k[9]), cmp_swap32(k[11], k[13]);
+		cmp_swap32(k[1], k[2]), cmp_swap32(k[3], k[4]), cmp_swap32(k[5], k[6]), cmp_swap32(k[7], k[8]);
+		cmp_swap32(k[9], k[10]), cmp_swap32(k[11], k[12]), cmp_swap32(k[13], k[14]);
+	}
+	LeafMean leaf;
+	leaf.clear();
+	uint32_t slot = 8u;
+#pragma unroll
+	for (uint32_t a = 0; a < kN; ++a)
+		if (a < n) {
+			const uint32_t s = k[a] >> 27u;
+			if (s != slot)
+				leaf.clear();
+			slot = s;
+			leaf.add(k[a]);
+			w[s * kThreads] = leaf.word();
+		}
 }
 
 __global__ void __launch_bounds__(kThreads)
     build_fold(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ bbeg, uint32_t S,
-               const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ aux, const uint2 *__restrict__ bucket,
+               const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ aux, const uint32_t *__restrict__ bucket,
                uint32_t *list, uint64_t cap) {
 	const uint64_t nbins = bbeg[S];
 	constexpr uint32_t kWaves = kThreads / 64;
-	__shared__ uint32_t s_magic[65];
 	__shared__ uint32_t s_bin[kThreads], s_n[kThreads];
 	__shared__ uint32_t s_cls[kWaves][3];
-	stage_magic(s_magic);
+	__shared__ uint32_t s_leaf[8 * kThreads]; // the threads' leaf words, by child slot
+	__shared__ uint32_t s_at[kThreads];       // first slot of the bin's bucket
 	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
 	const uint64_t below = (1ull << lane) - 1ull;
 	const uint64_t stride = (uint64_t)gridDim.x * kThreads;
-	uint32_t hint = 0;
+	uint32_t hint = 0, next_n = 0u, next_slot = 0u; // loaded one step ahead
+	auto ahead = [&](uint64_t at) {
+		if (at + threadIdx.x < nbins) {
+			next_n = cnt[at + threadIdx.x];
+			next_slot = aux[at + threadIdx.x];
+		}
+	};
+	ahead((uint64_t)blockIdx.x * kThreads);
 	for (uint64_t base = (uint64_t)blockIdx.x * kThreads; base < nbins; base += stride) {
 		const uint64_t jj = base + threadIdx.x;
-		uint32_t n = 0, cls = 3; // classes: <= 4, <= 8, <= 16 fragments; 3 = not folded here
+		const uint32_t n = next_n, slot0 = next_slot;
+		uint32_t cls = 3; // classes: <= 4, <= 8, <= 16 fragments; 3 = not folded here
+		if (base + stride < nbins)
+			ahead(base + stride);
 		if (jj < nbins) {
-			n = cnt[jj];
 			cls = n <= 4u ? 0u : n <= 8u ? 1u : n <= kRegBucket ? 2u : 3u;
 		}
 		const bool rest = jj < nbins && cls == 3u;
@@ -820,62 +930,65 @@ __global__ void __launch_bounds__(kThreads)
 			pos += (uint32_t)__popcll(mine & below);
 			s_bin[pos] = (uint32_t)jj;
 			s_n[pos] = n;
+			s_at[pos] = slot0;
 		}
 		__syncthreads();
 		if (threadIdx.x < total) {
 			const uint32_t j = s_bin[threadIdx.x], nj = s_n[threadIdx.x];
 			LeafTarget t;
 			with_seg<kThreads>(bbeg, S, hint, base, j, [&](uint32_t s) { t = leaf_target(segs[s], bbeg, s, j); });
-			const uint2 *b = bucket + aux[j];
-			uint32_t w[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-			if (nj <= 4u)
-				fold_small<4>(b, nj, t.res, s_magic, w);
+			uint32_t *w = s_leaf + threadIdx.x;
+#pragma unroll
+			for (uint32_t c = 0; c < 8u; ++c)
+				w[c * kThreads] = 0u;
+			const uint32_t at = s_at[threadIdx.x];
+			if (t.raw)
+				fold_raw(bucket + at, t.raw, nj, t.res, w);
+			else if (nj <= 4u)
+				fold_small<4>(bucket + at, nj, w);
 			else if (nj <= 8u)
-				fold_small<8>(b, nj, t.res, s_magic, w);
+				fold_small<8>(bucket + at, nj, w);
 			else
-				fold_small<16>(b, nj, t.res, s_magic, w);
-			store_block(t.oct, t.block, w);
+				fold_small<16>(bucket + at, nj, w);
+			uint32_t words[8];
+#pragma unroll
+			for (uint32_t c = 0; c < 8u; ++c)
+				words[c] = w[c * kThreads];
+			store_block(t.oct, t.block, words);
 		}
 		__syncthreads();
 	}
 }
 
-// Bitonic sort of m = 2^p keys (ascending) by one block; every comparator puts the minimum at the
-// lower index, so keys past the end behave as +infinity padding.
-template <class Get, class Put> __device__ void block_bitonic(uint32_t n, uint32_t m, Get get, Put put) {
-	for (uint32_t k = 2; k <= m; k <<= 1) {
-		for (uint32_t jj = k >> 1; jj > 0; jj >>= 1) {
-			for (uint32_t t = threadIdx.x; t < m / 2; t += blockDim.x) {
-				const uint32_t blk = t / jj, off = t % jj;
-				uint32_t a, b;
-				if (jj == (k >> 1)) { // first step of a merge: flip
-					a = blk * k + off;
-					b = blk * k + k - 1u - off;
-				} else {
-					a = blk * 2u * jj + off;
-					b = a + jj;
-				}
-				if (b < n) {
-					const uint64_t va = get(a), vb = get(b);
-					if (vb < va) {
-						put(a, vb);
-						put(b, va);
-					}
-				}
-			}
-			__syncthreads();
-		}
-	}
+// Index pair (a, b), a < b, of comparator t at distance jj of a bitonic merge to k, in the form whose
+// comparators all put the minimum at the lower index, so keys past the end behave as +infinity padding.
+__device__ __forceinline__ void bitonic_pair(uint32_t t, uint32_t k, uint32_t jj, uint32_t &a, uint32_t &b) {
+	const uint32_t blk = t / jj, off = t % jj;
+	const bool flip = jj == (k >> 1); // first step of a merge
+	a = flip ? blk * k + off : blk * 2u * jj + off;
+	b = flip ? blk * k + k - 1u - off : a + jj;
 }
 
-// Leaf blocks of 17..64 fragments, one wave each: lane i holds key i and its leaf slot (padding:
-// slot 8, key +inf); a bitonic sort over lane shuffles orders them by (slot, key), so every leaf's
-// fragments are consecutive and ascending.  Lane s < 8 then folds the run of slot s from LDS.
-// Blocks blk of nblk of the list launch; s_col: 64 words of LDS per wave.
+// Folds keys [beg, end) of one leaf, ascending; rgb(i) = colour of key i.
+template <class Rgb> __device__ __forceinline__ uint32_t fold_run(uint32_t beg, uint32_t end, Rgb rgb) {
+	if (beg >= end)
+		return 0u;
+	LeafMean leaf;
+	leaf.clear();
+	for (uint32_t i = beg; i < end; ++i)
+		leaf.add(rgb(i));
+	return leaf.word();
+}
+
+// Leaf blocks of 17..64 fragments, one wave each: lane i holds key i (padding: +inf); a bitonic sort over
+// lane shuffles orders them by leaf slot and key, so every leaf's fragments are consecutive and
+// ascending.  Lane s < 8 then folds the run of slot s from LDS.  A raw scene's wave sorts
+// (slot, whole fragment) pairs instead.  Blocks blk of nblk of the list launch; s_col: 64 words of LDS
+// per wave.
 __device__ void fold_mid_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__restrict__ segs,
                                 const uint64_t *__restrict__ bbeg, uint32_t S, const uint32_t *__restrict__ cnt,
-                                const uint32_t *__restrict__ aux, const uint2 *__restrict__ bucket, const uint32_t *list,
-                                uint64_t cap, uint32_t (*s_col)[64], const uint32_t *s_magic) {
+                                const uint32_t *__restrict__ aux, const uint32_t *__restrict__ bucket,
+                                const uint32_t *list, uint64_t cap, uint32_t (*s_col)[64]) {
 	constexpr uint32_t kWaves = kThreads / 64;
 	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
 	uint64_t count = list[0];
@@ -889,26 +1002,39 @@ __device__ void fold_mid_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__r
 		const uint32_t n = cnt[j];
 		const uint32_t s = S == 1u ? 0u : seg_find(bbeg, S, j);
 		const LeafTarget t = leaf_target(segs[s], bbeg, s, j);
-		uint64_t key = ~0ull;
-		uint32_t slot = 8u;
-		if (lane < n) {
-			key = frag_key(bucket[aux[j] + lane]);
-			slot = key_slot(key, t.res);
-		}
-#pragma unroll
-		for (uint32_t k = 2; k <= 64u; k <<= 1) {
-#pragma unroll
-			for (uint32_t d = k >> 1; d > 0u; d >>= 1) {
-				const uint64_t ok = __shfl_xor(key, (int)d, 64);
-				const uint32_t os = __shfl_xor(slot, (int)d, 64);
-				const bool other_less = os < slot || (os == slot && ok < key);
-				const bool take_min = ((lane & k) == 0u) == ((lane & d) == 0u);
-				const bool take_other = take_min == other_less;
-				key = take_other ? ok : key;
-				slot = take_other ? os : slot;
+		uint32_t key = lane < n ? bucket[aux[j] + lane] : kRawKey, slot = key >> 27u;
+		if (t.raw) { // wave-uniform
+			uint64_t whole = ~0ull;
+			slot = 8u;
+			if (lane < n) {
+				whole = frag_key(t.raw[key]);
+				slot = key_slot(whole, t.res);
 			}
+#pragma unroll 1
+			for (uint32_t k = 2; k <= 64u; k <<= 1)
+#pragma unroll 1
+				for (uint32_t d = k >> 1; d > 0u; d >>= 1) {
+					const uint64_t ok = __shfl_xor(whole, (int)d, 64);
+					const uint32_t os = __shfl_xor(slot, (int)d, 64);
+					const bool other_less = os < slot || (os == slot && ok < whole);
+					const bool take_min = ((lane & k) == 0u) == ((lane & d) == 0u);
+					const bool take_other = take_min == other_less;
+					whole = take_other ? ok : whole;
+					slot = take_other ? os : slot;
+				}
+			key = (uint32_t)whole;
+		} else {
+#pragma unroll
+			for (uint32_t k = 2; k <= 64u; k <<= 1)
+#pragma unroll
+				for (uint32_t d = k >> 1; d > 0u; d >>= 1) {
+					const uint32_t ok = __shfl_xor(key, (int)d, 64);
+					const bool take_min = ((lane & k) == 0u) == ((lane & d) == 0u);
+					key = take_min ? umin32(key, ok) : umax32(key, ok);
+				}
+			slot = key >> 27u;
 		}
-		s_col[wave][lane] = (uint32_t)key & 0xffffffu;
+		s_col[wave][lane] = key & 0xffffffu;
 		__builtin_amdgcn_wave_barrier();
 		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
 		uint64_t run = 0;
@@ -918,33 +1044,104 @@ __device__ void fold_mid_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__r
 			run = lane == u ? mu : run;
 		}
 		if (lane < 8u) {
-			uint32_t word = 0u;
-			if (run) {
-				const uint32_t beg = (uint32_t)__ffsll((unsigned long long)run) - 1u, len = (uint32_t)__popcll(run);
-				for (uint32_t i = beg; i < beg + len; ++i)
-					word = fold_word(word, s_col[wave][i], s_magic);
-			}
-			t.oct[8u * t.block + lane] = word;
+			const uint32_t beg = run ? (uint32_t)__ffsll((unsigned long long)run) - 1u : 0u;
+			t.oct[8u * t.block + lane] =
+			    fold_run(beg, beg + (uint32_t)__popcll(run), [&](uint32_t i) { return s_col[wave][i]; });
 		}
 		__builtin_amdgcn_wave_barrier();
 	}
 }
 
-// Leaf blocks of 65..512 fragments, one wave each: the (slot, key) pairs, padded to a power of two
-// with (8, +inf), are bitonic-sorted in the wave's LDS (no block barriers: the wave's LDS accesses
-// are ordered between stages by wave barriers), so every leaf's fragments are consecutive and
-// ascending; lane s < 8 then folds the run of slot s.
+// Bitonic sort of n (<= m = 2^p) keys in LDS by kStep lanes (one wave, or the block); sync() separates
+// the stages.
+template <uint32_t kStep, class Less, class Swap, class Sync>
+__device__ __forceinline__ void lds_bitonic(uint32_t n, uint32_t m, uint32_t lane, Less less, Swap swap, Sync sync) {
+	for (uint32_t k = 2; k <= m; k <<= 1)
+		for (uint32_t jj = k >> 1; jj > 0; jj >>= 1) {
+			for (uint32_t q = lane; q < m / 2u; q += kStep) {
+				uint32_t a, b;
+				bitonic_pair(q, k, jj, a, b);
+				if (b < n && less(b, a))
+					swap(a, b);
+			}
+			sync();
+		}
+}
 
-// Blocks blk of nblk of the list launch; s_keys / s_slots: kWideBucket entries per wave.
+// Sorts the n keys of one leaf block in LDS and finds the runs of its 8 leaves: s_beg / s_end[slot].
+// keys32: leaf_keys (or, of a raw scene, fragment indices on entry); keys64, slots: a raw scene's
+// whole fragments.  Called by kStep lanes.
+template <uint32_t kStep, class Sync>
+__device__ __forceinline__ void sort_leaves(uint32_t n, uint32_t lane, const LeafTarget &t,
+                                            const uint32_t *__restrict__ b, uint64_t *keys64, uint8_t *slots,
+                                            uint32_t *s_beg, uint32_t *s_end, Sync sync) {
+	uint32_t *keys32 = reinterpret_cast<uint32_t *>(keys64);
+	uint32_t m = 1u;
+	while (m < n)
+		m <<= 1;
+	if (lane < 8u)
+		s_beg[lane] = s_end[lane] = 0u;
+	if (t.raw) {
+		for (uint32_t i = lane; i < n; i += kStep) {
+			const uint64_t key = frag_key(t.raw[b[i]]);
+			keys64[i] = key;
+			slots[i] = (uint8_t)key_slot(key, t.res);
+		}
+		sync();
+		lds_bitonic<kStep>(
+		    n, m, lane,
+		    [&](uint32_t x, uint32_t y) { return slots[x] < slots[y] || (slots[x] == slots[y] && keys64[x] < keys64[y]); },
+		    [&](uint32_t x, uint32_t y) {
+			    const uint64_t kx = keys64[x];
+			    const uint8_t sx = slots[x];
+			    keys64[x] = keys64[y], keys64[y] = kx;
+			    slots[x] = slots[y], slots[y] = sx;
+		    },
+		    sync);
+	} else {
+		for (uint32_t i = lane; i < n; i += kStep)
+			keys32[i] = b[i];
+		sync();
+		for (uint32_t k = 2; k <= m; k <<= 1)
+			for (uint32_t jj = k >> 1; jj > 0; jj >>= 1) {
+				for (uint32_t q = lane; q < m / 2u; q += kStep) {
+					uint32_t x, y;
+					bitonic_pair(q, k, jj, x, y);
+					if (y < n) {
+						const uint32_t kx = keys32[x], ky = keys32[y];
+						if (ky < kx)
+							keys32[x] = ky, keys32[y] = kx;
+					}
+				}
+				sync();
+			}
+	}
+	auto slot_of = [&](uint32_t i) { return t.raw ? (uint32_t)slots[i] : keys32[i] >> 27u; };
+	for (uint32_t i = lane; i < n; i += kStep) {
+		const uint32_t sl = slot_of(i);
+		if (i == 0u || slot_of(i - 1u) != sl)
+			s_beg[sl] = i;
+		if (i + 1u == n || slot_of(i + 1u) != sl)
+			s_end[sl] = i + 1u;
+	}
+	sync();
+	if (lane < 8u)
+		t.oct[8u * t.block + lane] = fold_run(s_beg[lane], s_end[lane], [&](uint32_t i) {
+			return (t.raw ? (uint32_t)keys64[i] : keys32[i]) & 0xffffffu;
+		});
+	sync();
+}
+
+// Leaf blocks of 65..512 fragments, one wave each, sorted in the wave's LDS (no block barriers: the
+// wave's LDS accesses are ordered between stages by wave barriers).  Blocks blk of nblk of the list
+// launch; s_keys / s_slots: kWideBucket entries per wave.
 __device__ void fold_wide_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__restrict__ segs,
                                  const uint64_t *__restrict__ bbeg, uint32_t S, const uint32_t *__restrict__ cnt,
-                                 const uint32_t *__restrict__ aux, const uint2 *__restrict__ bucket, const uint32_t *list,
-                                 uint64_t cap, uint64_t *s_keys, uint8_t *s_slots, uint32_t (*s_beg)[8],
-                                 uint32_t (*s_end)[8], const uint32_t *s_magic) {
+                                 const uint32_t *__restrict__ aux, const uint32_t *__restrict__ bucket,
+                                 const uint32_t *list, uint64_t cap, uint64_t *s_keys, uint8_t *s_slots,
+                                 uint32_t (*s_beg)[8], uint32_t (*s_end)[8]) {
 	constexpr uint32_t kWaves = kThreads / 64;
 	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-	uint64_t *keys = s_keys + wave * kWideBucket;
-	uint8_t *slots = s_slots + wave * kWideBucket;
 	uint64_t count = list[2];
 	if (count > cap)
 		count = cap;
@@ -953,102 +1150,24 @@ __device__ void fold_wide_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__
 		if (item >= count)
 			break; // wave-uniform; no block barrier follows
 		const uint32_t j = list[3u + 2u * cap + item];
-		const uint32_t n = cnt[j];
 		const uint32_t s = S == 1u ? 0u : seg_find(bbeg, S, j);
 		const LeafTarget t = leaf_target(segs[s], bbeg, s, j);
-		const uint2 *b = bucket + aux[j];
-		uint32_t m = 128u;
-		while (m < n)
-			m <<= 1;
-		for (uint32_t i = lane; i < m; i += 64u) {
-			const uint64_t key = i < n ? frag_key(b[i]) : ~0ull;
-			keys[i] = key;
-			slots[i] = (uint8_t)(i < n ? key_slot(key, t.res) : 8u);
-		}
-		if (lane < 8u)
-			s_beg[wave][lane] = s_end[wave][lane] = 0u;
-		__builtin_amdgcn_wave_barrier();
-		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-		for (uint32_t k = 2; k <= m; k <<= 1) {
-			for (uint32_t jj = k >> 1; jj > 0; jj >>= 1) {
-				for (uint32_t q = lane; q < m / 2u; q += 64u) {
-					const uint32_t blk = q / jj, off = q % jj;
-					const uint32_t a = jj == (k >> 1) ? blk * k + off : blk * 2u * jj + off;
-					const uint32_t c = jj == (k >> 1) ? blk * k + k - 1u - off : a + jj;
-					const uint64_t ka = keys[a], kc = keys[c];
-					const uint8_t sa = slots[a], sc = slots[c];
-					if (sc < sa || (sc == sa && kc < ka)) {
-						keys[a] = kc;
-						keys[c] = ka;
-						slots[a] = sc;
-						slots[c] = sa;
-					}
-				}
-				__builtin_amdgcn_wave_barrier();
-				__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-			}
-		}
-		for (uint32_t i = lane; i < n; i += 64u) {
-			const uint32_t sl = slots[i];
-			if (i == 0u || slots[i - 1u] != sl)
-				s_beg[wave][sl] = i;
-			if (i + 1u == n || slots[i + 1u] != sl)
-				s_end[wave][sl] = i + 1u;
-		}
-		__builtin_amdgcn_wave_barrier();
-		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-		if (lane < 8u) {
-			uint32_t word = 0u;
-			for (uint32_t i = s_beg[wave][lane]; i < s_end[wave][lane]; ++i)
-				word = fold_word(word, (uint32_t)keys[i] & 0xffffffu, s_magic);
-			t.oct[8u * t.block + lane] = word;
-		}
-		__builtin_amdgcn_wave_barrier();
-		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+		sort_leaves<64u>(cnt[j], lane, t, bucket + aux[j], s_keys + wave * kWideBucket, s_slots + wave * kWideBucket,
+		                 s_beg[wave], s_end[wave], [] {
+			                 __builtin_amdgcn_wave_barrier();
+			                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+		                 });
 	}
 }
 
-// Bitonic sort of n (<= m = 2^p) (slot, key) pairs held in LDS by one block, ascending; pairs past
-// n behave as +infinity padding.
-__device__ void block_bitonic_kv(uint32_t n, uint32_t m, uint64_t *keys, uint8_t *slots) {
-	for (uint32_t k = 2; k <= m; k <<= 1) {
-		for (uint32_t jj = k >> 1; jj > 0; jj >>= 1) {
-			for (uint32_t t = threadIdx.x; t < m / 2; t += blockDim.x) {
-				const uint32_t blk = t / jj, off = t % jj;
-				uint32_t a, b;
-				if (jj == (k >> 1)) { // first step of a merge: flip
-					a = blk * k + off;
-					b = blk * k + k - 1u - off;
-				} else {
-					a = blk * 2u * jj + off;
-					b = a + jj;
-				}
-				if (b < n) {
-					const uint64_t ka = keys[a], kb = keys[b];
-					const uint8_t sa = slots[a], sb = slots[b];
-					if (sb < sa || (sb == sa && kb < ka)) {
-						keys[a] = kb;
-						keys[b] = ka;
-						slots[a] = sb;
-						slots[b] = sa;
-					}
-				}
-			}
-			__syncthreads();
-		}
-	}
-}
-
-// Leaf blocks of more than 512 fragments, one block each.  Up to kLdsBucket fragments: bitonic sort
-// of the (slot, key) pairs in LDS, then lane s < 8 folds the run of slot s.  Beyond (a global-memory
-// sort, rare): keys sorted in place in the bucket and each of the 8 lanes walks all of them,
+// Leaf blocks of more than 512 fragments, one block each.  Up to kLdsBucket fragments: sorted in LDS.
+// Beyond (rare): the keys are sorted in place in the bucket and each of the 8 lanes walks all of them,
 // taking those of its slot.  Blocks blk of nblk of the list launch; s_keys / s_slots: kLdsBucket
 // entries for the block.
 __device__ void fold_big_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__restrict__ segs,
                                 const uint64_t *__restrict__ bbeg, uint32_t S, const uint32_t *__restrict__ cnt,
-                                const uint32_t *__restrict__ aux, uint2 *bucket, const uint32_t *list, uint64_t cap,
-                                uint64_t *s_keys, uint8_t *s_slots, uint32_t *s_beg, uint32_t *s_end,
-                                const uint32_t *s_magic) {
+                                const uint32_t *__restrict__ aux, uint32_t *bucket, const uint32_t *list, uint64_t cap,
+                                uint64_t *s_keys, uint8_t *s_slots, uint32_t *s_beg, uint32_t *s_end) {
 	uint64_t count = list[1];
 	if (count > cap)
 		count = cap;
@@ -1057,76 +1176,62 @@ __device__ void fold_big_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__r
 		const uint32_t n = cnt[j];
 		const uint32_t s = S == 1u ? 0u : seg_find(bbeg, S, j);
 		const LeafTarget t = leaf_target(segs[s], bbeg, s, j);
-		uint2 *b = bucket + aux[j];
-		uint32_t m = 1;
-		while (m < n)
-			m <<= 1;
+		uint32_t *b = bucket + aux[j];
 		if (n <= kLdsBucket) {
-			if (threadIdx.x < 8u)
-				s_beg[threadIdx.x] = s_end[threadIdx.x] = 0u;
-			for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-				const uint64_t key = frag_key(b[i]);
-				s_keys[i] = key;
-				s_slots[i] = (uint8_t)key_slot(key, t.res);
-			}
-			__syncthreads();
-			block_bitonic_kv(n, m, s_keys, s_slots);
-			for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-				const uint32_t sl = s_slots[i];
-				if (i == 0u || s_slots[i - 1u] != sl)
-					s_beg[sl] = i;
-				if (i + 1u == n || s_slots[i + 1u] != sl)
-					s_end[sl] = i + 1u;
-			}
-			__syncthreads();
-			if (threadIdx.x < 8u) {
-				uint32_t word = 0u;
-				for (uint32_t i = s_beg[threadIdx.x]; i < s_end[threadIdx.x]; ++i)
-					word = fold_word(word, (uint32_t)s_keys[i] & 0xffffffu, s_magic);
-				t.oct[8u * t.block + threadIdx.x] = word;
-			}
+			sort_leaves<kThreads>(n, threadIdx.x, t, b, s_keys, s_slots, s_beg, s_end, [] { __syncthreads(); });
 		} else {
-			block_bitonic(
-			    n, m, [&](uint32_t i) { return frag_key(b[i]); },
-			    [&](uint32_t i, uint64_t v) { b[i] = make_uint2((uint32_t)(v >> 32), (uint32_t)v); });
+			uint32_t m = 1;
+			while (m < n)
+				m <<= 1;
+			// order of an entry: the whole fragment of a raw scene's index, else the key itself
+			auto order = [&](uint32_t e) { return t.raw ? frag_key(t.raw[e]) : (uint64_t)e; };
+			lds_bitonic<kThreads>(
+			    n, m, threadIdx.x, [&](uint32_t x, uint32_t y) { return order(b[x]) < order(b[y]); },
+			    [&](uint32_t x, uint32_t y) {
+				    const uint32_t e = b[x];
+				    b[x] = b[y], b[y] = e;
+			    },
+			    [] { __syncthreads(); });
 			if (threadIdx.x < 8u) {
-				uint32_t word = 0u;
+				LeafMean leaf;
+				leaf.clear();
+				bool any = false;
 				for (uint32_t i = 0; i < n; ++i) {
-					const uint64_t key = frag_key(b[i]);
-					if (key_slot(key, t.res) == threadIdx.x)
-						word = fold_word(word, (uint32_t)key & 0xffffffu, s_magic);
+					const uint64_t key = order(b[i]);
+					const uint32_t slot = t.raw ? key_slot(key, t.res) : (uint32_t)key >> 27u;
+					if (slot == threadIdx.x) {
+						leaf.add((uint32_t)key);
+						any = true;
+					}
 				}
-				t.oct[8u * t.block + threadIdx.x] = word;
+				t.oct[8u * t.block + threadIdx.x] = any ? leaf.word() : 0u;
 			}
 		}
 		__syncthreads();
 	}
 }
 
-
 // The fold's three work lists in one launch: blocks [0, g_mid) take the 17..64-fragment leaf blocks,
 // the next g_wide the 65..512-fragment ones, the rest the larger ones.  Each role is block-uniform,
 // so the big role's block barriers are safe; the LDS is shared between the roles.
 __global__ void __launch_bounds__(kThreads)
     build_fold_lists(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ bbeg, uint32_t S,
-                     const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ aux, uint2 *bucket,
+                     const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ aux, uint32_t *bucket,
                      const uint32_t *list, uint64_t cap, uint32_t g_mid, uint32_t g_wide) {
 	constexpr uint32_t kWaves = kThreads / 64;
 	static_assert(kWaves * kWideBucket == kLdsBucket, "the wide and big roles share the key arrays");
-	__shared__ uint32_t s_magic[65];
 	__shared__ uint64_t s_keys[kLdsBucket];
 	__shared__ uint8_t s_slots[kLdsBucket];
 	__shared__ uint32_t s_beg[kWaves][8], s_end[kWaves][8];
-	stage_magic(s_magic);
 	if (blockIdx.x < g_mid)
 		fold_mid_blocks(blockIdx.x, g_mid, segs, bbeg, S, cnt, aux, bucket, list, cap,
-		                reinterpret_cast<uint32_t (*)[64]>(s_keys), s_magic);
+		                reinterpret_cast<uint32_t (*)[64]>(s_keys));
 	else if (blockIdx.x < g_mid + g_wide)
 		fold_wide_blocks(blockIdx.x - g_mid, g_wide, segs, bbeg, S, cnt, aux, bucket, list, cap, s_keys, s_slots, s_beg,
-		                 s_end, s_magic);
+		                 s_end);
 	else
 		fold_big_blocks(blockIdx.x - g_mid - g_wide, gridDim.x - g_mid - g_wide, segs, bbeg, S, cnt, aux, bucket, list,
-		                cap, s_keys, s_slots, s_beg[0], s_end[0], s_magic);
+		                cap, s_keys, s_slots, s_beg[0], s_end[0]);
 }
 
 // ---- scan plumbing for the bin offsets ---------------------------------------------------------
@@ -1167,22 +1272,35 @@ void levels_for(uint32_t L, uint64_t *off) {
 	}
 }
 
-// Blocks for the per-fragment passes (kU fragments per thread and trip).
-uint32_t grid_tiles(uint64_t F, svo_ctx *ctx, uint32_t per_cu = 64u) { return grid_for(div_up(F, kU), ctx, per_cu); }
-
 uint64_t big_capacity(uint64_t F) { return F / (kRegBucket + 1u) + 1u; }
+
+// Grouping of the fragment tiles; index: the pass that rewrites the raw scenes' keys as fragment indices.
+hipError_t group_tiles(svo_ctx *ctx, const BuildBatch &bb, bool index) {
+	return launch(ctx, "bm_group", index ? bm_group<true> : bm_group<false>, dim3((uint32_t)bb.tiles), dim3(kThreads), 0,
+	              (const BuildSeg *)bb.segs, bb.tbeg(), bb.S, bb.bm, bb.keys, bb.heads, bb.runs, bb.nrun, bb.raw);
+}
+
+// tiles: whole tiles of F fragments; the tile arrays of `tiles` tiles, one allocation.
+uint64_t tiles_of(uint64_t F) { return (F + kTile - 1u) / kTile; }
+hipError_t alloc_tiles(Pool *pool, BuildBatch &bb) {
+	const uint64_t t = bb.tiles ? bb.tiles : 1u;
+	const hipError_t e = pool->alloc((void **)&bb.runs, t * (kTile * (sizeof(uint2) + sizeof(uint32_t)) +
+	                                                         kHeads * sizeof(uint64_t) + sizeof(uint32_t)));
+	bb.heads = reinterpret_cast<uint64_t *>(bb.runs + t * kTile);
+	bb.keys = reinterpret_cast<uint32_t *>(bb.heads + t * kHeads);
+	bb.nrun = bb.keys + t * kTile;
+	return e;
+}
 
 int structure_phase(svo_ctx *ctx, BuildBatch &bb) {
 	const uint32_t S = bb.S;
 	hipError_t e;
+	if ((e = launch(ctx, "bm_zero", bm_zero, dim3(grid_for(bb.TW, ctx)), dim3(kThreads), 0, bb.bm, bb.TW, bb.raw, S)) !=
+	    hipSuccess)
+		return hip_check(ctx, e, "bm_zero");
+	if (bb.tiles > 0 && (e = group_tiles(ctx, bb, false)) != hipSuccess)
+		return hip_check(ctx, e, "bm_group");
 	if (bb.TW > 0) {
-		if ((e = launch(ctx, "bm_zero", bm_zero, dim3(grid_for(bb.TW, ctx)), dim3(kThreads), 0, bb.bm, bb.TW)) !=
-		    hipSuccess)
-			return hip_check(ctx, e, "bm_zero");
-		if (bb.Ftot > 0 &&
-		    (e = launch(ctx, "bm_mark", bm_mark, dim3(grid_tiles(bb.Ftot, ctx)), dim3(kThreads), 0,
-		                (const BuildSeg *)bb.segs, bb.fbeg(), S, bb.bm)) != hipSuccess)
-			return hip_check(ctx, e, "bm_mark");
 		for (uint32_t d = bb.maxL >= 3 ? bb.maxL - 2 : 0; d > kTopDepth; --d) {
 			const uint64_t n = bb.h_index[(3 + kMaxLevel + d) * (uint64_t)(S + 1) + S];
 			if (n > 0 && (e = launch(ctx, "bm_reduce", bm_reduce, dim3(grid_for(n, ctx)), dim3(kThreads), 0,
@@ -1204,12 +1322,13 @@ int structure_phase(svo_ctx *ctx, BuildBatch &bb) {
 			return hip_check(ctx, e, "rank_down");
 	}
 	if ((e = launch(ctx, "bm_levels", bm_levels, dim3(div_up(S, 64)), dim3(64), 0, bb.segs, S,
-	                (const uint32_t *)bb.rk, (uint64_t)(1ull << 30))) != hipSuccess)
+	                (const uint32_t *)bb.rk, (const uint32_t *)bb.raw, (uint64_t)(1ull << 30))) != hipSuccess)
 		return hip_check(ctx, e, "bm_levels");
 	return SVO_OK;
 }
 
-int node_phase(svo_ctx *ctx, BuildBatch &bb) {
+// maybe_raw: a scene may be raw (a plan's replay cannot know).
+int node_phase(svo_ctx *ctx, BuildBatch &bb, bool maybe_raw) {
 	const uint32_t S = bb.S;
 	const BuildSeg *segs = bb.segs;
 	hipError_t e;
@@ -1222,13 +1341,13 @@ int node_phase(svo_ctx *ctx, BuildBatch &bb) {
 		                (const uint32_t *)bb.rk, bb.cnt, bb.bbeg() + S, bb.list)) != hipSuccess)
 			return hip_check(ctx, e, "bm_write_blocks");
 	}
-	const uint32_t gF = grid_tiles(bb.Ftot, ctx);
-	uint2 *node = reinterpret_cast<uint2 *>(bb.node);
-	if (bb.Ftot > 0 &&
-	    (e = launch(ctx, "build_tag_leaf", bb.maxL >= 12u ? build_tag_leaf<256> : build_tag_leaf<128>, dim3(gF),
-	                dim3(kThreads), 0, segs, bb.fbeg(), S, (const uint32_t *)bb.bm, (const uint32_t *)bb.rk,
-	                node, bb.cnt)) != hipSuccess)
-		return hip_check(ctx, e, "build_tag_leaf");
+	if (maybe_raw && bb.tiles > 0 && (e = group_tiles(ctx, bb, true)) != hipSuccess)
+		return hip_check(ctx, e, "bm_group");
+	const uint32_t gT = div_up(bb.tiles, kThreads / 64u);
+	if (bb.tiles > 0 && (e = launch(ctx, "tag_runs", tag_runs, dim3(gT), dim3(kThreads), 0, segs, bb.tbeg(), S,
+	                                (const uint32_t *)bb.bm, (const uint32_t *)bb.rk, bb.runs,
+	                                (const uint32_t *)bb.nrun, bb.cnt)) != hipSuccess)
+		return hip_check(ctx, e, "tag_runs");
 	BinCounts bc{bb.cnt, bb.bbeg() + S};
 	if ((e = launch(ctx, "bin_reduce", scan_reduce<BinCounts>, dim3(kScanBlocks), dim3(kScanThreads), 0, bc,
 	                ctx->d_scan_parts)) != hipSuccess)
@@ -1236,20 +1355,19 @@ int node_phase(svo_ctx *ctx, BuildBatch &bb) {
 	if ((e = launch(ctx, "bin_offsets", scan_down<BinCounts, BinOffsets>, dim3(kScanBlocks), dim3(kScanThreads), 0, bc,
 	                BinOffsets{bb.aux}, (const uint64_t *)ctx->d_scan_parts, NoCommit{})) != hipSuccess)
 		return hip_check(ctx, e, "bin_offsets");
-	uint2 *bucket = reinterpret_cast<uint2 *>(bb.bucket);
-	if (bb.Ftot > 0 && (e = launch(ctx, "build_scatter", build_scatter, dim3(grid_tiles(bb.Ftot, ctx, 256u)),
-	                               dim3(kThreads), 0, segs, bb.fbeg(), S, (const uint2 *)node,
-	                               (const uint32_t *)bb.aux, bucket)) != hipSuccess)
-		return hip_check(ctx, e, "build_scatter");
+	if (bb.tiles > 0 && (e = launch(ctx, "scatter_runs", scatter_runs, dim3(gT), dim3(kThreads), 0, segs, bb.tbeg(), S,
+	                                (const uint32_t *)bb.keys, (const uint64_t *)bb.heads, (const uint2 *)bb.runs,
+	                                (const uint32_t *)bb.nrun, (const uint32_t *)bb.aux, bb.bucket)) != hipSuccess)
+		return hip_check(ctx, e, "scatter_runs");
 	const uint64_t cap = big_capacity(bb.Ftot);
 	if ((e = launch(ctx, "build_fold", build_fold, dim3(grid_for(bb.nbins, ctx)), dim3(kThreads), 0, segs, bb.bbeg(),
-	                S, (const uint32_t *)bb.cnt, (const uint32_t *)bb.aux, (const uint2 *)bucket, bb.list, cap)) !=
+	                S, (const uint32_t *)bb.cnt, (const uint32_t *)bb.aux, (const uint32_t *)bb.bucket, bb.list, cap)) !=
 	    hipSuccess)
 		return hip_check(ctx, e, "build_fold");
 	const uint32_t g_mid = (uint32_t)ctx->cu_count * 8u, g_wide = (uint32_t)ctx->cu_count * 8u,
 	               g_big = (uint32_t)ctx->cu_count * 2u;
 	if ((e = launch(ctx, "build_fold_lists", build_fold_lists, dim3(g_mid + g_wide + g_big), dim3(kThreads), 0, segs,
-	                bb.bbeg(), S, (const uint32_t *)bb.cnt, (const uint32_t *)bb.aux, bucket, (const uint32_t *)bb.list,
+	                bb.bbeg(), S, (const uint32_t *)bb.cnt, (const uint32_t *)bb.aux, bb.bucket, (const uint32_t *)bb.list,
 	                cap, g_mid, g_wide)) != hipSuccess)
 		return hip_check(ctx, e, "build_fold_lists");
 	return SVO_OK;
@@ -1265,23 +1383,25 @@ uint64_t build_bitmap_words(uint32_t L) {
 
 void build_batch_release(svo_ctx *ctx, BuildBatch *bb) {
 	for (void *p : {(void *)bb->segs, (void *)bb->bm, (void *)bb->rk, (void *)bb->cnt, (void *)bb->aux,
-	                (void *)bb->node, (void *)bb->bucket, (void *)bb->list}) // index lives in segs' allocation
+	                (void *)bb->runs, (void *)bb->bucket, (void *)bb->list}) // index lives in segs' allocation
 		ctx->pool->free(p);
 	bb->segs = nullptr;
 	bb->index = nullptr;
-	bb->bm = bb->rk = bb->cnt = bb->aux = bb->node = bb->bucket = bb->list = nullptr;
+	bb->bm = bb->rk = bb->raw = bb->cnt = bb->aux = bb->keys = bb->nrun = bb->bucket = bb->list = nullptr;
+	bb->runs = nullptr;
+	bb->heads = nullptr;
 }
 
 namespace {
 
 // Host layout of a build batch of S scenes with F[s] fragments at level L[s]: descriptors (bitmap
-// offsets), fragment begins, per-depth bitmap word tables and the block writer's parent words.
+// offsets), tile begins, per-depth bitmap word tables and the block writer's parent words.
 void batch_layout(BuildBatch &bb, uint32_t S, const uint2 *const *frags, const uint64_t *F, const uint32_t *L) {
 	bb.S = S;
 	bb.h_segs.assign(S, BuildSeg{});
 	const uint64_t stride = S + 1;
 	bb.h_index.assign(bb.pw_at() + bb.pw_segs() + 1, 0);
-	uint64_t *fbeg = bb.h_index.data();
+	uint64_t *tbeg = bb.h_index.data();
 	for (uint32_t s = 0; s < S; ++s) {
 		BuildSeg &g = bb.h_segs[s];
 		g.frags = frags[s];
@@ -1290,11 +1410,12 @@ void batch_layout(BuildBatch &bb, uint32_t S, const uint2 *const *frags, const u
 		g.bm = bb.TW;
 		levels_for(g.L, g.off);
 		bb.TW += g.off[g.L];
-		fbeg[s] = bb.Ftot;
+		tbeg[s] = bb.tiles;
+		bb.tiles += tiles_of(g.F);
 		bb.Ftot += g.F;
 		bb.maxL = std::max(bb.maxL, g.L);
 	}
-	fbeg[S] = bb.Ftot;
+	tbeg[S] = bb.tiles;
 	// per-depth begin tables: dw[d] over scenes with B[d] (L > d), dr[d] over scenes with B[d+1] (L > d+1)
 	for (uint32_t d = 1; d <= kMaxLevel; ++d) {
 		uint64_t *dw = bb.h_index.data() + (2 + d) * stride, *dr = bb.h_index.data() + (3 + kMaxLevel + d) * stride;
@@ -1365,13 +1486,13 @@ int build_batch(svo_ctx *ctx, svo_octree *const *octs, uint32_t S) {
 	const size_t seg_bytes = seg_table_bytes(S), idx_bytes = sizeof(uint64_t) * bb.h_index.size();
 	if (pool->alloc((void **)&bb.segs, seg_bytes + idx_bytes) != hipSuccess ||
 	    pool->alloc((void **)&bb.bm, sizeof(uint32_t) * (bb.TW ? bb.TW : 1)) != hipSuccess ||
-	    pool->alloc((void **)&bb.rk, sizeof(uint32_t) * (bb.TW / 8u + 1)) != hipSuccess ||
-	    pool->alloc((void **)&bb.node, sizeof(uint32_t) * 2 * Fa) != hipSuccess ||
-	    pool->alloc((void **)&bb.bucket, sizeof(uint32_t) * 2 * Fa) != hipSuccess ||
+	    pool->alloc((void **)&bb.rk, sizeof(uint32_t) * (bb.TW / 8u + 1 + S)) != hipSuccess ||
+	    alloc_tiles(pool, bb) != hipSuccess || pool->alloc((void **)&bb.bucket, sizeof(uint32_t) * Fa) != hipSuccess ||
 	    pool->alloc((void **)&bb.list, sizeof(uint32_t) * (3 + 3 * cap)) != hipSuccess)
 		rc = set_error(ctx, SVO_ERR_OUT_OF_MEMORY, "octree build allocation failed");
 	if (!rc) {
 		bb.index = reinterpret_cast<uint64_t *>(reinterpret_cast<uint8_t *>(bb.segs) + seg_bytes);
+		bb.raw = bb.rk + bb.TW / 8u + 1;
 		rc = upload_batch_tables(ctx, bb);
 	}
 	// structure phase: bitmaps + ranks decide every W exactly; one read-back sizes the octrees
@@ -1413,7 +1534,10 @@ int build_batch(svo_ctx *ctx, svo_octree *const *octs, uint32_t S) {
 		rc = upload_batch_tables(ctx, bb);
 	if (!rc) {
 		ctx->t_build2.start(ctx->stream);
-		rc = node_phase(ctx, bb);
+		bool raw = false;
+		for (const BuildSeg &g : bb.h_segs)
+			raw |= g.raw != 0u;
+		rc = node_phase(ctx, bb, raw);
 		ctx->t_build2.stop(ctx->stream);
 	}
 	build_batch_release(ctx, &bb);
@@ -1425,33 +1549,54 @@ namespace {
 
 constexpr uint32_t kPlanThreads = kMaxBatch; // the check kernels take one scene per thread
 
+// Exclusive prefix of one value per thread over the block; total = the sum.  Every thread calls it.
+__device__ __forceinline__ uint64_t plan_excl(uint64_t v, uint64_t &total) {
+	__shared__ uint64_t s_wave[kPlanThreads / 64];
+	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+	uint64_t incl = v;
+#pragma unroll
+	for (uint32_t d = 1; d < 64u; d <<= 1) {
+		const uint64_t t = __shfl_up(incl, d, 64);
+		incl += lane >= d ? t : 0u;
+	}
+	if (lane == 63u)
+		s_wave[wave] = incl;
+	__syncthreads();
+	uint64_t below = 0;
+	total = 0;
+	for (uint32_t w = 0; w < kPlanThreads / 64; ++w) {
+		below += w < wave ? s_wave[w] : 0u;
+		total += s_wave[w];
+	}
+	return below + incl - v;
+}
+
 // Between the voxelize count and fill passes: the scenes' fragment counts become the build's
-// fragment begins.  A count above its list's capacity sets status bit 1 and empties the batch:
-// fill limit, every fragment begin and the fragment total 0, so no later pass reads or writes a
-// list past its end.  Also restores the block writer's parent-word total, which the node check
-// of the previous run may have cleared.  out = {status, F[S], W[S]}.
+// tile begins.  A count above its list's capacity sets status bit 1 and empties the batch: fill limit
+// and every tile begin 0, so no later pass reads or writes a list past its end.  Also restores the
+// block writer's parent-word total, which the node check of the previous run may have cleared.
+// out = {status, F[S], W[S]}.
 __global__ void __launch_bounds__(kPlanThreads)
-    plan_check_frags(const VoxSeg *__restrict__ vsegs, BuildSeg *bsegs, uint64_t *fbeg, uint32_t S,
+    plan_check_frags(const VoxSeg *__restrict__ vsegs, BuildSeg *bsegs, uint64_t *tbeg, uint32_t S,
                      const uint64_t *__restrict__ fcap, uint64_t *fend, uint64_t *pw_total, uint64_t pw_value,
                      uint64_t *out) {
 	const uint32_t s = threadIdx.x;
-	uint64_t F = 0, b = 0;
+	uint64_t F = 0, tiles;
 	int over = 0;
 	if (s < S) {
 		F = vsegs[s].F;
-		b = vsegs[s].frag_begin;
 		over = F > fcap[s];
 		out[1u + s] = F;
 		out[1u + S + s] = 0u;
 		bsegs[s].F = F;
 	}
 	over = __syncthreads_or(over);
+	const uint64_t first = plan_excl((F + kTile - 1u) / kTile, tiles);
 	if (s < S)
-		fbeg[s] = over ? 0u : b;
+		tbeg[s] = over ? 0u : first;
 	if (s == 0u) {
-		const uint64_t total = over ? 0u : fend[0];
-		fend[1] = total;
-		fbeg[S] = total;
+		fend[1] = over ? 0u : fend[0];
+		tbeg[S] = over ? 0u : tiles;
 		*pw_total = pw_value;
 		out[0] = over ? 1u : 0u;
 	}
@@ -1460,12 +1605,11 @@ __global__ void __launch_bounds__(kPlanThreads)
 // Between the structure and node phases: leaf-block begins (an exclusive scan of the scenes' leaf
 // blocks) and W against each octree's capacity.  A W above its capacity (or above 2^30 words), or
 // a fragment overflow found before, sets status bit 2 and empties the node phase: leaf blocks,
-// fragments and parent words 0, so it writes nothing but the root blocks.
+// tiles and parent words 0, so it writes nothing but the root blocks.
 __global__ void __launch_bounds__(kPlanThreads)
-    plan_check_nodes(BuildSeg *segs, uint64_t *bbeg, uint32_t S, const uint64_t *__restrict__ wcap, uint64_t *fbeg,
+    plan_check_nodes(BuildSeg *segs, uint64_t *bbeg, uint32_t S, const uint64_t *__restrict__ wcap, uint64_t *tbeg,
                      uint64_t *pw_total, uint64_t *out) {
-	__shared__ uint64_t s_wave[kPlanThreads / 64];
-	const uint32_t s = threadIdx.x, lane = s & 63u, wave = s >> 6;
+	const uint32_t s = threadIdx.x;
 	uint64_t nb = 0;
 	int over = 0;
 	if (s < S) {
@@ -1475,21 +1619,8 @@ __global__ void __launch_bounds__(kPlanThreads)
 		out[1u + S + s] = g.W;
 	}
 	over = __syncthreads_or(over) || out[0] != 0u;
-	uint64_t incl = nb;
-#pragma unroll
-	for (uint32_t d = 1; d < 64u; d <<= 1) {
-		const uint64_t t = __shfl_up(incl, d, 64);
-		incl += lane >= d ? t : 0u;
-	}
-	if (lane == 63u)
-		s_wave[wave] = incl;
-	__syncthreads();
-	uint64_t below = 0, total = 0;
-	for (uint32_t w = 0; w < kPlanThreads / 64; ++w) {
-		below += w < wave ? s_wave[w] : 0u;
-		total += s_wave[w];
-	}
-	const uint64_t excl = below + incl - nb;
+	uint64_t total;
+	const uint64_t excl = plan_excl(nb, total);
 	if (s < S) {
 		segs[s].bin_begin = over ? 0u : excl;
 		bbeg[s] = over ? 0u : excl;
@@ -1497,7 +1628,7 @@ __global__ void __launch_bounds__(kPlanThreads)
 	if (s == 0u) {
 		bbeg[S] = over ? 0u : total;
 		if (over) {
-			fbeg[S] = 0u;
+			tbeg[S] = 0u;
 			*pw_total = 0u;
 			out[0] |= 2u;
 		}
@@ -1523,7 +1654,7 @@ int plan_enqueue(svo_ctx *ctx, BuildPlan &p) {
 	if ((e = launch(ctx, "plan_check_nodes", plan_check_nodes, dim3(1), dim3(kPlanThreads), 0, bb.segs,
 	                bb.index + (S + 1), S, (const uint64_t *)p.caps + S, bb.index, pw_total, p.out)) != hipSuccess)
 		return hip_check(ctx, e, "plan_check_nodes");
-	return node_phase(ctx, bb);
+	return node_phase(ctx, bb, true);
 }
 
 } // namespace
@@ -1578,9 +1709,9 @@ int build_plan_init(svo_ctx *ctx, BuildPlan *p, const svo_scene *const *scenes, 
 	const size_t seg_bytes = seg_table_bytes(S), idx_bytes = sizeof(uint64_t) * bb.h_index.size();
 	if (pool->alloc((void **)&bb.segs, seg_bytes + idx_bytes) != hipSuccess ||
 	    pool->alloc((void **)&bb.bm, sizeof(uint32_t) * (bb.TW ? bb.TW : 1)) != hipSuccess ||
-	    pool->alloc((void **)&bb.rk, sizeof(uint32_t) * (bb.TW / 8u + 1)) != hipSuccess ||
-	    pool->alloc((void **)&bb.node, sizeof(uint32_t) * 2 * Fcap) != hipSuccess ||
-	    pool->alloc((void **)&bb.bucket, sizeof(uint32_t) * 2 * Fcap) != hipSuccess ||
+	    pool->alloc((void **)&bb.rk, sizeof(uint32_t) * (bb.TW / 8u + 1 + S)) != hipSuccess ||
+	    alloc_tiles(pool, bb) != hipSuccess ||
+	    pool->alloc((void **)&bb.bucket, sizeof(uint32_t) * Fcap) != hipSuccess ||
 	    pool->alloc((void **)&bb.list, sizeof(uint32_t) * (3 + 3 * big_capacity(Fcap))) != hipSuccess ||
 	    pool->alloc((void **)&bb.cnt, sizeof(uint32_t) * Bcap) != hipSuccess ||
 	    pool->alloc((void **)&bb.aux, sizeof(uint32_t) * Bcap) != hipSuccess ||
@@ -1588,6 +1719,7 @@ int build_plan_init(svo_ctx *ctx, BuildPlan *p, const svo_scene *const *scenes, 
 	    pool->alloc((void **)&p->out, sizeof(uint64_t) * (1 + 2 * (size_t)S)) != hipSuccess)
 		return set_error(ctx, SVO_ERR_OUT_OF_MEMORY, "plan build allocation failed");
 	bb.index = reinterpret_cast<uint64_t *>(reinterpret_cast<uint8_t *>(bb.segs) + seg_bytes);
+	bb.raw = bb.rk + bb.TW / 8u + 1;
 	if (int rc = upload_batch_tables(ctx, bb))
 		return rc;
 	if (int rc = upload_table(ctx, p->caps, caps.data(), sizeof(uint64_t) * 2 * S))
