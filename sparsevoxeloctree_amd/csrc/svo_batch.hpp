@@ -126,7 +126,7 @@ struct VoxBatch {
 	uint64_t *tbeg = nullptr;   // S + 1 triangle begins
 	uint64_t *fend = nullptr;   // the fill's {fragment total, limit}, after tbeg
 	uint64_t *offsets = nullptr; // Ttot exclusive fragment offsets (global)
-	uint32_t *big = nullptr;    // big-triangle list: count, then global triangle indices
+	uint32_t *general = nullptr; // triangles in the general form: count, then global indices
 };
 
 // Build batch state, from the structure phase to the node phase.
@@ -177,7 +177,7 @@ int build_batch(svo_ctx *ctx, svo_octree *const *octs, uint32_t S);
 // (fend[0] = total) and the fill (limited by fend[1]) with no read-back between them.
 int voxelize_plan_init(svo_ctx *ctx, VoxBatch *vb, svo_fraglist *const *fls, uint32_t S);
 hipError_t voxelize_plan_count(svo_ctx *ctx, VoxBatch *vb);
-hipError_t voxelize_plan_fill(svo_ctx *ctx, VoxBatch *vb);
+hipError_t voxelize_plan_fill(svo_ctx *ctx, VoxBatch *vb, uint64_t Fcap);
 
 // A voxelize + build of a fixed set of scenes whose fragment lists and octrees are allocated at
 // capacities, so no pass waits for the host: the counts stay on the device, the grids and scratch

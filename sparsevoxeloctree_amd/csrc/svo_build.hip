@@ -1647,7 +1647,7 @@ int plan_enqueue(svo_ctx *ctx, BuildPlan &p) {
 	                (const VoxSeg *)p.vb.segs, bb.segs, bb.index, S, (const uint64_t *)p.caps, p.vb.fend, pw_total,
 	                p.pw_value, p.out)) != hipSuccess)
 		return hip_check(ctx, e, "plan_check_frags");
-	if ((e = voxelize_plan_fill(ctx, &p.vb)) != hipSuccess)
+	if ((e = voxelize_plan_fill(ctx, &p.vb, p.bb.Ftot)) != hipSuccess)
 		return hip_check(ctx, e, "plan voxelize fill");
 	if (int rc = structure_phase(ctx, bb))
 		return rc;

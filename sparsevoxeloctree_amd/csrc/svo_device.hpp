@@ -16,13 +16,12 @@ __device__ __forceinline__ float gmax(float x, float y) { return x < y ? y : x; 
 __device__ __forceinline__ uint32_t umin32(uint32_t a, uint32_t b) { return b < a ? b : a; }
 __device__ __forceinline__ uint32_t umax32(uint32_t a, uint32_t b) { return a < b ? b : a; }
 
-// uint(float): truncation, negative and NaN -> 0, saturating above.
+// uint(float): truncation, negative and NaN -> 0, saturating above.  The instruction does just that; a
+// C++ cast leaves all but the first undefined, and testing for them costs ten instructions.
 __device__ __forceinline__ uint32_t f2u_sat(float f) {
-	if (!(f > 0.0f))
-		return 0u;
-	if (f >= 4294967296.0f)
-		return 0xFFFFFFFFu;
-	return (uint32_t)f;
+	uint32_t u;
+	asm("v_cvt_u32_f32_e32 %0, %1" : "=v"(u) : "v"(f));
+	return u;
 }
 
 __device__ __forceinline__ uint32_t fbits(float f) { return __float_as_uint(f); }

@@ -5,9 +5,10 @@
 //     projection, pixel AABB and voxel depth range, exactly as the geometry shader computes them;
 //   coverage (conservative rasterization, src/Voxelizer.cpp:112-127): pixel (i,j) is covered when
 //     the closed triangle, with vertices snapped to 1/256 pixel, meets the half-open pixel square
-//     [i,i+1) x [j,j+1).  Written as three linear constraints lo_k <= Sx_k*i + Sy_k*j <= hi_k
-//     (one per edge normal, exact int64), so every row's covered pixels form one span found with
-//     two divisions per edge instead of testing pixels one by one;
+//     [i,i+1) x [j,j+1).  A closed triangle and a half-open square are disjoint exactly when the
+//     square's or the triangle's own sides separate them, so the covered pixels of the AABB are
+//     those inside three half-planes A_k i + B_k j >= C_k with integer coefficients, one per edge
+//     (RowPlanes); every row's covered pixels form one span, found with exact double arithmetic;
 //   per pixel (shader/voxelizer.frag:17-44): depth of the triangle's plane at the pixel centre,
 //     clamps to [0,res-1] and to the depth range, swizzle back, fragment packing.
 // Two passes like the reference's count-only + fill draws: vox_count writes the per-triangle count,
@@ -31,19 +32,31 @@ namespace {
 
 constexpr int kThreads = 256;
 
-struct Edge {
-	int64_t sx, sy; // 256 * edge normal
-	int64_t lo, hi; // covered iff lo <= sx*i + sy*j <= hi
-};
+// |pixel coordinates| below this are RowPlanes' (2^30 in 1/256 pixels).
+constexpr float kMaxPixel = 4194304.0f;
 
-struct Setup {
-	bool empty;
+// A triangle as the geometry shader sees it.
+struct TriBase {
+	bool degenerate;
 	uint32_t axis;
 	uint32_t dr0, dr1;
-	int32_t ilo, ihi, jlo, jhi; // pixel rectangle: AABB ∩ snapped bbox ∩ [0, res)
-	float px0, py0, pz0;
+	uint32_t a0, a1, a2, a3; // AABB
+	float px[3], py[3], pz0;
 	float dzdx, dzdy; // plane of the projected triangle (pixel units, depth in [0,1])
-	Edge e[3];
+};
+
+// What a fragment needs of its triangle: the plane, the depth range with res - 1 folded in, the shifts
+// of i, j and depth in the packed word (0 for the volume's x, 12 for y, 24 for z; one byte each).
+struct FragTri {
+	float px0, py0, pz0, dzdx, dzdy, fres;
+	uint32_t zmin, zmax, shifts, colour;
+};
+
+// Any triangle, in 64-bit integers: the general form of RowPlanes, for coordinates from kMaxPixel on.
+struct Setup {
+	bool empty;
+	int32_t ilo, ihi, jlo, jhi; // pixel rectangle: AABB ∩ snapped bbox ∩ [0, res)
+	int64_t X[3], Y[3];         // snapped vertices
 };
 
 __device__ __forceinline__ f3 project(f3 v, uint32_t axis) { // voxelizer.geom:15-19
@@ -55,90 +68,115 @@ __device__ __forceinline__ f3 project(f3 v, uint32_t axis) { // voxelizer.geom:1
 __device__ __forceinline__ int64_t imin64(int64_t a, int64_t b) { return a < b ? a : b; }
 __device__ __forceinline__ int64_t imax64(int64_t a, int64_t b) { return a < b ? b : a; }
 
-__device__ void tri_setup(const float *__restrict__ tri, uint64_t t, uint32_t res, Setup &s) {
+__device__ __forceinline__ void tri_base(const float *__restrict__ tri, uint64_t t, uint32_t res, TriBase &s) {
 	const float *p = tri + 9 * t;
 	f3 p0{p[0], p[1], p[2]}, p1{p[3], p[4], p[5]}, p2{p[6], p[7], p[8]};
 	f3 e1{p1.x - p0.x, p1.y - p0.y, p1.z - p0.z}, e2{p2.x - p0.x, p2.y - p0.y, p2.z - p0.z};
 	f3 n = cross3(e1, e2); // voxelizer.geom:29
 	float wx = fabsf(n.x), wy = fabsf(n.y), wz = fabsf(n.z);
 	s.axis = (wx > wy && wx > wz) ? 0u : (wy > wz ? 1u : 2u);
-	bool degenerate = (n.x == 0.0f && n.y == 0.0f && n.z == 0.0f);
+	s.degenerate = (n.x == 0.0f && n.y == 0.0f && n.z == 0.0f);
 	f3 q0 = project(p0, s.axis), q1 = project(p1, s.axis), q2 = project(p2, s.axis);
 	const float fres = (float)res;
 	// voxelizer.geom:40-43
 	float mnx = gmin(q0.x, gmin(q1.x, q2.x)), mny = gmin(q0.y, gmin(q1.y, q2.y));
 	float mxx = gmax(q0.x, gmax(q1.x, q2.x)), mxy = gmax(q0.y, gmax(q1.y, q2.y));
-	uint32_t a0 = f2u_sat((mnx + 1.0f) * 0.5f * fres), a1 = f2u_sat((mny + 1.0f) * 0.5f * fres);
-	uint32_t a2 = f2u_sat((mxx + 1.0f) * 0.5f * fres), a3 = f2u_sat((mxy + 1.0f) * 0.5f * fres);
+	s.a0 = f2u_sat((mnx + 1.0f) * 0.5f * fres);
+	s.a1 = f2u_sat((mny + 1.0f) * 0.5f * fres);
+	s.a2 = f2u_sat((mxx + 1.0f) * 0.5f * fres);
+	s.a3 = f2u_sat((mxy + 1.0f) * 0.5f * fres);
 	s.dr0 = f2u_sat(gmin(q0.z, gmin(q1.z, q2.z)) * fres);
 	s.dr1 = f2u_sat(gmax(q0.z, gmax(q1.z, q2.z)) * fres);
-
-	float px[3] = {(q0.x + 1.0f) * 0.5f * fres, (q1.x + 1.0f) * 0.5f * fres, (q2.x + 1.0f) * 0.5f * fres};
-	float py[3] = {(q0.y + 1.0f) * 0.5f * fres, (q1.y + 1.0f) * 0.5f * fres, (q2.y + 1.0f) * 0.5f * fres};
-	float pz[3] = {q0.z, q1.z, q2.z};
-	int64_t X[3], Y[3];
-#pragma unroll
-	for (int k = 0; k < 3; ++k) {
-		X[k] = (int64_t)__builtin_rintf(px[k] * 256.0f);
-		Y[k] = (int64_t)__builtin_rintf(py[k] * 256.0f);
-	}
-	s.px0 = px[0];
-	s.py0 = py[0];
-	s.pz0 = pz[0];
-	{
-		float ax = px[1] - px[0], ay = py[1] - py[0], az = pz[1] - pz[0];
-		float bx = px[2] - px[0], by = py[2] - py[0], bz = pz[2] - pz[0];
-		float nx = ay * bz - az * by, ny = az * bx - ax * bz, nz = ax * by - ay * bx;
-		s.dzdx = 0.0f;
-		s.dzdy = 0.0f;
-		if (nz != 0.0f) {
-			s.dzdx = -nx / nz;
-			s.dzdy = -ny / nz;
-		}
-	}
-	int64_t xmn = imin64(X[0], imin64(X[1], X[2])), xmx = imax64(X[0], imax64(X[1], X[2]));
-	int64_t ymn = imin64(Y[0], imin64(Y[1], Y[2])), ymx = imax64(Y[0], imax64(Y[1], Y[2]));
-	int64_t ilo = imax64((int64_t)a0, xmn >> 8), ihi = imin64(imin64((int64_t)a2, (int64_t)res - 1), xmx >> 8);
-	int64_t jlo = imax64((int64_t)a1, ymn >> 8), jhi = imin64(imin64((int64_t)a3, (int64_t)res - 1), ymx >> 8);
-	s.ilo = (int32_t)imax64(ilo, 0);
-	s.ihi = (int32_t)imax64(ihi, -1);
-	s.jlo = (int32_t)imax64(jlo, 0);
-	s.jhi = (int32_t)imax64(jhi, -1);
-	s.empty = degenerate || s.ilo > s.ihi || s.jlo > s.jhi;
-#pragma unroll
-	for (int k = 0; k < 3; ++k) {
-		const int a = k, b = (k + 1) % 3, c = (k + 2) % 3;
-		int64_t A = Y[b] - Y[a], B = X[a] - X[b];
-		int64_t ce = A * X[a] + B * Y[a], cc = A * X[c] + B * Y[c];
-		int64_t tlo = imin64(ce, cc), thi = imax64(ce, cc);
-		bool lo_att = A >= 0 && B >= 0, hi_att = A <= 0 && B <= 0;
-		int64_t thi2 = lo_att ? thi : thi - 1, tlo2 = hi_att ? tlo : tlo + 1;
-		int64_t sx = A * 256, sy = B * 256;
-		int64_t off_lo = (A < 0 ? sx : 0) + (B < 0 ? sy : 0);
-		int64_t width = (sx < 0 ? -sx : sx) + (sy < 0 ? -sy : sy);
-		s.e[k] = Edge{sx, sy, tlo2 - off_lo - width, thi2 - off_lo};
+	s.px[0] = (q0.x + 1.0f) * 0.5f * fres;
+	s.px[1] = (q1.x + 1.0f) * 0.5f * fres;
+	s.px[2] = (q2.x + 1.0f) * 0.5f * fres;
+	s.py[0] = (q0.y + 1.0f) * 0.5f * fres;
+	s.py[1] = (q1.y + 1.0f) * 0.5f * fres;
+	s.py[2] = (q2.y + 1.0f) * 0.5f * fres;
+	s.pz0 = q0.z;
+	float ax = s.px[1] - s.px[0], ay = s.py[1] - s.py[0], az = q1.z - q0.z;
+	float bx = s.px[2] - s.px[0], by = s.py[2] - s.py[0], bz = q2.z - q0.z;
+	float nx = ay * bz - az * by, ny = az * bx - ax * bz, nz = ax * by - ay * bx;
+	s.dzdx = 0.0f;
+	s.dzdy = 0.0f;
+	if (nz != 0.0f) {
+		s.dzdx = -nx / nz;
+		s.dzdy = -ny / nz;
 	}
 }
 
-// Covered pixels of row j: [i0, i1] (empty when i0 > i1).  Exact: the double quotient of two
-// integers below 2^53 never crosses an integer for |quotient| < 2^25 (|sx| <= 2^29), and bounds
-// further out are clamped away by the pixel rectangle.
-__device__ __forceinline__ void row_span(const Setup &s, int32_t j, int32_t &i0, int32_t &i1) {
-	double lo = (double)s.ilo, hi = (double)s.ihi;
+// NaN is not below kMaxPixel
+__device__ __forceinline__ bool pixels_ok(const TriBase &t) {
+	bool ok = true;
+#pragma unroll
+	for (int k = 0; k < 3; ++k)
+		ok = ok && fabsf(t.px[k]) < kMaxPixel && fabsf(t.py[k]) < kMaxPixel;
+	return ok;
+}
+
+// Depth clamps (voxelizer.frag:21-22): min(max(min(z, res - 1), dr0), dr1) with dr0 <= dr1 is z clamped
+// to [dr0, max(dr0, min(res - 1, dr1))].
+__device__ __forceinline__ FragTri frag_tri(const TriBase &b, uint32_t res, uint32_t rgb) {
+	return FragTri{b.px[0], b.py[0], b.pz0, b.dzdx, b.dzdy, (float)res,
+	               b.dr0, umax32(b.dr0, umin32(res - 1u, b.dr1)),
+	               b.axis == 0u ? 0x00180cu : b.axis == 1u ? 0x0c0018u : 0x180c00u, rgb & 0x00ffffffu};
+}
+
+__device__ void tri_setup(const TriBase &b, uint32_t res, Setup &s) {
+	int64_t *X = s.X, *Y = s.Y;
 #pragma unroll
 	for (int k = 0; k < 3; ++k) {
-		const Edge &e = s.e[k];
-		int64_t syj = e.sy * (int64_t)j;
-		int64_t nlo = e.lo - syj, nhi = e.hi - syj;
-		if (e.sx > 0) {
-			lo = fmax(lo, ceil((double)nlo / (double)e.sx));
-			hi = fmin(hi, floor((double)nhi / (double)e.sx));
-		} else if (e.sx < 0) {
-			lo = fmax(lo, ceil((double)nhi / (double)e.sx));
-			hi = fmin(hi, floor((double)nlo / (double)e.sx));
+		X[k] = (int64_t)__builtin_rintf(b.px[k] * 256.0f);
+		Y[k] = (int64_t)__builtin_rintf(b.py[k] * 256.0f);
+	}
+	int64_t xmn = imin64(X[0], imin64(X[1], X[2])), xmx = imax64(X[0], imax64(X[1], X[2]));
+	int64_t ymn = imin64(Y[0], imin64(Y[1], Y[2])), ymx = imax64(Y[0], imax64(Y[1], Y[2]));
+	int64_t ilo = imax64((int64_t)b.a0, xmn >> 8), ihi = imin64(imin64((int64_t)b.a2, (int64_t)res - 1), xmx >> 8);
+	int64_t jlo = imax64((int64_t)b.a1, ymn >> 8), jhi = imin64(imin64((int64_t)b.a3, (int64_t)res - 1), ymx >> 8);
+	s.empty = b.degenerate || imax64(ilo, 0) > imax64(ihi, -1) || imax64(jlo, 0) > imax64(jhi, -1);
+	s.ilo = (int32_t)imin64(imax64(ilo, 0), res);
+	s.ihi = (int32_t)imax64(ihi, -1);
+	s.jlo = (int32_t)imin64(imax64(jlo, 0), res);
+	s.jhi = (int32_t)imax64(jhi, -1);
+}
+
+// Exact floor(a / b) for b > 0: the double quotient is within one of it wherever it matters (a
+// quotient inside the pixel grid), and the integer remainder corrects it.
+__device__ __forceinline__ int64_t floor_div(int64_t a, int64_t b) {
+	int64_t q = (int64_t)floor((double)a / (double)b);
+	const int64_t r = a - q * b;
+	q -= r < 0 ? 1 : 0;
+	q += r >= b ? 1 : 0;
+	return q;
+}
+
+// Covered pixels of row j: [i0, i1] (empty when i0 > i1).  Edge k admits lo <= sx i + sy j <= hi with
+// (sx, sy) = 256 times its normal; one edge at a time, as few registers as possible.
+__device__ __forceinline__ void row_span(const Setup &s, int32_t j, int32_t &i0, int32_t &i1) {
+	int64_t lo = s.ilo, hi = s.ihi;
+	int64_t ax = s.X[0], ay = s.Y[0], bx = s.X[1], by = s.Y[1], cx = s.X[2], cy = s.Y[2];
+#pragma unroll 1
+	for (int k = 0; k < 3; ++k) {
+		const int64_t A = by - ay, B = ax - bx;
+		const int64_t ce = A * ax + B * ay, cc = A * cx + B * cy;
+		const int64_t tlo = imin64(ce, cc), thi = imax64(ce, cc);
+		const bool lo_att = A >= 0 && B >= 0, hi_att = A <= 0 && B <= 0;
+		const int64_t sx = A * 256, sy = B * 256;
+		const int64_t off_lo = (A < 0 ? sx : 0) + (B < 0 ? sy : 0);
+		const int64_t width = (sx < 0 ? -sx : sx) + (sy < 0 ? -sy : sy);
+		const int64_t syj = sy * (int64_t)j;
+		const int64_t nlo = (hi_att ? tlo : tlo + 1) - off_lo - width - syj;
+		const int64_t nhi = (lo_att ? thi : thi - 1) - off_lo - syj;
+		if (sx != 0) {
+			lo = imax64(lo, -floor_div(sx > 0 ? -nlo : nhi, sx > 0 ? sx : -sx));
+			hi = imin64(hi, floor_div(sx > 0 ? nhi : -nlo, sx > 0 ? sx : -sx));
 		} else if (nlo > 0 || nhi < 0) {
-			hi = -1.0;
+			hi = -1;
 		}
+		const int64_t tx = ax, ty = ay;
+		ax = bx, ay = by;
+		bx = cx, by = cy;
+		cx = tx, cy = ty;
 	}
 	if (lo > hi) {
 		i0 = 1;
@@ -149,158 +187,244 @@ __device__ __forceinline__ void row_span(const Setup &s, int32_t j, int32_t &i0,
 	}
 }
 
-// Exact floor(a / b) for b > 0 and |a| < 2^53: the double quotient is within one of it, and the
-// integer remainder corrects it.
-__device__ __forceinline__ int64_t floor_div(int64_t a, int64_t b) {
-	int64_t q = (int64_t)floor((double)a / (double)b);
-	const int64_t r = a - q * b;
-	q -= r < 0 ? 1 : 0;
-	q += r >= b ? 1 : 0;
-	return q;
+__device__ __forceinline__ int32_t lane_of(int32_t v, uint32_t l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ uint64_t lane_of(uint64_t u, uint32_t l) {
+	const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((uint32_t)u, l);
+	const uint32_t h = (uint32_t)__builtin_amdgcn_readlane((uint32_t)(u >> 32), l);
+	return a | ((uint64_t)h << 32);
+}
+__device__ __forceinline__ double lane_of(double v, uint32_t l) {
+	return __longlong_as_double((long long)lane_of((uint64_t)__double_as_longlong(v), l));
 }
 
-// floor(X_j / p) for X_j = X_0 + j * s, kept as X_j = q p + r (0 <= r < p) and advanced one step at
-// a time with integer adds only.  p = 256 |A| and |s| = 256 |B| for snapped edge vectors (A, B)
-// below 2^21, so p < 2^29, r fits 32 bits and the per-step quotient |floor(s / p)| < 2^21.
-struct FloorTrack {
-	int64_t q;
-	int32_t dq;
-	uint32_t r, dr;
-	__device__ void init(int64_t X, int64_t step, uint32_t p) {
-		q = floor_div(X, p);
-		r = (uint32_t)(X - q * (int64_t)p);
-		const int64_t d = floor_div(step, p);
-		dq = (int32_t)d;
-		dr = (uint32_t)(step - d * (int64_t)p);
-	}
-	__device__ __forceinline__ void next(uint32_t p) {
-		q += dq;
-		r += dr;
-		if (r >= p) {
-			r -= p;
-			++q;
+// 1 / a within 2^-51 of its value: two Newton steps from the instruction's 23 bits or more.
+__device__ __forceinline__ double reciprocal(double a) {
+	double x = __builtin_amdgcn_rcp(a);
+	x = fma(fma(-a, x, 1.0), x, x);
+	return fma(fma(-a, x, 1.0), x, x);
+}
+
+// The covered spans of a triangle's rows, from three half-planes A i + B j >= C.  The vertices are
+// put in the order in which the triangle lies on the positive side of every edge; then an edge from
+// (x, y) covers the pixels whose square reaches it:
+//     256 (A i + B j) >= A x + B y + (corner attained ? 0 : 1) - 256 (max(A, 0) + max(B, 0)).
+// The A of the three edges sum to 0, so rows are mirrored (i -> -i) where needed to have one upper
+// bound of i (A < 0) and two lower ones (A >= 0), and the vertices rotated to have it last.  With
+// M = B j - C the bounds are i <= floor(M / |A|) and i >= -floor(M / |A|), and
+//     floor(M / |A|) = round((M + 1/2 - |A| / 2) / |A|),
+// two fused multiply-adds and no conversion when the second adds 1.5 * 2^52, which leaves the rounded
+// integer in the low word.  C is exact in 64 bits (|x|, |y| < 2^30).  Where the bound lies within the
+// pixel grid, |M| < 2^45 is exact in double; what is rounded stays 1/(2 |A|) away from a tie, more than
+// the 2^-51 |M / |A|| by which the reciprocal can err, so the result is exact.  Further out it only has
+// to stay there: a line moves |B / A| pixels a row, so where the width times the height of the triangle
+// is below 2^29 bounds fit the word (`near`); else they are clamped.  A = 0 bounds the rows only, by
+// nothing that the snapped bounding box does not.  A triangle that is a segment or a point after
+// snapping gets its line's both sides.
+// Doubles rather than 32- or 64-bit integers: v_fma_f64 runs at the rate of an integer add here.
+struct RowPlanes {
+	double iv[3], b[3], d[3];
+	int32_t ilo, ihi; // mirrored if mir
+	int32_t jlo, jhi;
+	bool mir, near;
+
+	// false (and no rows) if a coordinate is kMaxPixel or more, or not a number
+	__device__ __forceinline__ bool init(const TriBase &t, uint32_t res) {
+		jlo = 0;
+		jhi = -1;
+		near = true;
+		if (!pixels_ok(t))
+			return t.degenerate;
+		int32_t x[3], y[3];
+#pragma unroll
+		for (int k = 0; k < 3; ++k) {
+			x[k] = (int32_t)__builtin_rintf(t.px[k] * 256.0f);
+			y[k] = (int32_t)__builtin_rintf(t.py[k] * 256.0f);
 		}
+		const int32_t xmn = min(x[0], min(x[1], x[2])), xmx = max(x[0], max(x[1], x[2]));
+		const int32_t ymn = min(y[0], min(y[1], y[2])), ymx = max(y[0], max(y[1], y[2]));
+		const int32_t i0 = max((int32_t)t.a0, xmn >> 8), i1 = min(min((int32_t)t.a2, (int32_t)res - 1), xmx >> 8);
+		const int32_t j0 = max((int32_t)t.a1, ymn >> 8), j1 = min(min((int32_t)t.a3, (int32_t)res - 1), ymx >> 8);
+		if (t.degenerate || i0 > i1)
+			return true;
+		jlo = j0;
+		jhi = j1;
+		const int64_t area = (int64_t)(y[1] - y[0]) * (x[2] - x[0]) - (int64_t)(x[1] - x[0]) * (y[2] - y[0]);
+		if (area == 0) {
+			// on a line: its ends P and Q, as the edges P Q, Q Q (which bounds nothing) and Q P
+			const bool flat = ymn == ymx;
+			int32_t p = 0, q = 0;
+#pragma unroll
+			for (int k = 1; k < 3; ++k) {
+				const int32_t vk = flat ? x[k] : y[k];
+				p = vk < (flat ? pick(x, p) : pick(y, p)) ? k : p;
+				q = vk > (flat ? pick(x, q) : pick(y, q)) ? k : q;
+			}
+			const int32_t xp = pick(x, p), yp = pick(y, p), xq = pick(x, q), yq = pick(y, q);
+			x[0] = xp, y[0] = yp;
+			x[1] = x[2] = xq, y[1] = y[2] = yq;
+			mir = false;
+		} else {
+			if (area < 0) {
+				const int32_t tx = x[1], ty = y[1];
+				x[1] = x[2], y[1] = y[2];
+				x[2] = tx, y[2] = ty;
+			}
+			const int32_t a0 = y[1] - y[0], a1 = y[2] - y[1], a2 = y[0] - y[2];
+			mir = (a0 > 0) + (a1 > 0) + (a2 > 0) == 1;
+			const bool u0 = mir ? a0 > 0 : a0 < 0, u1 = mir ? a1 > 0 : a1 < 0;
+			const int32_t x0 = x[0], x1 = x[1], x2 = x[2], y0 = y[0], y1 = y[1], y2 = y[2];
+			x[0] = u0 ? x1 : u1 ? x2 : x0, y[0] = u0 ? y1 : u1 ? y2 : y0;
+			x[1] = u0 ? x2 : u1 ? x0 : x1, y[1] = u0 ? y2 : u1 ? y0 : y1;
+			x[2] = u0 ? x0 : u1 ? x1 : x2, y[2] = u0 ? y0 : u1 ? y1 : y2;
+		}
+		ilo = mir ? -i1 : i0;
+		ihi = mir ? -i0 : i1;
+		near = (float)(xmx - xmn) * (float)((ymx - ymn) >> 8) < 536870912.0f;
+#pragma unroll
+		for (int k = 0; k < 3; ++k) {
+			const int32_t A = y[(k + 1) % 3] - y[k], B = x[k] - x[(k + 1) % 3];
+			const int64_t r = (int64_t)A * x[k] + (int64_t)B * y[k] + (A <= 0 && B <= 0 ? 255 : 256);
+			const double a = (double)(A < 0 ? -A : A);
+			b[k] = A == 0 ? 0.0 : (double)B;
+			d[k] = A == 0 ? 1073741824.0 : 0.5 - 0.5 * a - (double)((r >> 8) - max(A, 0) - max(B, 0));
+			iv[k] = A == 0 ? 1.0 : reciprocal(a);
+			iv[k] = k == 2 ? iv[k] : -iv[k];
+		}
+		return true;
+	}
+	static __device__ __forceinline__ int32_t pick(const int32_t *v, int32_t k) {
+		return k == 0 ? v[0] : k == 1 ? v[1] : v[2];
+	}
+	template <bool kNear> __device__ __forceinline__ int32_t bound(int k, double j) const {
+		const double magic = 6755399441055744.0, m = fma(b[k], j, d[k]);
+		const double q = kNear ? fma(m, iv[k], magic) : fmin(fmax(m * iv[k], -1073741824.0), 1073741824.0) + magic;
+		return (int32_t)(uint32_t)__double_as_longlong(q);
+	}
+	// number of covered pixels of row j, and the first one
+	template <bool kNear> __device__ __forceinline__ int32_t span(int32_t j, int32_t &i0) const {
+		const double dj = (double)j;
+		const int32_t lo = max(max(bound<kNear>(0, dj), bound<kNear>(1, dj)), ilo), hi = min(bound<kNear>(2, dj), ihi);
+		i0 = mir ? -hi : lo;
+		return max(hi - lo + 1, 0);
+	}
+	template <bool kNear> __device__ __forceinline__ uint32_t count(int32_t j) const {
+		int32_t i0;
+		return (uint32_t)span<kNear>(j, i0);
+	}
+	__device__ __forceinline__ RowPlanes of_lane(uint32_t l) const {
+		RowPlanes w;
+#pragma unroll
+		for (int k = 0; k < 3; ++k) {
+			w.iv[k] = lane_of(iv[k], l);
+			w.b[k] = lane_of(b[k], l);
+			w.d[k] = lane_of(d[k], l);
+		}
+		w.ilo = lane_of(ilo, l);
+		w.ihi = lane_of(ihi, l);
+		w.jlo = lane_of(jlo, l);
+		w.jhi = lane_of(jhi, l);
+		w.mir = lane_of((int32_t)mir, l) != 0;
+		return w;
 	}
 };
 
-// The covered spans of consecutive rows, as row_span computes them, with no division per row.  An
-// edge with sx = 0 constrains only which rows are covered, once per triangle (rows() narrows the
-// triangle's row range).  For the others, with p = |sx| and U_j, V_j the constraint's two sides
-// mirrored to a positive divisor (both change by the same step per row), row j's span is
-// [max(ilo, ceil(U_j / p)), min(ihi, floor(V_j / p))], and ceil(U / p) = -floor(-U / p).
-struct RowSpans {
-	FloorTrack lo[3], hi[3];
-	uint32_t p[3]; // |sx| per edge
-	bool on[3];
-	int32_t ilo, ihi;
-	// rows [j0, j1] that every sx = 0 edge admits, within the triangle's [jlo, jhi]; then the
-	// trackers start at row j0
-	__device__ void init(const Setup &s, int32_t &j0, int32_t &j1) {
-		ilo = s.ilo;
-		ihi = s.ihi;
-		int64_t jl = s.jlo, jh = s.jhi;
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
 #pragma unroll
-		for (int k = 0; k < 3; ++k) {
-			const Edge &e = s.e[k];
-			on[k] = e.sx != 0;
-			if (e.sx != 0)
-				continue;
-			// covered iff lo <= sy j <= hi
-			if (e.sy == 0) {
-				if (e.lo > 0 || e.hi < 0)
-					jh = jl - 1;
-			} else if (e.sy > 0) {
-				jl = imax64(jl, -floor_div(-e.lo, e.sy));
-				jh = imin64(jh, floor_div(e.hi, e.sy));
-			} else {
-				jl = imax64(jl, -floor_div(e.hi, -e.sy));
-				jh = imin64(jh, floor_div(-e.lo, -e.sy));
-			}
-		}
-		j0 = (int32_t)jl;
-		j1 = (int32_t)imax64(jh, jl - 1);
-#pragma unroll
-		for (int k = 0; k < 3; ++k) {
-			const Edge &e = s.e[k];
-			if (!on[k])
-				continue;
-			const int64_t nlo = e.lo - e.sy * (int64_t)j0, nhi = e.hi - e.sy * (int64_t)j0;
-			const uint32_t pk = (uint32_t)(e.sx > 0 ? e.sx : -e.sx);
-			p[k] = pk;
-			const int64_t step = e.sx > 0 ? -e.sy : e.sy;   // per row, of U and V
-			const int64_t U = e.sx > 0 ? nlo : -nhi, V = e.sx > 0 ? nhi : -nlo;
-			lo[k].init(-U, -step, pk); // floor(-U_j / p)
-			hi[k].init(V, step, pk);   // floor(V_j / p)
-		}
-	}
-	__device__ __forceinline__ void span(int32_t &i0, int32_t &i1) const {
-		int64_t a = ilo, b = ihi;
-#pragma unroll
-		for (int k = 0; k < 3; ++k)
-			if (on[k]) {
-				a = imax64(a, -lo[k].q);
-				b = imin64(b, hi[k].q);
-			}
-		if (a > b) {
-			i0 = 1;
-			i1 = 0;
-		} else {
-			i0 = (int32_t)a;
-			i1 = (int32_t)b;
-		}
-	}
-	__device__ __forceinline__ void next() {
-#pragma unroll
-		for (int k = 0; k < 3; ++k)
-			if (on[k]) {
-				lo[k].next(p[k]);
-				hi[k].next(p[k]);
-			}
-	}
-};
+	for (int d = 32; d; d >>= 1)
+		v += (uint32_t)__shfl_xor((int)v, d, 64);
+	return v;
+}
+// LDS that a wave alone uses: its stores before are seen by its loads after
+__device__ __forceinline__ void wave_sync() {
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+}
 
 __global__ void vox_zero_counter(uint32_t *c) { c[0] = 0u; }
 
-// Count pass.  Triangles with more than kBigTri fragments are also appended to `big` (big[0] is
-// the count) for vox_fill_big; the per-lane fill skips them.
-constexpr uint32_t kBigTri = 128;
+// Count pass: a lane walks its triangle's rows.  A few tall triangles in a wave of flat ones are
+// instead taken by the whole wave, a row per lane; so are those in the general form, after the others
+// (in a loop of its own: it needs the registers).  `general` lists the latter, [0] is their number.
+// Bound by VALU issue (1.0 busy, a third of it the triangles' setup): 990,800 triangles of a room at
+// 2^10 65 -> 22 us, 8.0M with slivers at 2^12 465 -> 108 us, against 64-bit integers with a division
+// per edge side; 870 triangles of 500 rows 56 -> 7 us by the wave-wide walk.
+constexpr int32_t kTallRows = 32;
 
 __global__ void __launch_bounds__(kThreads)
     vox_count(const VoxSeg *__restrict__ segs, const uint64_t *__restrict__ tbeg, uint32_t S, uint64_t T,
-              uint64_t *__restrict__ counts, uint32_t *__restrict__ big) {
-	const uint64_t stride = (uint64_t)gridDim.x * kThreads;
+              uint64_t *__restrict__ counts, uint32_t *__restrict__ general, uint32_t per) {
+	const uint32_t lane = threadIdx.x & 63u;
+	const uint64_t first = ((uint64_t)blockIdx.x * (kThreads / 64) + (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * per;
+	const uint64_t stride = (uint64_t)gridDim.x * (kThreads / 64) * per;
 	uint32_t hint = 0;
-	for (uint64_t base = (uint64_t)blockIdx.x * kThreads; base < T; base += stride) {
-		const uint64_t t = base + threadIdx.x;
-		if (t >= T)
-			continue;
+	bool again = false;
+	for (uint64_t base = first; base < T; base += stride) {
+		const bool in = lane < per && base + lane < T;
+		const uint64_t t = in ? base + lane : base;
 		const float *xyz;
 		uint64_t tl;
 		uint32_t level;
-		with_seg<kThreads>(tbeg, S, hint, base, t, [&](uint32_t sg) {
+		with_seg<64u>(tbeg, S, hint, base, t, [&](uint32_t sg) {
 			xyz = segs[sg].xyz;
 			level = segs[sg].level;
 			tl = t - tbeg[sg];
 		});
-		Setup s;
-		tri_setup(xyz, tl, 1u << level, s);
+		TriBase tri;
+		tri_base(xyz, tl, 1u << level, tri);
+		RowPlanes rp;
+		const bool wild = !rp.init(tri, 1u << level) && in;
+		const int32_t rows = in ? rp.jhi - rp.jlo + 1 : 0;
+		// a tall triangle's share of the wave costs what about six rows of the lanes' walk cost
+		const int32_t tall_rows = per == 64u ? kTallRows : 8;
+		bool tall = rows > tall_rows;
+		const bool far = rows > 0 && !rp.near;
+		int32_t most = 0, n = 0;
+		for (uint64_t m = __ballot(tall); m; m &= m - 1u, ++n)
+			most = max(most, lane_of(rows, (uint32_t)__ffsll((unsigned long long)m) - 1u));
+		tall = far || (tall && n * 6 < most - tall_rows);
 		uint32_t c = 0;
-		if (!s.empty) {
-			RowSpans rs;
-			int32_t j0, j1;
-			rs.init(s, j0, j1);
-			for (int32_t j = j0; j <= j1; ++j) {
-				int32_t i0, i1;
-				rs.span(i0, i1);
-				if (i0 <= i1)
+		if (!tall && in)
+			for (int32_t j = rp.jlo; j <= rp.jhi; ++j)
+				c += rp.count<true>(j);
+		for (uint64_t m = __ballot(tall); m; m &= m - 1u) {
+			const uint32_t l = (uint32_t)__ffsll((unsigned long long)m) - 1u;
+			const RowPlanes w = rp.of_lane(l);
+			uint32_t wc = 0;
+			for (int32_t j = w.jlo + (int32_t)lane; j <= w.jhi; j += 64)
+				wc += w.count<false>(j);
+			wc = wave_sum(wc);
+			c = lane == l ? wc : c;
+		}
+		again |= __ballot(wild) != 0u;
+		if (in && !wild)
+			counts[t] = c;
+	}
+	if (!again)
+		return;
+	for (uint64_t base = first; base < T; base += stride) {
+		for (uint64_t t = base; t < T && t < base + per; ++t) {
+			const uint32_t sg = S == 1u ? 0u : seg_find(tbeg, S, t);
+			const uint32_t res = 1u << segs[sg].level;
+			TriBase tri;
+			tri_base(segs[sg].xyz, t - tbeg[sg], res, tri);
+			if (pixels_ok(tri) || tri.degenerate)
+				continue;
+			Setup s;
+			tri_setup(tri, res, s);
+			uint32_t c = 0;
+			if (!s.empty)
+				for (int32_t j = s.jlo + (int32_t)lane; j <= s.jhi; j += 64) {
+					int32_t i0, i1;
+					row_span(s, j, i0, i1);
 					c += (uint32_t)(i1 - i0 + 1);
-				rs.next();
+				}
+			c = wave_sum(c);
+			if (lane == 0u) {
+				counts[t] = c;
+				if (c)
+					general[1 + atomicAdd(&general[0], 1u)] = (uint32_t)t;
 			}
 		}
-		counts[t] = c;
-		const uint32_t q = wave_append(&big[0], c > kBigTri);
-		if (c > kBigTri)
-			big[1 + q] = (uint32_t)t;
 	}
 }
 
@@ -317,169 +441,240 @@ __global__ void vox_seg_totals(VoxSeg *segs, const uint64_t *__restrict__ tbeg, 
 }
 
 // One fragment: depth at the pixel centre, clamps, swizzle back (voxelizer.frag:17-25) and packing
-// (voxelizer.frag:38-42).  dy = dz/dy * (j + 0.5 - py0) of the row.
-__device__ __forceinline__ uint2 make_frag(const Setup &s, int32_t i, int32_t j, float dy, uint32_t res,
-                                          uint32_t colour) {
-	const float zc = s.pz0 + (s.dzdx * (((float)i + 0.5f) - s.px0) + dy);
-	uint32_t uz = umin32(f2u_sat(zc * (float)res), res - 1u);
-	uz = umin32(umax32(uz, s.dr0), s.dr1);
-	const uint32_t ui = (uint32_t)i, uj = (uint32_t)j;
-	uint32_t vx, vy, vz;
-	if (s.axis == 0u)
-		vx = uz, vy = ui, vz = uj;
-	else if (s.axis == 1u)
-		vx = uj, vy = uz, vz = ui;
-	else
-		vx = ui, vy = uj, vz = uz;
-	return make_uint2(vx | (vy << 12u) | ((vz & 0xffu) << 24u), ((vz >> 8u) << 28u) | colour);
+// (voxelizer.frag:38-42: x | y << 12 | z << 24, (z >> 8) << 28 | rgb).
+__device__ __forceinline__ uint64_t make_frag(const FragTri &s, uint32_t i, uint32_t j) {
+	const float dy = s.dzdy * (((float)(int32_t)j + 0.5f) - s.py0);
+	const float zc = s.pz0 + (s.dzdx * (((float)(int32_t)i + 0.5f) - s.px0) + dy);
+	const uint32_t z = umin32(umax32(f2u_sat(zc * s.fres), s.zmin), s.zmax);
+	const uint32_t sj = s.shifts >> 8, sz = s.shifts >> 16;
+	const uint32_t lo = i << (s.shifts & 31u) | j << (sj & 31u) | z << (sz & 31u);
+	const uint32_t vz = sz == 24u ? z : (s.shifts & 255u) == 24u ? i : j;
+	return (uint64_t)(((vz << 20u) & 0xf0000000u) | s.colour) << 32 | lo;
 }
+// a fragment list as a place in global memory, also where the address comes from LDS
+using FragOut = __attribute__((address_space(1))) uint64_t;
 
-// Fill of the small triangles: each lane walks its triangle's rows and writes its fragments at the
-// triangle's offset (triangle order, row-major inside the triangle).  Offsets are global over the
-// batch; fend = {the batch's fragment total, the fill limit}: a triangle whose fragments end past
-// the limit is not written (the limit is the total, or 0 when a captured plan found a fragment
-// count above its list's capacity).
-__global__ void __launch_bounds__(kThreads)
-    vox_fill(const VoxSeg *__restrict__ segs, const uint64_t *__restrict__ tbeg, uint32_t S, uint64_t T,
-             const uint64_t *__restrict__ offsets, const uint64_t *__restrict__ fend) {
-	const uint64_t Ftot = fend[0], lim = fend[1];
-	const uint64_t stride = (uint64_t)gridDim.x * kThreads;
-	uint32_t hint = 0;
-	for (uint64_t base = (uint64_t)blockIdx.x * kThreads; base < T; base += stride) {
-		const uint64_t t = base + threadIdx.x;
-		if (t >= T)
-			continue;
-		uint64_t k = offsets[t];
-		const uint64_t kend = (t + 1 < T) ? offsets[t + 1] : Ftot;
-		if (k == kend || kend - k > kBigTri || kend > lim)
-			continue;
-		const float *xyz;
-		const uint32_t *rgb;
-		uint2 *frags;
-		uint64_t tl, fb; // fb: offsets are global over the batch
-		uint32_t level;
-		with_seg<kThreads>(tbeg, S, hint, base, t, [&](uint32_t sg) {
-			const VoxSeg &g = segs[sg];
-			xyz = g.xyz;
-			rgb = g.rgb;
-			frags = g.frags;
-			fb = g.frag_begin;
-			level = g.level;
-			tl = t - tbeg[sg];
-		});
-		const uint32_t res = 1u << level;
-		Setup s;
-		tri_setup(xyz, tl, res, s);
-		const uint32_t colour = rgb[tl] & 0x00ffffffu;
-		RowSpans rs;
-		int32_t j0, j1;
-		rs.init(s, j0, j1);
-		for (int32_t j = j0; j <= j1 && k < kend; ++j) {
-			int32_t i0, i1;
-			rs.span(i0, i1);
-			rs.next();
-			const float dy = s.dzdy * (((float)j + 0.5f) - s.py0);
-			for (int32_t i = i0; i <= i1 && k < kend; ++i)
-				frags[(k++) - fb] = make_frag(s, i, j, dy, res, colour);
-		}
+// Fill (triangle order, row-major inside a triangle), split by work: triangle t costs kTriCost plus
+// one per fragment, so it owns the keys from K(t) = offsets[t] + kTriCost t on, and a wave takes the
+// work of `unit` consecutive keys, which may be many triangles or a small part of one.  Triangles are
+// taken in groups of 64, one per lane: a group of at most `unit` keys by the wave that has its first
+// key, a larger one by all that have a part of it, each its fragments.  The group's fragments are laid
+// end to end, kWin of them per window: the lanes walk the rows and leave each row's {triangle, i, j} in
+// LDS at its first fragment's place; then a lane per fragment finds its row by the heads at or below
+// its place and its triangle's parameters in LDS, and writes: even work and whole lines, whatever the
+// triangles' shapes.  Rows are walked a triangle per lane, or, where a window holds few triangles (tall
+// ones, or of many fragments), a row per lane.
+// Bound by VALU issue (0.9 busy; per 64 fragments 46 instructions, and 25 per row of the tallest
+// triangle of a window): 35M fragments of a room at 2^10 245 -> 116 us, 173M with slivers at 2^12
+// 1472 -> 560 us, 32 mixed scenes 990 -> 396 us, against a triangle per lane writing its own fragments
+// and a block per triangle above 128 of them; where few triangles hold most (room of 220,848 at 2^11,
+// 54M fragments) 659 -> 153 us.  Windows of 512 / 1024: 598 / 576 us with slivers, 404 / 415 the batch.
+// Offsets are global over the batch; fend = {the batch's fragment total, the fill limit}: a triangle
+// whose fragments end past the limit is not written (the limit is the total, or 0 when a captured
+// plan found a fragment count above its list's capacity).
+constexpr uint32_t kWin = 768;
+constexpr uint32_t kTriCost = 8;
+// Units: 48 waves per CU (twice what it holds) or more, for an even end, and at least 256 keys for the
+// search and the group's setup; above 4096 the last waves run alone (870 triangles, 20,631 fragments:
+// 256 / 1024 / 4096 12 / 14 / 28 us; slivers: 2048 / 4096 668 / 576 us; room: 4096 / 8192 139 / 159 us).
+constexpr uint32_t kMinUnit = 256, kMaxUnit = 4096;
+
+// Last group of 64 triangles whose keys begin at or below key.
+__device__ __forceinline__ uint64_t key_group(const uint64_t *__restrict__ offsets, uint64_t groups, uint64_t key,
+                                              uint32_t lane) {
+	uint64_t lo = 0, hi = groups;
+	while (hi - lo > 1u) {
+		const uint64_t step = (hi - lo + 63u) / 64u, g = lo + lane * step, t = 64u * (g < hi ? g : lo);
+		const uint64_t m = __ballot(g < hi && offsets[t] + kTriCost * t <= key);
+		lo += ((uint32_t)__popcll(m) - 1u) * step; // lane 0's holds
+		hi = lo + step < hi ? lo + step : hi;
 	}
+	return lo;
 }
 
-// Fill of the big triangles: one block per triangle.  Rows are taken kRowChunk at a time: one
-// thread per row computes the row's span into LDS, a block scan gives each row's first output
-// position, then every thread maps output positions p = tid, tid + 256, ... to (row, column) by a
-// binary search over the row offsets, so stores are coalesced and the work is even whatever the
-// triangle's shape.
-constexpr int kRowChunk = 1024;
-
-__global__ void __launch_bounds__(kThreads)
-    vox_fill_big(const VoxSeg *__restrict__ segs, const uint64_t *__restrict__ tbeg, uint32_t S, uint64_t T,
-                 const uint64_t *__restrict__ offsets, const uint32_t *__restrict__ big,
-                 const uint64_t *__restrict__ fend) {
-	__shared__ int32_t s_i0[kRowChunk];
-	__shared__ uint32_t s_off[kRowChunk + 1];
-	__shared__ uint32_t s_wave[kThreads / 64];
+__global__ void __launch_bounds__(kThreads, 6)
+    vox_fill(const VoxSeg *__restrict__ segs, const uint64_t *__restrict__ tbeg, uint32_t S, uint64_t T,
+             const uint64_t *__restrict__ offsets, const uint32_t *__restrict__ general,
+             const uint64_t *__restrict__ fend, uint32_t unit) {
+	__shared__ uint32_t s_head[kThreads / 64][kWin]; // row heads: 1 << 31 | lane << 24 | j << 12 | i - place (12 bits); 0: none
+	__shared__ uint4 s_tri[kThreads / 64][64][3];
+	const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	uint32_t *head = s_head[wave];
+	uint4(*par)[3] = s_tri[wave];
+	for (uint32_t q = lane; q < kWin; q += 64u)
+		head[q] = 0u;
 	const uint64_t Ftot = fend[0], lim = fend[1];
-	const uint32_t nbig = big[0];
-	for (uint32_t b = blockIdx.x; b < nbig; b += gridDim.x) {
-		const uint64_t t = big[1 + b];
-		if (t >= T)
-			continue;
-		uint64_t k = offsets[t];
-		const uint64_t kend = (t + 1 < T) ? offsets[t + 1] : Ftot;
-		if (kend > lim) // block-uniform: t is the block's triangle
-			continue;
-		const uint32_t sg = S == 1u ? 0u : seg_find(tbeg, S, t);
-		const VoxSeg &g = segs[sg];
-		const uint64_t tl = t - tbeg[sg];
-		const uint32_t res = 1u << g.level;
-		uint2 *frags = g.frags;
-		const uint64_t fb = g.frag_begin; // offsets are global over the batch
-		Setup s;
-		tri_setup(g.xyz, tl, res, s);
-		const uint32_t colour = g.rgb[tl] & 0x00ffffffu;
-		for (int32_t r0 = s.jlo; r0 <= s.jhi && k < kend; r0 += kRowChunk) {
-			const int32_t nrows = (s.jhi - r0 + 1) < kRowChunk ? (s.jhi - r0 + 1) : kRowChunk;
-			// spans and counts, kRowChunk / kThreads rows per thread
-			uint32_t local = 0;
-			int32_t cnt[kRowChunk / kThreads];
-#pragma unroll
-			for (int q = 0; q < kRowChunk / kThreads; ++q) {
-				const int32_t r = (int32_t)threadIdx.x * (kRowChunk / kThreads) + q;
-				int32_t i0 = 1, i1 = 0;
-				if (r < nrows)
-					row_span(s, r0 + r, i0, i1);
-				cnt[q] = i0 <= i1 ? i1 - i0 + 1 : 0;
-				if (r < nrows)
-					s_i0[r] = i0;
-				local += (uint32_t)cnt[q];
-			}
-			// block exclusive scan of the per-thread totals
-			const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-			uint32_t incl = local;
+	if (lim == 0u)
+		return;
+	const uint64_t keys = Ftot + kTriCost * T;
+	const uint64_t waves = (uint64_t)gridDim.x * (kThreads / 64);
+	for (uint64_t key = ((uint64_t)blockIdx.x * (kThreads / 64) + wave) * unit; key < keys; key += waves * unit) {
+		const uint64_t key_end = key + unit;
+		uint64_t t0 = 64u * key_group(offsets, (T + 63u) / 64u, key, lane);
+		uint32_t hint = S == 1u ? 0u : seg_find(tbeg, S, t0);
+		for (bool more = true; more; t0 += 64u) {
+			const bool in = t0 + lane < T;
+			const uint64_t t = in ? t0 + lane : T - 1u;
+			const uint64_t k = offsets[t];
+			const uint64_t kend = (t + 1 < T) ? offsets[t + 1] : Ftot;
+			const uint64_t kb = k + kTriCost * (t + 1u); // key of its first fragment
+			const uint64_t gb = lane_of(kb, 0u) - kTriCost, ge = lane_of(kb + (kend - k), 63u); // the group's keys
+			more = t0 + 64u < T && ge < key_end;
+			const bool whole = ge - gb <= unit;
+			if (whole && gb < key)
+				continue;
+			// its fragments to write: [skip, skip + c)
+			const uint64_t from = whole ? gb : key, to = whole ? ge : key_end;
+			const uint32_t skip = kb < from ? (uint32_t)(from - kb) : 0u;
+			const uint64_t ke = kb + (kend - k) < to ? kb + (kend - k) : to;
+			uint32_t c = in && kend <= lim && ke > kb + skip ? (uint32_t)(ke - kb) - skip : 0u;
+			if (!__any(c != 0u))
+				continue;
+			const float *xyz;
+			const uint32_t *rgb;
+			uint2 *frags;
+			uint64_t tl, fb; // fb: offsets are global over the batch
+			uint32_t level;
+			with_seg<64u>(tbeg, S, hint, t0, t, [&](uint32_t sg) {
+				const VoxSeg &g = segs[sg];
+				xyz = g.xyz;
+				rgb = g.rgb;
+				frags = g.frags;
+				fb = g.frag_begin;
+				level = g.level;
+				tl = t - tbeg[sg];
+			});
+			RowPlanes rp;
+			TriBase tri;
+			tri_base(xyz, tl, 1u << level, tri);
+			if (!rp.init(tri, 1u << level))
+				c = 0u; // in the general list
+			uint32_t incl = c;
 #pragma unroll
 			for (int d = 1; d < 64; d <<= 1) {
-				uint32_t o = __shfl_up(incl, (unsigned)d, 64);
+				const uint32_t o = (uint32_t)__shfl_up((int)incl, (unsigned)d, 64);
 				if ((int)lane >= d)
 					incl += o;
 			}
-			if (lane == 63u)
-				s_wave[wave] = incl;
-			__syncthreads();
-			uint32_t base = 0, total = 0;
-#pragma unroll
-			for (int w = 0; w < kThreads / 64; ++w) {
-				base += (w < (int)wave) ? s_wave[w] : 0u;
-				total += s_wave[w];
+			const uint32_t N = (uint32_t)lane_of((int32_t)incl, 63u);
+			// places of the batch's fragments: [0, N); the next row starts at p, its triangle ends at pend
+			const int32_t pend = (int32_t)incl;
+			int32_t p = (int32_t)(incl - c) - (int32_t)skip;
+			{
+				const FragTri ft = frag_tri(tri, 1u << level, rgb[tl]);
+				const uint64_t out = (uint64_t)(uintptr_t)(frags + (k - fb)) - (int64_t)p * (int64_t)sizeof(uint2);
+				par[lane][0] = make_uint4(fbits(ft.px0), fbits(ft.py0), fbits(ft.pz0), fbits(ft.dzdx));
+				par[lane][1] = make_uint4(fbits(ft.dzdy), fbits(ft.fres), ft.zmin, ft.zmax);
+				par[lane][2] = make_uint4(ft.shifts, ft.colour, (uint32_t)out, (uint32_t)(out >> 32));
 			}
-			uint32_t run = base + incl - local;
-#pragma unroll
-			for (int q = 0; q < kRowChunk / kThreads; ++q) {
-				const int32_t r = (int32_t)threadIdx.x * (kRowChunk / kThreads) + q;
-				s_off[r] = run; // rows past nrows get the chunk total and are never selected
-				run += (uint32_t)cnt[q];
-			}
-			if (threadIdx.x == 0)
-				s_off[kRowChunk] = total;
-			__syncthreads();
-			const uint32_t avail = (uint32_t)((kend - k) < (uint64_t)total ? (kend - k) : total);
-			for (uint32_t p = threadIdx.x; p < avail; p += kThreads) {
-				// last row with s_off[row] <= p
-				int32_t lo = 0, hi = nrows - 1;
-				while (lo < hi) {
-					const int32_t mid = (lo + hi + 1) >> 1;
-					if (s_off[mid] <= p)
-						lo = mid;
-					else
-						hi = mid - 1;
+			int32_t j = rp.jlo;
+			const int32_t rows = rp.jhi - j + 1;
+			const bool tall = !rp.near || rows > kTallRows || (rows > 12 && c + skip >= 128u);
+			const uint32_t mark = 0x80000000u | lane << 24;
+			uint32_t last = 0u; // lane 0: the newest head before the step
+			for (int32_t w0 = 0; w0 < (int32_t)N; w0 += (int32_t)kWin) {
+				const int32_t wend = c ? min(w0 + (int32_t)kWin, pend) : p;
+				// a row of no fragments leaves its head to the next row's; rows before the unit do so at 0
+				if (!tall) {
+					for (; p < wend && j <= rp.jhi; ++j) {
+						int32_t i0;
+						const int32_t n = rp.span<true>(j, i0);
+						head[max(p, w0) - w0] = mark | (uint32_t)j << 12 | ((uint32_t)(i0 - p) & 4095u);
+						p += n;
+					}
+					if (p < wend) { // never: the rows hold the fragments counted
+						head[max(p, w0) - w0] = mark;
+						p = pend;
+					}
 				}
-				const int32_t j = r0 + lo;
-				const int32_t i = s_i0[lo] + (int32_t)(p - s_off[lo]);
-				const float dy = s.dzdy * (((float)j + 0.5f) - s.py0);
-				frags[k + p - fb] = make_frag(s, i, j, dy, res, colour);
+				for (uint64_t m = __ballot(tall && p < wend); m; m &= m - 1u) {
+					const uint32_t l = (uint32_t)__ffsll((unsigned long long)m) - 1u;
+					const RowPlanes w = rp.of_lane(l);
+					const int32_t le = lane_of(pend, l), lw = lane_of(wend, l);
+					int32_t lj = lane_of(j, l), lp = lane_of(p, l);
+					while (lp < lw) {
+						int32_t i0 = 0, n = 0;
+						if (lj + (int32_t)lane <= w.jhi)
+							n = w.span<false>(lj + (int32_t)lane, i0);
+						else if (lj + (int32_t)lane == w.jhi + 1 || (lane == 0u && lj > w.jhi))
+							n = le; // never used, as above
+						int32_t end = n;
+#pragma unroll
+						for (int d = 1; d < 64; d <<= 1) {
+							const int32_t o = __shfl_up(end, (unsigned)d, 64);
+							if ((int)lane >= d)
+								end += o;
+						}
+						end = min(end + lp, le);
+						const int32_t before = __shfl_up(end, 1u, 64), beg = lane ? before : lp;
+						const int32_t at = max(beg, w0);
+						if (beg < lw && end > at)
+							head[at - w0] = 0x80000000u | l << 24 | ((uint32_t)(lj + (int32_t)lane) & 4095u) << 12 |
+							                ((uint32_t)(i0 - beg) & 4095u);
+						// rows that begin in this window or before it are done
+						const uint32_t done = (uint32_t)__popcll(__ballot(beg < lw));
+						lp = lane_of(end, done - 1u);
+						lj += (int32_t)done;
+					}
+					j = lane == l ? lj : j;
+					p = lane == l ? lp : p;
+				}
+				wave_sync();
+				for (uint32_t q = 0; q < kWin && (uint32_t)w0 + q < N; q += 64u) {
+					const uint32_t at = (uint32_t)w0 + q + lane;
+					uint32_t h = head[q + lane];
+					head[q + lane] = 0u;
+					const uint64_t m = __ballot(h != 0u) | 1u;
+					h = h ? h : last;
+					const uint64_t below = m & (~0ull >> (63u - lane));
+					const uint32_t row = (uint32_t)__shfl((int)h, 63 - __clzll((long long)below), 64);
+					const uint32_t top = (uint32_t)lane_of((int32_t)h, 63u - (uint32_t)__clzll((long long)m));
+					last = lane == 0u ? top : 0u;
+					if (at < N) {
+						const uint4 *tp = par[(row >> 24) & 63u];
+						const uint4 f0 = tp[0], f1 = tp[1], f2 = tp[2];
+						const FragTri ft{bitsf(f0.x), bitsf(f0.y), bitsf(f0.z), bitsf(f0.w), bitsf(f1.x),
+						                 bitsf(f1.y), f1.z, f1.w, f2.x, f2.y};
+						FragOut *out = (FragOut *)(uintptr_t)(f2.z | (uint64_t)f2.w << 32);
+						out[at] = make_frag(ft, (row + at) & 4095u, (row >> 12) & 4095u);
+					}
+				}
+				wave_sync();
 			}
-			k += total;
-			__syncthreads();
+		}
+	}
+	// the triangles in the general form, a wave each, 64 rows at a time
+	const uint32_t ngen = general[0];
+	for (uint64_t g = (uint64_t)blockIdx.x * (kThreads / 64) + wave; g < ngen; g += waves) {
+		const uint64_t t = general[1 + g];
+		if (t >= T)
+			continue;
+		uint64_t k = offsets[t];
+		const uint64_t kend = (t + 1 < T) ? offsets[t + 1] : Ftot;
+		if (kend > lim)
+			continue;
+		const uint32_t sg = S == 1u ? 0u : seg_find(tbeg, S, t);
+		const uint64_t tl = t - tbeg[sg];
+		const uint32_t res = 1u << segs[sg].level;
+		TriBase tri;
+		tri_base(segs[sg].xyz, tl, res, tri);
+		Setup s;
+		tri_setup(tri, res, s);
+		if (s.empty)
+			continue;
+		const FragTri ft = frag_tri(tri, res, segs[sg].rgb[tl]);
+		FragOut *frags = (FragOut *)(uintptr_t)(segs[sg].frags - segs[sg].frag_begin);
+		for (int32_t j0 = s.jlo; j0 <= s.jhi && k < kend; j0 += 64) {
+			int32_t i0 = 1, i1 = 0;
+			if (j0 + (int32_t)lane <= s.jhi)
+				row_span(s, j0 + (int32_t)lane, i0, i1);
+			for (int32_t r = 0; r < 64 && k < kend; ++r) {
+				const int32_t a = lane_of(i0, (uint32_t)r), b = lane_of(i1, (uint32_t)r);
+				for (int32_t i = a + (int32_t)lane; i <= b; i += 64)
+					if (k + (uint32_t)(i - a) < kend)
+						frags[k + (uint32_t)(i - a)] = make_frag(ft, (uint32_t)i, (uint32_t)(j0 + r));
+				k += (uint32_t)(b - a + 1);
+			}
 		}
 	}
 }
@@ -576,6 +771,30 @@ uint32_t grid_for(uint64_t items, const svo_ctx *ctx) {
 	return (uint32_t)(g ? g : 1);
 }
 
+// vox_count: 64 triangles per wave, fewer where that would leave SIMDs without a wave (then a wave's
+// other lanes help with its tall triangles).
+hipError_t launch_count(svo_ctx *ctx, const VoxBatch *vb) {
+	const uint64_t T = vb->Ttot, want = (T + ctx->cu_count * 16u - 1) / (ctx->cu_count * 16u);
+	const uint32_t per = want < 64u ? (uint32_t)want : 64u;
+	const uint64_t blocks = (T + per * (kThreads / 64) - 1) / (per * (kThreads / 64)), cap = (uint64_t)ctx->cu_count * 64u;
+	return launch(ctx, "vox_count", vox_count, dim3((uint32_t)(blocks < cap ? blocks : cap)), dim3(kThreads), 0,
+	              (const VoxSeg *)vb->segs, (const uint64_t *)vb->tbeg, vb->S, T, vb->offsets, vb->general, per);
+}
+
+// vox_fill over T triangles with at most Fcap fragments.
+hipError_t launch_fill(svo_ctx *ctx, const VoxBatch *vb, uint64_t Fcap) {
+	const uint64_t keys = Fcap + kTriCost * vb->Ttot;
+	const uint64_t fill = (uint64_t)ctx->cu_count * 48u;
+	uint32_t unit = kMinUnit;
+	while (unit < kMaxUnit && unit * fill < keys)
+		unit *= 2u;
+	const uint64_t blocks = (keys + (uint64_t)unit * (kThreads / 64) - 1) / ((uint64_t)unit * (kThreads / 64));
+	const uint64_t cap = (uint64_t)ctx->cu_count * 64u;
+	return launch(ctx, "vox_fill", vox_fill, dim3((uint32_t)(blocks < cap ? blocks : cap)), dim3(kThreads), 0,
+	              (const VoxSeg *)vb->segs, (const uint64_t *)vb->tbeg, vb->S, vb->Ttot, (const uint64_t *)vb->offsets,
+	              (const uint32_t *)vb->general, (const uint64_t *)vb->fend, unit);
+}
+
 } // namespace
 
 int normalize_scene(svo_ctx *ctx, svo_scene *scene) {
@@ -602,13 +821,13 @@ int normalize_scene(svo_ctx *ctx, svo_scene *scene) {
 }
 
 void vox_batch_release(svo_ctx *ctx, VoxBatch *vb) {
-	for (void *p : {(void *)vb->segs, (void *)vb->offsets}) // tbeg and big live in segs' allocation
+	for (void *p : {(void *)vb->segs, (void *)vb->offsets}) // tbeg and general live in segs' allocation
 		ctx->pool->free(p);
 	vb->segs = nullptr;
 	vb->tbeg = nullptr;
 	vb->fend = nullptr;
 	vb->offsets = nullptr;
-	vb->big = nullptr;
+	vb->general = nullptr;
 }
 
 // Count pass over a batch + scan + one read-back of every scene's F + allocation of the lists
@@ -638,7 +857,7 @@ int voxelize_count_batch(svo_ctx *ctx, svo_fraglist *const *fls, uint32_t S, Vox
 		return set_error(ctx, SVO_ERR_OVERFLOW, "more than 2^32-1 triangles in one voxelize call");
 	Pool *pool = ctx->pool;
 	hipError_t e;
-	// descriptors, triangle begins (+ the fill's {total, limit}) and the big-triangle list share one
+	// descriptors, triangle begins (+ the fill's {total, limit}) and the general list share one
 	// allocation, so one copy uploads the tables and clears the list's count
 	const size_t seg_bytes = (sizeof(VoxSeg) * S + 255) & ~size_t(255);
 	const size_t tbeg_bytes = (sizeof(uint64_t) * (S + 3) + 255) & ~size_t(255);
@@ -647,21 +866,19 @@ int voxelize_count_batch(svo_ctx *ctx, svo_fraglist *const *fls, uint32_t S, Vox
 		return set_error(ctx, SVO_ERR_OUT_OF_MEMORY, "count-pass allocation failed");
 	vb->tbeg = reinterpret_cast<uint64_t *>(reinterpret_cast<uint8_t *>(vb->segs) + seg_bytes);
 	vb->fend = vb->tbeg + S + 1;
-	vb->big = reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(vb->segs) + seg_bytes + tbeg_bytes);
+	vb->general = reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(vb->segs) + seg_bytes + tbeg_bytes);
 	{
 		std::vector<uint8_t> tables(seg_bytes + tbeg_bytes + sizeof(uint32_t), 0);
 		std::memcpy(tables.data(), vb->h_segs.data(), sizeof(VoxSeg) * S);
 		std::memcpy(tables.data() + seg_bytes, vb->h_tbeg.data(), sizeof(uint64_t) * (S + 1));
 		if (int rc = upload_table(ctx, vb->segs, tables.data(), tables.size()))
-			return rc; // big[0] = 0 came with the tables
+			return rc; // general[0] = 0 came with the tables
 	}
 	int rc = SVO_OK;
 	uint64_t *total = ctx->d_scan_parts + 2 * kScanBlocks;
 	ctx->t_count.start(ctx->stream);
 	if (T > 0) {
-		if ((e = launch(ctx, "vox_count", vox_count, dim3(grid_for(T, ctx)), dim3(kThreads), 0,
-		                (const VoxSeg *)vb->segs, (const uint64_t *)vb->tbeg, S, T, vb->offsets, vb->big)) !=
-		    hipSuccess)
+		if ((e = launch_count(ctx, vb)) != hipSuccess)
 			return hip_check(ctx, e, "vox_count");
 		CountSrc src{vb->offsets, T};
 		if ((e = launch(ctx, "vox_scan_reduce", scan_reduce<CountSrc>, dim3(kScanBlocks), dim3(kScanThreads), 0, src,
@@ -716,14 +933,8 @@ int voxelize_fill_batch(svo_ctx *ctx, VoxBatch *vb) {
 	hipError_t e;
 	ctx->t_fill.start(ctx->stream);
 	if (T > 0 && Ftot > 0) {
-		if ((e = launch(ctx, "vox_fill", vox_fill, dim3(grid_for(T, ctx)), dim3(kThreads), 0, (const VoxSeg *)vb->segs,
-		                (const uint64_t *)vb->tbeg, S, T, (const uint64_t *)vb->offsets, (const uint64_t *)vb->fend)) !=
-		    hipSuccess)
+		if ((e = launch_fill(ctx, vb, Ftot)) != hipSuccess)
 			return hip_check(ctx, e, "vox_fill");
-		if ((e = launch(ctx, "vox_fill_big", vox_fill_big, dim3((uint32_t)ctx->cu_count * 4u), dim3(kThreads), 0,
-		                (const VoxSeg *)vb->segs, (const uint64_t *)vb->tbeg, S, T, (const uint64_t *)vb->offsets,
-		                (const uint32_t *)vb->big, (const uint64_t *)vb->fend)) != hipSuccess)
-			return hip_check(ctx, e, "vox_fill_big");
 	}
 	ctx->t_fill.stop(ctx->stream);
 	return SVO_OK;
@@ -758,22 +969,21 @@ int voxelize_plan_init(svo_ctx *ctx, VoxBatch *vb, svo_fraglist *const *fls, uin
 		return set_error(ctx, SVO_ERR_OUT_OF_MEMORY, "plan voxelize allocation failed");
 	vb->tbeg = reinterpret_cast<uint64_t *>(reinterpret_cast<uint8_t *>(vb->segs) + seg_bytes);
 	vb->fend = vb->tbeg + S + 1;
-	vb->big = reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(vb->segs) + seg_bytes + tbeg_bytes);
+	vb->general = reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(vb->segs) + seg_bytes + tbeg_bytes);
 	std::vector<uint8_t> tables(seg_bytes + tbeg_bytes, 0);
 	std::memcpy(tables.data(), vb->h_segs.data(), sizeof(VoxSeg) * S);
 	std::memcpy(tables.data() + seg_bytes, vb->h_tbeg.data(), sizeof(uint64_t) * (S + 1));
 	return upload_table(ctx, vb->segs, tables.data(), tables.size());
 }
 
-// Count pass of a plan: big-triangle list cleared by a kernel (the pass may be captured, so no
+// Count pass of a plan: general list cleared by a kernel (the pass may be captured, so no
 // memset), counts, scan into offsets and fend[0] = total, per-scene F and frag_begin.
 hipError_t voxelize_plan_count(svo_ctx *ctx, VoxBatch *vb) {
 	const uint64_t T = vb->Ttot;
 	const uint32_t S = vb->S;
 	hipError_t e;
-	if ((e = launch(ctx, "vox_zero", vox_zero_counter, dim3(1), dim3(1), 0, vb->big)) != hipSuccess ||
-	    (e = launch(ctx, "vox_count", vox_count, dim3(grid_for(T, ctx)), dim3(kThreads), 0, (const VoxSeg *)vb->segs,
-	                (const uint64_t *)vb->tbeg, S, T, vb->offsets, vb->big)) != hipSuccess)
+	if ((e = launch(ctx, "vox_zero", vox_zero_counter, dim3(1), dim3(1), 0, vb->general)) != hipSuccess ||
+	    (e = launch_count(ctx, vb)) != hipSuccess)
 		return e;
 	CountSrc src{vb->offsets, T};
 	if ((e = launch(ctx, "vox_scan_reduce", scan_reduce<CountSrc>, dim3(kScanBlocks), dim3(kScanThreads), 0, src,
@@ -787,17 +997,6 @@ hipError_t voxelize_plan_count(svo_ctx *ctx, VoxBatch *vb) {
 }
 
 // Fill pass of a plan: writes nothing when fend[1] (set between the passes) is 0.
-hipError_t voxelize_plan_fill(svo_ctx *ctx, VoxBatch *vb) {
-	const uint64_t T = vb->Ttot;
-	const uint32_t S = vb->S;
-	hipError_t e;
-	if ((e = launch(ctx, "vox_fill", vox_fill, dim3(grid_for(T, ctx)), dim3(kThreads), 0, (const VoxSeg *)vb->segs,
-	                (const uint64_t *)vb->tbeg, S, T, (const uint64_t *)vb->offsets, (const uint64_t *)vb->fend)) !=
-	    hipSuccess)
-		return e;
-	return launch(ctx, "vox_fill_big", vox_fill_big, dim3((uint32_t)ctx->cu_count * 4u), dim3(kThreads), 0,
-	              (const VoxSeg *)vb->segs, (const uint64_t *)vb->tbeg, S, T, (const uint64_t *)vb->offsets,
-	              (const uint32_t *)vb->big, (const uint64_t *)vb->fend);
-}
+hipError_t voxelize_plan_fill(svo_ctx *ctx, VoxBatch *vb, uint64_t Fcap) { return launch_fill(ctx, vb, Fcap); }
 
 } // namespace svo

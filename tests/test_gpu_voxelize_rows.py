@@ -1,0 +1,99 @@
+"""The voxelizer's row spans (three half-planes per triangle in double), the wave-wide walk of tall
+triangles, and the fill's windows and units of work, against the oracle's separating-axis
+test.  Lists are exact, so no tolerance.
+
+Reference: shader/voxelizer.geom:15-54, shader/voxelizer.frag:17-44, src/Voxelizer.cpp:112-127.
+"""
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def check(ctx, tri, level, name):
+    import sparsevoxeloctree_amd as S
+
+    xyz = np.ascontiguousarray(tri, np.float32).reshape(-1, 9)
+    rgb = np.random.default_rng(xyz.shape[0]).integers(0, 1 << 24, xyz.shape[0]).astype(np.uint32)
+    print(name, "level", level, "T", xyz.shape[0], flush=True)
+    vox = S.Voxelizer.Create(S.Scene.Create(ctx, xyz, rgb, normalize=False), level)
+    vox.CmdVoxelize()
+    ref = oracle.voxelize(xyz, rgb, level)
+    assert vox.GetVoxelFragmentCount() == ref.shape[0]
+    assert np.array_equal(vox.GetVoxelFragmentList(), ref)
+
+
+def grid_triangles(rng, T, level, step, extent):
+    """Vertices on multiples of `step` pixels (1/256: the snapping grid), in a plane tilted a little, so
+    that edges pass exactly through pixel corners and many triangles are segments or points there."""
+    res = 1 << level
+    p = rng.integers(0, int(res / step), (T, 1, 2)) + rng.integers(-extent, extent + 1, (T, 3, 2))
+    p = np.clip(p * step, 0, res) / res * 2.0 - 1.0
+    z = rng.uniform(-1, 1, (T, 1)) + rng.uniform(-0.5, 0.5, (T, 3)) / res
+    axis = rng.integers(0, 3, T)
+    tri = np.concatenate([p, z[:, :, None]], 2)
+    return np.stack([np.roll(tri[k], axis[k], 1) for k in range(T)])
+
+
+@pytest.mark.parametrize("level", [3, 8, 12])
+@pytest.mark.parametrize("step,extent", [(1.0, 1), (1.0, 4), (0.5, 3), (1 / 256, 2), (1 / 256, 300), (1 / 256, 4000)])
+def test_ties_and_snapped_degenerates(ctx, no_device_errors, level, step, extent):
+    rng = np.random.default_rng([level, extent, int(256 * step)])
+    check(ctx, grid_triangles(rng, 1500, level, step, extent), level, "ties %g %d" % (step, extent))
+
+
+@pytest.mark.parametrize("every", [0, 1, 5, 37])
+@pytest.mark.parametrize("level,rows", [(8, 33), (10, 130), (11, 1500)])
+def test_tall_among_flat(ctx, no_device_errors, level, rows, every):
+    # every: a tall triangle in each `every` (0: a single one), so a wave holds 64, 13, 2 or 1 of them, thin and wide ones
+    rng = np.random.default_rng([level, rows, every])
+    res, T = 1 << level, 200
+    tri = rng.uniform(-0.9, 0.9, (T, 1, 3)) + rng.uniform(-3, 3, (T, 3, 3)) / res
+    tall = np.arange(T) % every == 0 if every else np.arange(T) == 101
+    n = int(tall.sum())
+    o = np.concatenate([rng.uniform(-0.9, 0.9, (n, 1)), np.full((n, 1), -0.9), rng.uniform(-0.9, 0.9, (n, 1))], 1)
+    tri[tall] = o[:, None, :]
+    tri[tall, 1, 1] += 2.0 * rows / res
+    tri[tall, 2, 1] += rows / res
+    tri[tall, 2, 0] += rng.choice([0.5, 3.0, 200.0], n) / res
+    check(ctx, np.clip(tri, -1, 1), level, "tall %d/%d" % (rows, every))
+
+
+@pytest.mark.parametrize("far", [3.0, 1000.0, 30000.0, 34000.0, 43000.0])
+def test_far_vertices(ctx, no_device_errors, far):
+    # a vertex or two far outside the volume: coordinates around and above 2^22 pixels at level 8 take
+    # the 64-bit form
+    rng = np.random.default_rng(int(far))
+    tri = rng.uniform(-1, 1, (130, 3, 3))
+    tri[::2, 0] *= far
+    tri[::3, 1, :2] *= far
+    tri[5::13] = tri[5::13] * 1e-2
+    check(ctx, tri, 8, "far %g" % far)
+
+
+@pytest.mark.parametrize("T", [777, 1 << 18])
+def test_fill_units(ctx, no_device_errors, T):
+    # the fill's units of work: triangles of 100 to 1500 fragments (a whole wave of them, and scattered)
+    # among points, small ones and long runs of triangles without a fragment
+    rng = np.random.default_rng(T)
+    tri = np.repeat(rng.uniform(-0.9, 0.9, (T, 1, 3)), 3, 1)
+    k = rng.choice(T, min(700, T // 2), replace=False)
+    k[:64] = T // 3 + np.arange(64)
+    tri[k] = tri[k] + rng.normal(size=(len(k), 3, 3)) * rng.choice([8, 20, 40], (len(k), 1, 1)) / 1024
+    k = rng.choice(T // 2, T // 13, replace=False)
+    tri[k] = tri[k] + rng.normal(size=(len(k), 3, 3)) * 2 / 1024
+    check(ctx, np.clip(tri, -1, 1), 10, "units")
+
+
+@pytest.mark.parametrize("level", [9, 11])
+@pytest.mark.parametrize("points", [0, 1, 5000])
+def test_fill_giants(ctx, no_device_errors, level, points):
+    # triangles that fill many units, as faces of the volume, at a slant and as one long sliver
+    rng = np.random.default_rng([level, points])
+    tri = [[(-1, -1, 1), (1, -1, 1), (1, 1, 1)], [(-1, -1, -1), (-1, 1, -1), (-1, 1, 1)],
+           [(-1, -0.9, -1), (1, 0.8, -0.9), (0.3, 1, 0.2)], [(-1, -1, -0.5), (1, 0.999, 0.5), (1, 1, 0.5)]]
+    tri = np.concatenate([np.repeat(rng.uniform(-1, 1, (points, 1, 3)), 3, 1), np.array(tri, float),
+                          rng.uniform(-0.1, 0.1, (70, 3, 3))])
+    check(ctx, tri, level, "giants")
