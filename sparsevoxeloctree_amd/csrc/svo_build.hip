@@ -102,8 +102,12 @@ __device__ __forceinline__ uint32_t bits_before(const uint32_t *__restrict__ B, 
 	return R[w >> 3] + chunk_before(B + (w & ~7ull), (uint32_t)(w & 7u), word);
 }
 
-// Clears the bitmaps and the scenes' raw flags.
-__global__ void __launch_bounds__(kThreads) bm_zero(uint32_t *B, uint64_t n, uint32_t *raw, uint32_t S) {
+// Clears the bitmaps and the scenes' raw flags, and writes the batch's tables when they fit a kernel
+// argument (words = 0: they are there already).
+__global__ void __launch_bounds__(kThreads) bm_zero(uint32_t *B, uint64_t n, uint32_t *raw, uint32_t S, uint32_t *dst,
+                                                    uint32_t words, SmallTable t) {
+	if (blockIdx.x == 0u && threadIdx.x < words)
+		dst[threadIdx.x] = t.w[threadIdx.x];
 	const uint64_t stride = (uint64_t)gridDim.x * kThreads;
 	for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride)
 		B[i] = 0u;
@@ -372,9 +376,8 @@ __global__ void __launch_bounds__(kThreads)
 constexpr uint32_t kTopDepth = 5;
 constexpr uint32_t kTopWords = 1u << (3u * kTopDepth - 5u);
 
-__global__ void __launch_bounds__(kThreads) bm_reduce_top(const BuildSeg *__restrict__ segs, uint32_t *B, uint32_t *R) {
+template <uint32_t kT> __device__ __forceinline__ void reduce_top(const BuildSeg &g, uint32_t *B, uint32_t *R) {
 	__shared__ uint32_t s_b[2][kTopWords]; // B[d+1] of the previous depth, B[d]
-	const BuildSeg &g = segs[blockIdx.x];
 	const uint32_t L = g.L;
 	if (L <= 1u)
 		return; // no bitmaps
@@ -383,7 +386,7 @@ __global__ void __launch_bounds__(kThreads) bm_reduce_top(const BuildSeg *__rest
 	for (uint32_t d = d0; d >= 1u; --d) {
 		const uint32_t nw = (uint32_t)(g.off[d + 1u] - g.off[d]);      // words of B[d], padded
 		const uint32_t nc = (uint32_t)(g.off[d + 2u] - g.off[d + 1u]); // words of B[d+1], padded
-		for (uint32_t w = threadIdx.x; w < nw; w += kThreads) {
+		for (uint32_t w = threadIdx.x; w < nw; w += kT) {
 			uint32_t bits = 0u;
 			if (8u * w < nc) {
 				uint32_t v[8];
@@ -416,6 +419,9 @@ __global__ void __launch_bounds__(kThreads) bm_reduce_top(const BuildSeg *__rest
 	if (threadIdx.x == 0u)
 		R[g.bm >> 3] = (uint32_t)__popc(d0 >= 1u ? s_b[cur][0] : B[g.bm]);
 }
+__global__ void __launch_bounds__(kThreads) bm_reduce_top(const BuildSeg *__restrict__ segs, uint32_t *B, uint32_t *R) {
+	reduce_top<kThreads>(segs[blockIdx.x], B, R);
+}
 
 // Set bits of 8-word chunk i, as stored by rank_top and bm_reduce.
 struct ChunkCounts {
@@ -436,31 +442,55 @@ struct RankDst {
 	__device__ void operator()(uint64_t i, uint64_t k, uint32_t) const { R[i] = (uint32_t)k; }
 };
 
-// One thread per scene: per-depth node counts -> first block of every depth (fb[0] = 0 is the root
-// block, fb[1] = 1), the leaf blocks and W (src/OctreeBuilder.cpp:212-214: W = (counter + 1) * 8).
-__global__ void bm_levels(BuildSeg *segs, uint32_t S, const uint32_t *__restrict__ R, const uint32_t *__restrict__ raw,
-                          uint64_t cap) {
-	const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-	if (s >= S)
-		return;
-	BuildSeg &g = segs[s];
-	const uint32_t L = g.L;
-	const uint32_t *Rs = R + (g.bm >> 3); // every depth starts a chunk
-	uint64_t first = 1;
-	g.fb[0] = 0u;
-	g.fb[1] = 1u;
-	uint64_t nlast = 1; // nodes at depth L-1 (the root when L == 1)
-	for (uint32_t d = 1; d < L; ++d) {
-		const uint64_t nd = (uint32_t)(Rs[g.off[d + 1u] >> 3] - Rs[g.off[d] >> 3]);
-		first += nd;
-		g.fb[d + 1u] = (uint32_t)(first < 0xFFFFFFFFull ? first : 0xFFFFFFFFull);
-		nlast = nd;
+// Scene s: per-depth node counts -> first block of every depth (fb[0] = 0 is the root block, fb[1] = 1),
+// the leaf blocks and W (src/OctreeBuilder.cpp:212-214: W = (counter + 1) * 8); also into the host's
+// copy of the descriptors (out, pinned memory) when there is one.
+struct Levels {
+	BuildSeg *segs;
+	uint32_t S;
+	const uint32_t *R, *raw;
+	uint64_t cap;
+	BuildSeg *out;
+	__device__ void scene(uint32_t s) const {
+		BuildSeg &o = segs[s];
+		const uint32_t L = o.L;
+		const uint32_t *Rs = R + (o.bm >> 3); // every depth starts a chunk
+		uint64_t first = 1;
+		o.fb[0] = 0u;
+		o.fb[1] = 1u;
+		uint64_t nlast = 1; // nodes at depth L-1 (the root when L == 1)
+		for (uint32_t d = 1; d < L; ++d) {
+			const uint64_t nd = (uint32_t)(Rs[o.off[d + 1u] >> 3] - Rs[o.off[d] >> 3]);
+			first += nd;
+			o.fb[d + 1u] = (uint32_t)(first < 0xFFFFFFFFull ? first : 0xFFFFFFFFull);
+			nlast = nd;
+		}
+		o.W = 8u * first;
+		o.overflow = 8u * first > cap ? 1u : 0u;
+		o.nbins = nlast;
+		o.raw = raw[s];
+		if (out)
+			out[s] = o;
 	}
-	g.W = 8u * first;
-	g.overflow = g.W > cap ? 1u : 0u;
-	g.nbins = nlast;
-	g.raw = raw[s];
+	__device__ void operator()() const {
+		if (threadIdx.x < S)
+			scene(threadIdx.x);
+	}
+};
+static_assert(kMaxBatch <= kOneThreads, "a scene per thread");
+__global__ void bm_levels(Levels levels) {
+	const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+	if (s < levels.S)
+		levels.scene(s);
 }
+struct ReduceTop { // bm_reduce_top of a batch of one scene
+	const BuildSeg *segs;
+	uint32_t *B, *R;
+	__device__ void operator()() const {
+		reduce_top<kOneThreads>(segs[0], B, R);
+		__threadfence_block(); // the scan reads R
+	}
+};
 
 // The 8 words of the block of one depth-(d-1) parent: pointers to the blocks of its occupied
 // children (bits of its byte in B[d]), zeros otherwise; r = rank of its first child among depth d.
@@ -1292,14 +1322,24 @@ hipError_t alloc_tiles(Pool *pool, BuildBatch &bb) {
 	return e;
 }
 
-int structure_phase(svo_ctx *ctx, BuildBatch &bb) {
+// tables: the batch's, to be written first (nullptr: they are in place); out: pinned copy of the
+// descriptors for the host, or nullptr.
+int structure_phase(svo_ctx *ctx, BuildBatch &bb, const std::vector<uint8_t> *tables, BuildSeg *out) {
 	const uint32_t S = bb.S;
 	hipError_t e;
-	if ((e = launch(ctx, "bm_zero", bm_zero, dim3(grid_for(bb.TW, ctx)), dim3(kThreads), 0, bb.bm, bb.TW, bb.raw, S)) !=
-	    hipSuccess)
+	const size_t bytes = tables ? tables->size() : 0;
+	const bool small = bytes > 0 && SmallTable::fits(bytes);
+	if (bytes > 0 && !small)
+		if (int rc = upload_table(ctx, bb.segs, tables->data(), bytes))
+			return rc;
+	static_assert(kThreads >= SmallTable::kWords, "a word per thread");
+	if ((e = launch(ctx, "bm_zero", bm_zero, dim3(grid_for(bb.TW, ctx)), dim3(kThreads), 0, bb.bm, bb.TW, bb.raw, S,
+	                reinterpret_cast<uint32_t *>(bb.segs), small ? (uint32_t)(bytes / 4u) : 0u,
+	                small ? SmallTable(tables->data(), bytes) : SmallTable())) != hipSuccess)
 		return hip_check(ctx, e, "bm_zero");
 	if (bb.tiles > 0 && (e = group_tiles(ctx, bb, false)) != hipSuccess)
 		return hip_check(ctx, e, "bm_group");
+	const Levels levels{bb.segs, S, bb.rk, bb.raw, 1ull << 30, out};
 	if (bb.TW > 0) {
 		for (uint32_t d = bb.maxL >= 3 ? bb.maxL - 2 : 0; d > kTopDepth; --d) {
 			const uint64_t n = bb.h_index[(3 + kMaxLevel + d) * (uint64_t)(S + 1) + S];
@@ -1308,21 +1348,32 @@ int structure_phase(svo_ctx *ctx, BuildBatch &bb) {
 			                         d, bb.bm, bb.rk)) != hipSuccess)
 				return hip_check(ctx, e, "bm_reduce");
 		}
+		// exclusive scan of the chunk counts, in place (each item is read and written by one thread)
+		const ChunkCounts src{bb.rk, bb.TW / 8u};
+		const RankDst dst{bb.rk};
+		const RankTotal total{bb.rk, bb.TW / 8u};
+		const bool one = src.n <= kScanOne;
+		if (one && S == 1u) {
+			e = launch(ctx, "rank", scan_one<ChunkCounts, RankDst, RankTotal, ReduceTop, Levels>, dim3(1),
+			           dim3(kOneThreads), 0, src, dst, total, ReduceTop{bb.segs, bb.bm, bb.rk}, levels);
+			return e == hipSuccess ? SVO_OK : hip_check(ctx, e, "rank");
+		}
 		if ((e = launch(ctx, "bm_reduce_top", bm_reduce_top, dim3(S), dim3(kThreads), 0, (const BuildSeg *)bb.segs,
 		                bb.bm, bb.rk)) != hipSuccess)
 			return hip_check(ctx, e, "bm_reduce_top");
-		// exclusive scan of the chunk counts, in place (each item is read and written by one thread)
-		ChunkCounts src{bb.rk, bb.TW / 8u};
+		if (one) {
+			e = launch(ctx, "rank", scan_one<ChunkCounts, RankDst, RankTotal, NoStep, Levels>, dim3(1),
+			           dim3(kOneThreads), 0, src, dst, total, NoStep{}, levels);
+			return e == hipSuccess ? SVO_OK : hip_check(ctx, e, "rank");
+		}
 		if ((e = launch(ctx, "rank_reduce", scan_reduce<ChunkCounts>, dim3(kScanBlocks), dim3(kScanThreads), 0, src,
 		                ctx->d_scan_parts)) != hipSuccess)
 			return hip_check(ctx, e, "rank_reduce");
 		if ((e = launch(ctx, "rank_down", scan_down<ChunkCounts, RankDst, RankTotal>, dim3(kScanBlocks),
-		                dim3(kScanThreads), 0, src, RankDst{bb.rk}, (const uint64_t *)ctx->d_scan_parts,
-		                RankTotal{bb.rk, bb.TW / 8u})) != hipSuccess)
+		                dim3(kScanThreads), 0, src, dst, (const uint64_t *)ctx->d_scan_parts, total)) != hipSuccess)
 			return hip_check(ctx, e, "rank_down");
 	}
-	if ((e = launch(ctx, "bm_levels", bm_levels, dim3(div_up(S, 64)), dim3(64), 0, bb.segs, S,
-	                (const uint32_t *)bb.rk, (const uint32_t *)bb.raw, (uint64_t)(1ull << 30))) != hipSuccess)
+	if ((e = launch(ctx, "bm_levels", bm_levels, dim3(div_up(S, 64)), dim3(64), 0, levels)) != hipSuccess)
 		return hip_check(ctx, e, "bm_levels");
 	return SVO_OK;
 }
@@ -1349,12 +1400,17 @@ int node_phase(svo_ctx *ctx, BuildBatch &bb, bool maybe_raw) {
 	                                (const uint32_t *)bb.nrun, bb.cnt)) != hipSuccess)
 		return hip_check(ctx, e, "tag_runs");
 	BinCounts bc{bb.cnt, bb.bbeg() + S};
-	if ((e = launch(ctx, "bin_reduce", scan_reduce<BinCounts>, dim3(kScanBlocks), dim3(kScanThreads), 0, bc,
-	                ctx->d_scan_parts)) != hipSuccess)
-		return hip_check(ctx, e, "bin_reduce");
-	if ((e = launch(ctx, "bin_offsets", scan_down<BinCounts, BinOffsets>, dim3(kScanBlocks), dim3(kScanThreads), 0, bc,
-	                BinOffsets{bb.aux}, (const uint64_t *)ctx->d_scan_parts, NoCommit{})) != hipSuccess)
+	const BinOffsets offsets{bb.aux};
+	if (bb.nbins <= kScanOne) {
+		if ((e = launch(ctx, "bin_offsets", scan_one<BinCounts, BinOffsets, NoCommit, NoStep, NoStep>, dim3(1),
+		                dim3(kOneThreads), 0, bc, offsets, NoCommit{}, NoStep{}, NoStep{})) != hipSuccess)
+			return hip_check(ctx, e, "bin_offsets");
+	} else if ((e = launch(ctx, "bin_reduce", scan_reduce<BinCounts>, dim3(kScanBlocks), dim3(kScanThreads), 0, bc,
+	                       ctx->d_scan_parts)) != hipSuccess ||
+	           (e = launch(ctx, "bin_offsets", scan_down<BinCounts, BinOffsets>, dim3(kScanBlocks), dim3(kScanThreads),
+	                       0, bc, offsets, (const uint64_t *)ctx->d_scan_parts, NoCommit{})) != hipSuccess) {
 		return hip_check(ctx, e, "bin_offsets");
+	}
 	if (bb.tiles > 0 && (e = launch(ctx, "scatter_runs", scatter_runs, dim3(gT), dim3(kThreads), 0, segs, bb.tbeg(), S,
 	                                (const uint32_t *)bb.keys, (const uint64_t *)bb.heads, (const uint2 *)bb.runs,
 	                                (const uint32_t *)bb.nrun, (const uint32_t *)bb.aux, bb.bucket)) != hipSuccess)
@@ -1364,8 +1420,13 @@ int node_phase(svo_ctx *ctx, BuildBatch &bb, bool maybe_raw) {
 	                S, (const uint32_t *)bb.cnt, (const uint32_t *)bb.aux, (const uint32_t *)bb.bucket, bb.list, cap)) !=
 	    hipSuccess)
 		return hip_check(ctx, e, "build_fold");
-	const uint32_t g_mid = (uint32_t)ctx->cu_count * 8u, g_wide = (uint32_t)ctx->cu_count * 8u,
-	               g_big = (uint32_t)ctx->cu_count * 2u;
+	// the roles' loops take any number of blocks: no more than the fragments can fill with listed leaf
+	// blocks (17, 65 and 513 fragments at least), a wave or a block each
+	constexpr uint64_t kWaves = kThreads / 64u;
+	const uint32_t cu = (uint32_t)ctx->cu_count;
+	const uint32_t g_mid = (uint32_t)std::min<uint64_t>(cu * 8u, bb.Ftot / (17u * kWaves) + 1u),
+	               g_wide = (uint32_t)std::min<uint64_t>(cu * 8u, bb.Ftot / (65u * kWaves) + 1u),
+	               g_big = (uint32_t)std::min<uint64_t>(cu * 2u, bb.Ftot / 513u + 1u);
 	if ((e = launch(ctx, "build_fold_lists", build_fold_lists, dim3(g_mid + g_wide + g_big), dim3(kThreads), 0, segs,
 	                bb.bbeg(), S, (const uint32_t *)bb.cnt, (const uint32_t *)bb.aux, bb.bucket, (const uint32_t *)bb.list,
 	                cap, g_mid, g_wide)) != hipSuccess)
@@ -1445,11 +1506,16 @@ void batch_layout(BuildBatch &bb, uint32_t S, const uint2 *const *frags, const u
 // Descriptors and begin tables in one device allocation, so each upload is one copy.
 size_t seg_table_bytes(uint32_t S) { return (sizeof(BuildSeg) * S + 255) & ~size_t(255); }
 
-int upload_batch_tables(svo_ctx *ctx, BuildBatch &bb) {
+std::vector<uint8_t> batch_tables(const BuildBatch &bb) {
 	const size_t seg_bytes = seg_table_bytes(bb.S), idx_bytes = sizeof(uint64_t) * bb.h_index.size();
 	std::vector<uint8_t> tables(seg_bytes + idx_bytes);
 	std::memcpy(tables.data(), bb.h_segs.data(), sizeof(BuildSeg) * bb.S);
 	std::memcpy(tables.data() + seg_bytes, bb.h_index.data(), idx_bytes);
+	return tables;
+}
+
+int upload_batch_tables(svo_ctx *ctx, const BuildBatch &bb) {
+	const std::vector<uint8_t> tables = batch_tables(bb);
 	return upload_table(ctx, bb.segs, tables.data(), tables.size());
 }
 
@@ -1490,19 +1556,21 @@ int build_batch(svo_ctx *ctx, svo_octree *const *octs, uint32_t S) {
 	    alloc_tiles(pool, bb) != hipSuccess || pool->alloc((void **)&bb.bucket, sizeof(uint32_t) * Fa) != hipSuccess ||
 	    pool->alloc((void **)&bb.list, sizeof(uint32_t) * (3 + 3 * cap)) != hipSuccess)
 		rc = set_error(ctx, SVO_ERR_OUT_OF_MEMORY, "octree build allocation failed");
+	// structure phase: bitmaps + ranks decide every W exactly; one read-back sizes the octrees
+	BuildSeg *out = nullptr;
+	if (!rc && S <= kReadbackScenes && !(out = static_cast<BuildSeg *>(readback_slot(ctx, sizeof(BuildSeg) * S))))
+		rc = SVO_ERR_INVALID_ARGUMENT;
 	if (!rc) {
 		bb.index = reinterpret_cast<uint64_t *>(reinterpret_cast<uint8_t *>(bb.segs) + seg_bytes);
 		bb.raw = bb.rk + bb.TW / 8u + 1;
-		rc = upload_batch_tables(ctx, bb);
-	}
-	// structure phase: bitmaps + ranks decide every W exactly; one read-back sizes the octrees
-	if (!rc) {
+		const std::vector<uint8_t> tables = batch_tables(bb);
 		ctx->t_build.start(ctx->stream);
-		rc = structure_phase(ctx, bb);
+		rc = structure_phase(ctx, bb, &tables, out);
 		ctx->t_build.stop(ctx->stream);
 	}
 	if (!rc)
-		rc = download_table(ctx, bb.h_segs.data(), bb.segs, sizeof(BuildSeg) * S);
+		rc = out ? readback_wait(ctx, bb.h_segs.data(), out, sizeof(BuildSeg) * S)
+		         : download_table(ctx, bb.h_segs.data(), bb.segs, sizeof(BuildSeg) * S);
 	if (!rc)
 		for (uint32_t s = 0; s < S; ++s)
 			if (bb.h_segs[s].overflow) {
@@ -1649,7 +1717,7 @@ int plan_enqueue(svo_ctx *ctx, BuildPlan &p) {
 		return hip_check(ctx, e, "plan_check_frags");
 	if ((e = voxelize_plan_fill(ctx, &p.vb, p.bb.Ftot)) != hipSuccess)
 		return hip_check(ctx, e, "plan voxelize fill");
-	if (int rc = structure_phase(ctx, bb))
+	if (int rc = structure_phase(ctx, bb, nullptr, nullptr))
 		return rc;
 	if ((e = launch(ctx, "plan_check_nodes", plan_check_nodes, dim3(1), dim3(kPlanThreads), 0, bb.segs,
 	                bb.index + (S + 1), S, (const uint64_t *)p.caps + S, bb.index, pw_total, p.out)) != hipSuccess)

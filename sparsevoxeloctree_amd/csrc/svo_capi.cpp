@@ -236,6 +236,8 @@ hipError_t Staging::release(hipStream_t s) {
 int upload_table(svo_ctx *ctx, void *dst, const void *src, size_t bytes) {
 	if (bytes == 0)
 		return SVO_OK;
+	if (SmallTable::fits(bytes))
+		return hip_check(ctx, table_write(ctx, dst, SmallTable(src, bytes), bytes), "table upload");
 	void *slot = ctx->stage.acquire(bytes);
 	if (!slot)
 		return set_error(ctx, SVO_ERR_INVALID_ARGUMENT, "table larger than the staging slot");
@@ -255,6 +257,21 @@ int download_table(svo_ctx *ctx, void *dst, const void *src, size_t bytes) {
 	hipError_t e = hipMemcpyAsync(slot, src, bytes, hipMemcpyDeviceToHost, ctx->stream);
 	if (e == hipSuccess)
 		e = hipStreamSynchronize(ctx->stream);
+	if (e != hipSuccess)
+		return hip_check(ctx, e, "table read-back");
+	std::memcpy(dst, slot, bytes);
+	return SVO_OK;
+}
+
+void *readback_slot(svo_ctx *ctx, size_t bytes) {
+	void *slot = ctx->stage.acquire(bytes);
+	if (!slot)
+		(void)set_error(ctx, SVO_ERR_INVALID_ARGUMENT, "table larger than the staging slot");
+	return slot;
+}
+
+int readback_wait(svo_ctx *ctx, void *dst, const void *slot, size_t bytes) {
+	const hipError_t e = hipStreamSynchronize(ctx->stream);
 	if (e != hipSuccess)
 		return hip_check(ctx, e, "table read-back");
 	std::memcpy(dst, slot, bytes);

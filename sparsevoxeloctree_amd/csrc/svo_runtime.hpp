@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
@@ -203,10 +204,28 @@ inline hipError_t launch(svo_ctx *ctx, const char *name, Kernel k, dim3 grid, di
 
 inline uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
-// Stream-ordered copy of a small host table into device memory through the staging ring.
+// A table of up to 1 KB as a kernel argument.
+struct SmallTable {
+	static constexpr uint32_t kWords = 256;
+	uint32_t w[kWords];
+	static bool fits(size_t bytes) { return bytes <= sizeof(uint32_t) * kWords && bytes % 4u == 0u; }
+	SmallTable() = default;
+	SmallTable(const void *src, size_t bytes) : w{} { std::memcpy(w, src, bytes); }
+};
+hipError_t table_write(svo_ctx *ctx, void *dst, const SmallTable &t, size_t bytes);
+
+// Stream-ordered copy of a small host table into device memory: as a kernel argument when it fits
+// (a launch, where a copy command is a launch, a staging slot and its event), else through the staging
+// ring.
 int upload_table(svo_ctx *ctx, void *dst, const void *src, size_t bytes);
 // Copy of a small device table to the host; waits for the stream.
 int download_table(svo_ctx *ctx, void *dst, const void *src, size_t bytes);
+// Read-back that the last kernel itself writes: a pinned slot for it to fill (null: error set), then
+// the wait and the copy out of the slot.
+// Small batches only: every scene's thread stores its own descriptor over the bus.
+constexpr uint32_t kReadbackScenes = 64;
+void *readback_slot(svo_ctx *ctx, size_t bytes);
+int readback_wait(svo_ctx *ctx, void *dst, const void *slot, size_t bytes);
 
 // Entry points implemented per stage.
 int normalize_scene(svo_ctx *ctx, svo_scene *scene);

@@ -6,6 +6,7 @@
 //                             (block 0 also passes the grand total to commit), re-reads the chunk,
 //                             block-local scan + chunk offset, calls dst(i, exclusive_prefix, value)
 //                             for every item
+// Sequences of at most kScanOne items: scan_one, one launch.
 // Src: __device__ uint64_t size() const; __device__ uint32_t operator()(uint64_t i) const;
 // static constexpr int kItems: consecutive items per thread and tile of scan_down
 #pragma once
@@ -166,6 +167,61 @@ __global__ void __launch_bounds__(kScanThreads)
 		}
 		base += total;
 	}
+}
+
+// A short sequence in one launch of one block: before(), the scan, after(), with block barriers between
+// (after() sees what dst and commit wrote).  Small builds are bound by launches and their gaps (24 launches
+// and copies, 200 us for 1000 triangles at 2^6); the two launches above take 2.8 + 3.3 us whatever the
+// length.  The line lies at one trip of the block: 14,000 triangles of spheres at 2^8 (9,363 rank chunks)
+// build in 192 us with it there, 199 us with up to 16384 items in one block and up to 65536; 60,000 at
+// 2^9 in 219, 220 and 294 us.
+constexpr int kOneThreads = 1024;
+constexpr uint64_t kScanOne = 4096;
+struct NoStep {
+	__device__ void operator()() const {}
+};
+template <class Src, class Dst, class Commit, class Before, class After>
+__global__ void __launch_bounds__(kOneThreads)
+    scan_one(Src src, Dst dst, Commit commit, Before before, After after) {
+	constexpr int kItems = Src::kItems, kWaves = kOneThreads / 64;
+	__shared__ uint64_t s_wave[kWaves];
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	before();
+	__syncthreads();
+	const uint64_t n = src.size();
+	uint64_t base = 0;
+	for (uint64_t t0 = 0; t0 < n; t0 += (uint64_t)kOneThreads * kItems) {
+		uint32_t v[kItems];
+		const uint64_t first = t0 + (uint64_t)threadIdx.x * kItems;
+		uint64_t sum = 0;
+#pragma unroll
+		for (int k = 0; k < kItems; ++k) {
+			v[k] = first + k < n ? src(first + k) : 0u;
+			sum += v[k];
+		}
+		const uint64_t incl = wave_incl_scan(sum);
+		if (lane == 63)
+			s_wave[wave] = incl;
+		__syncthreads();
+		uint64_t run = base + incl - sum;
+#pragma unroll
+		for (int w = 0; w < kWaves; ++w) {
+			run += w < wave ? s_wave[w] : 0;
+			base += s_wave[w];
+		}
+		__syncthreads();
+#pragma unroll
+		for (int k = 0; k < kItems; ++k) {
+			if (first + k < n)
+				dst(first + k, run, v[k]);
+			run += v[k];
+		}
+	}
+	if (threadIdx.x == 0)
+		commit(base);
+	__threadfence_block();
+	__syncthreads();
+	after();
 }
 
 } // namespace svo

@@ -20,7 +20,19 @@ __global__ void __launch_bounds__(kThreads) copy_u8(uint8_t *__restrict__ dst, c
 		dst[i] = src[i];
 }
 
+// A table that came as kernel argument: no staging slot, no copy command.
+__global__ void __launch_bounds__(kThreads) table_set(uint32_t *__restrict__ dst, uint32_t words, SmallTable t) {
+	const uint32_t i = threadIdx.x;
+	if (i < words)
+		dst[i] = t.w[i];
+}
+
 } // namespace
+
+hipError_t table_write(svo_ctx *ctx, void *dst, const SmallTable &t, size_t bytes) {
+	static_assert(kThreads >= SmallTable::kWords, "a word per thread");
+	return launch(ctx, "table", table_set, dim3(1), dim3(kThreads), 0, (uint32_t *)dst, (uint32_t)(bytes / 4), t);
+}
 
 int copy_device(svo_ctx *ctx, void *dst, const void *src, uint64_t bytes) {
 	if (bytes == 0)

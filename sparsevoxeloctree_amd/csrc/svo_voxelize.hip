@@ -428,16 +428,25 @@ __global__ void __launch_bounds__(kThreads)
 	}
 }
 
-// Per scene: first fragment and fragment count from the scanned offsets (total = all fragments).
-__global__ void vox_seg_totals(VoxSeg *segs, const uint64_t *__restrict__ tbeg, uint32_t S, uint64_t T,
-                               const uint64_t *__restrict__ offsets, const uint64_t *__restrict__ total) {
-	const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-	if (s >= S)
-		return;
+// Scene s: first fragment and fragment count from the scanned offsets (total = all fragments), also into
+// the host's copy of the descriptors (out, pinned memory) when there is one.
+__device__ __forceinline__ void vox_seg_total(VoxSeg *segs, const uint64_t *tbeg, uint32_t s, uint64_t T,
+                                              const uint64_t *offsets, const uint64_t *total, VoxSeg *out) {
 	const uint64_t b = tbeg[s] < T ? offsets[tbeg[s]] : *total;
 	const uint64_t e = tbeg[s + 1u] < T ? offsets[tbeg[s + 1u]] : *total;
-	segs[s].frag_begin = b;
-	segs[s].F = e - b;
+	VoxSeg g = segs[s];
+	g.frag_begin = b;
+	g.F = e - b;
+	segs[s].frag_begin = g.frag_begin;
+	segs[s].F = g.F;
+	if (out)
+		out[s] = g;
+}
+__global__ void vox_seg_totals(VoxSeg *segs, const uint64_t *__restrict__ tbeg, uint32_t S, uint64_t T,
+                               const uint64_t *__restrict__ offsets, const uint64_t *__restrict__ total, VoxSeg *out) {
+	const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+	if (s < S)
+		vox_seg_total(segs, tbeg, s, T, offsets, total, out);
 }
 
 // One fragment: depth at the pixel centre, clamps, swizzle back (voxelizer.frag:17-25) and packing
@@ -696,6 +705,20 @@ struct OffsetDst {
 	__device__ void operator()(uint64_t i, uint64_t k, uint32_t) const { offsets[i] = k; }
 };
 
+struct SegTotals { // vox_seg_totals after a scan of one block
+	VoxSeg *segs;
+	const uint64_t *tbeg;
+	uint32_t S;
+	uint64_t T;
+	const uint64_t *offsets, *total;
+	VoxSeg *out;
+	__device__ void operator()() const {
+		if (threadIdx.x < S)
+			vox_seg_total(segs, tbeg, threadIdx.x, T, offsets, total, out);
+	}
+};
+static_assert(kMaxBatch <= kOneThreads, "a scene per thread");
+
 // ---- normalisation (src/Scene.cpp:62-99) -------------------------------------------------------
 // Per-block bounding box of the vertices -> parts[6 * b].
 __global__ void __launch_bounds__(kThreads) norm_bbox(const float *__restrict__ xyz, uint64_t nverts, float *parts) {
@@ -830,6 +853,28 @@ void vox_batch_release(svo_ctx *ctx, VoxBatch *vb) {
 	vb->general = nullptr;
 }
 
+namespace {
+// Counts -> offsets, the sum into total, the scenes' first fragments and counts (out: see vox_seg_total).
+hipError_t vox_scan(svo_ctx *ctx, const VoxBatch *vb, uint64_t *total, VoxSeg *out) {
+	const uint64_t T = vb->Ttot;
+	const uint32_t S = vb->S;
+	const CountSrc src{vb->offsets, T};
+	hipError_t e;
+	if (T <= kScanOne)
+		return launch(ctx, "vox_scan", scan_one<CountSrc, OffsetDst, TotalCommit, NoStep, SegTotals>, dim3(1),
+		              dim3(kOneThreads), 0, src, OffsetDst{vb->offsets}, TotalCommit{total}, NoStep{},
+		              SegTotals{vb->segs, vb->tbeg, S, T, vb->offsets, total, out});
+	if ((e = launch(ctx, "vox_scan_reduce", scan_reduce<CountSrc>, dim3(kScanBlocks), dim3(kScanThreads), 0, src,
+	                ctx->d_scan_parts)) != hipSuccess ||
+	    (e = launch(ctx, "vox_scan_down", scan_down<CountSrc, OffsetDst, TotalCommit>, dim3(kScanBlocks),
+	                dim3(kScanThreads), 0, src, OffsetDst{vb->offsets}, (const uint64_t *)ctx->d_scan_parts,
+	                TotalCommit{total})) != hipSuccess)
+		return e;
+	return launch(ctx, "vox_seg_totals", vox_seg_totals, dim3(div_up(S, 64)), dim3(64), 0, vb->segs,
+	              (const uint64_t *)vb->tbeg, S, T, (const uint64_t *)vb->offsets, (const uint64_t *)total, out);
+}
+} // namespace
+
 // Count pass over a batch + scan + one read-back of every scene's F + allocation of the lists
 // (Voxelizer::count_and_create_fragment_list, src/Voxelizer.cpp:134-179).
 int voxelize_count_batch(svo_ctx *ctx, svo_fraglist *const *fls, uint32_t S, VoxBatch *vb) {
@@ -874,32 +919,18 @@ int voxelize_count_batch(svo_ctx *ctx, svo_fraglist *const *fls, uint32_t S, Vox
 		if (int rc = upload_table(ctx, vb->segs, tables.data(), tables.size()))
 			return rc; // general[0] = 0 came with the tables
 	}
-	int rc = SVO_OK;
 	uint64_t *total = ctx->d_scan_parts + 2 * kScanBlocks;
+	VoxSeg *out = nullptr;
+	if (S <= kReadbackScenes && !(out = static_cast<VoxSeg *>(readback_slot(ctx, sizeof(VoxSeg) * S))))
+		return SVO_ERR_INVALID_ARGUMENT;
 	ctx->t_count.start(ctx->stream);
-	if (T > 0) {
-		if ((e = launch_count(ctx, vb)) != hipSuccess)
-			return hip_check(ctx, e, "vox_count");
-		CountSrc src{vb->offsets, T};
-		if ((e = launch(ctx, "vox_scan_reduce", scan_reduce<CountSrc>, dim3(kScanBlocks), dim3(kScanThreads), 0, src,
-		                ctx->d_scan_parts)) != hipSuccess)
-			return hip_check(ctx, e, "vox_scan_reduce");
-		if ((e = launch(ctx, "vox_scan_down", scan_down<CountSrc, OffsetDst, TotalCommit>, dim3(kScanBlocks),
-		                dim3(kScanThreads), 0, src, OffsetDst{vb->offsets}, (const uint64_t *)ctx->d_scan_parts,
-		                TotalCommit{total})) != hipSuccess)
-			return hip_check(ctx, e, "vox_scan_down");
-	} else if ((e = launch(ctx, "vox_zero", vox_zero_counter, dim3(1), dim3(1), 0,
-	                       reinterpret_cast<uint32_t *>(total))) != hipSuccess ||
-	           (e = launch(ctx, "vox_zero", vox_zero_counter, dim3(1), dim3(1), 0,
-	                       reinterpret_cast<uint32_t *>(total) + 1)) != hipSuccess) {
-		return hip_check(ctx, e, "vox_zero");
-	}
-	if ((e = launch(ctx, "vox_seg_totals", vox_seg_totals, dim3(div_up(S, 64)), dim3(64), 0, vb->segs,
-	                (const uint64_t *)vb->tbeg, S, T, (const uint64_t *)vb->offsets, (const uint64_t *)total)) !=
-	    hipSuccess)
-		return hip_check(ctx, e, "vox_seg_totals");
+	if (T > 0 && (e = launch_count(ctx, vb)) != hipSuccess)
+		return hip_check(ctx, e, "vox_count");
+	if ((e = vox_scan(ctx, vb, total, out)) != hipSuccess) // without triangles: every count 0
+		return hip_check(ctx, e, "vox_scan");
 	ctx->t_count.stop(ctx->stream);
-	if ((rc = download_table(ctx, vb->h_segs.data(), vb->segs, sizeof(VoxSeg) * S)) != SVO_OK)
+	if (int rc = out ? readback_wait(ctx, vb->h_segs.data(), out, sizeof(VoxSeg) * S)
+	                 : download_table(ctx, vb->h_segs.data(), vb->segs, sizeof(VoxSeg) * S))
 		return rc;
 	uint64_t Ftot = 0;
 	for (uint32_t s = 0; s < S; ++s) {
@@ -979,21 +1010,11 @@ int voxelize_plan_init(svo_ctx *ctx, VoxBatch *vb, svo_fraglist *const *fls, uin
 // Count pass of a plan: general list cleared by a kernel (the pass may be captured, so no
 // memset), counts, scan into offsets and fend[0] = total, per-scene F and frag_begin.
 hipError_t voxelize_plan_count(svo_ctx *ctx, VoxBatch *vb) {
-	const uint64_t T = vb->Ttot;
-	const uint32_t S = vb->S;
 	hipError_t e;
 	if ((e = launch(ctx, "vox_zero", vox_zero_counter, dim3(1), dim3(1), 0, vb->general)) != hipSuccess ||
 	    (e = launch_count(ctx, vb)) != hipSuccess)
 		return e;
-	CountSrc src{vb->offsets, T};
-	if ((e = launch(ctx, "vox_scan_reduce", scan_reduce<CountSrc>, dim3(kScanBlocks), dim3(kScanThreads), 0, src,
-	                ctx->d_scan_parts)) != hipSuccess ||
-	    (e = launch(ctx, "vox_scan_down", scan_down<CountSrc, OffsetDst, TotalCommit>, dim3(kScanBlocks),
-	                dim3(kScanThreads), 0, src, OffsetDst{vb->offsets}, (const uint64_t *)ctx->d_scan_parts,
-	                TotalCommit{vb->fend})) != hipSuccess)
-		return e;
-	return launch(ctx, "vox_seg_totals", vox_seg_totals, dim3(div_up(S, 64)), dim3(64), 0, vb->segs,
-	              (const uint64_t *)vb->tbeg, S, T, (const uint64_t *)vb->offsets, (const uint64_t *)vb->fend);
+	return vox_scan(ctx, vb, vb->fend, nullptr);
 }
 
 // Fill pass of a plan: writes nothing when fend[1] (set between the passes) is 0.
