@@ -49,8 +49,9 @@ namespace {
 constexpr int kThreads = 256;
 constexpr uint32_t kLdsBucket = 2048; // largest bucket sorted in LDS
 constexpr uint32_t kRegBucket = 16;   // leaf blocks up to this size: one thread each (build_fold)
-constexpr uint32_t kWaveBucket = 64;  // up to this size: one wave each (build_fold_mid)
-constexpr uint32_t kWideBucket = 512; // up to this size: one wave each, sorted in LDS (build_fold_wide)
+constexpr uint32_t kPairBucket = 32;  // up to this size: half a wave each (build_fold_lists)
+constexpr uint32_t kWaveBucket = 64;  // up to this size: a wave each (build_fold_lists)
+constexpr uint32_t kWideBucket = 512; // up to this size: one wave each, sorted in LDS (build_fold_lists)
 
 // Effective voxel coordinate seen by the reference's descent: the coordinate's bits, saturating
 // at res-1 for coordinates >= res (shader/octree_tag_node.comp:18-30).
@@ -764,12 +765,12 @@ __device__ __forceinline__ void store_block(uint32_t *oct, uint64_t block, const
 
 // Work lists of leaf blocks too large for build_fold: list[0..2] = mid, big and wide counts; mid
 // blocks (17..64 fragments) at list[3 ..], big ones (> 512) at list[3 + cap ..], wide ones
-// (65..512) at list[3 + 2 cap ..] (each list holds at most Ftot / 17).  Every lane of the wave calls
-// it (the appends are aggregated per wave).
-__device__ __forceinline__ void push_bins(uint32_t *list, uint64_t cap, uint32_t j, bool mid, bool wide, bool big) {
-	const uint32_t qm = wave_append(&list[0], mid), qb = wave_append(&list[1], big), qw = wave_append(&list[2], wide);
-	if (mid && qm < cap)
-		list[3u + qm] = j;
+// (65..512) at list[3 + 2 cap ..] (each list holds at most Ftot / 17).  The mid list is long, and atomics on
+// one address go one after another (12 ns each): the block appends to it once a step, 57,000 -> 14,000
+// atomics and build_fold 712 -> 452 us for 32 mixed scenes.  This is for the big and wide ones: every
+// lane of the wave calls it (the appends are aggregated per wave).
+__device__ __forceinline__ void push_bins(uint32_t *list, uint64_t cap, uint32_t j, bool wide, bool big) {
+	const uint32_t qb = wave_append(&list[1], big), qw = wave_append(&list[2], wide);
 	if (big && qb < cap)
 		list[3u + cap + qb] = j;
 	if (wide && qw < cap)
@@ -913,7 +914,7 @@ __global__ void __launch_bounds__(kThreads)
 	const uint64_t nbins = bbeg[S];
 	constexpr uint32_t kWaves = kThreads / 64;
 	__shared__ uint32_t s_bin[kThreads], s_n[kThreads];
-	__shared__ uint32_t s_cls[kWaves][3];
+	__shared__ uint32_t s_cls[kWaves][5], s_mid;
 	__shared__ uint32_t s_leaf[8 * kThreads]; // the threads' leaf words, by child slot
 	__shared__ uint32_t s_at[kThreads];       // first slot of the bin's bucket
 	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -930,34 +931,37 @@ __global__ void __launch_bounds__(kThreads)
 	for (uint64_t base = (uint64_t)blockIdx.x * kThreads; base < nbins; base += stride) {
 		const uint64_t jj = base + threadIdx.x;
 		const uint32_t n = next_n, slot0 = next_slot;
-		uint32_t cls = 3; // classes: <= 4, <= 8, <= 16 fragments; 3 = not folded here
+		uint32_t cls = 5; // classes: <= 4, <= 8, <= 16 fragments; for the mid list <= 32, <= 64; 5 = neither
 		if (base + stride < nbins)
 			ahead(base + stride);
 		if (jj < nbins) {
-			cls = n <= 4u ? 0u : n <= 8u ? 1u : n <= kRegBucket ? 2u : 3u;
+			cls = n <= 4u ? 0u : n <= 8u ? 1u : n <= kRegBucket ? 2u : n <= kPairBucket ? 3u : n <= kWaveBucket ? 4u : 5u;
 		}
-		const bool rest = jj < nbins && cls == 3u;
-		push_bins(list, cap, (uint32_t)jj, rest && n <= kWaveBucket, rest && n > kWaveBucket && n <= kWideBucket,
-		          rest && n > kWideBucket);
-		const uint64_t m0 = __ballot(cls == 0u), m1 = __ballot(cls == 1u), m2 = __ballot(cls == 2u);
-		if (lane == 0u) {
-			s_cls[wave][0] = (uint32_t)__popcll(m0);
-			s_cls[wave][1] = (uint32_t)__popcll(m1);
-			s_cls[wave][2] = (uint32_t)__popcll(m2);
+		const bool rest = jj < nbins && cls == 5u;
+		push_bins(list, cap, (uint32_t)jj, rest && n <= kWideBucket, rest && n > kWideBucket);
+		uint64_t mine = 0u; // the wave's lanes of the same class
+#pragma unroll
+		for (uint32_t c = 0; c < 5u; ++c) {
+			const uint64_t m = __ballot(cls == c);
+			mine = cls == c ? m : mine;
+			if (lane == c)
+				s_cls[wave][c] = (uint32_t)__popcll(m);
 		}
 		__syncthreads();
-		uint32_t pos = 0, total = 0;
+		uint32_t pos = 0, total = 0, mids = 0;
 #pragma unroll
-		for (uint32_t c = 0; c < 3u; ++c)
+		for (uint32_t c = 0; c < 5u; ++c)
 #pragma unroll
 			for (uint32_t v = 0; v < kWaves; ++v) {
 				const uint32_t k = s_cls[v][c];
 				pos += (c < cls || (c == cls && v < wave)) ? k : 0u;
-				total += k;
+				(c < 3u ? total : mids) += k;
 			}
+		pos += (uint32_t)__popcll(mine & below);
+		uint32_t first = 0u; // of the step's places in the mid list; used after the fold
+		if (threadIdx.x == 0u && mids)
+			first = atomicAdd(&list[0], mids);
 		if (cls < 3u) {
-			const uint64_t mine = cls == 0u ? m0 : cls == 1u ? m1 : m2;
-			pos += (uint32_t)__popcll(mine & below);
 			s_bin[pos] = (uint32_t)jj;
 			s_n[pos] = n;
 			s_at[pos] = slot0;
@@ -986,7 +990,11 @@ __global__ void __launch_bounds__(kThreads)
 				words[c] = w[c * kThreads];
 			store_block(t.oct, t.block, words);
 		}
+		if (threadIdx.x == 0u)
+			s_mid = first;
 		__syncthreads();
+		if ((cls == 3u || cls == 4u) && s_mid + pos - total < cap)
+			list[3u + s_mid + pos - total] = (uint32_t)jj;
 	}
 }
 
@@ -1010,75 +1018,154 @@ template <class Rgb> __device__ __forceinline__ uint32_t fold_run(uint32_t beg, 
 	return leaf.word();
 }
 
-// Leaf blocks of 17..64 fragments, one wave each: lane i holds key i (padding: +inf); a bitonic sort over
-// lane shuffles orders them by leaf slot and key, so every leaf's fragments are consecutive and
-// ascending.  Lane s < 8 then folds the run of slot s from LDS.  A raw scene's wave sorts
-// (slot, whole fragment) pairs instead.  Blocks blk of nblk of the list launch; s_col: 64 words of LDS
-// per wave.
-__device__ void fold_mid_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__restrict__ segs,
-                                const uint64_t *__restrict__ bbeg, uint32_t S, const uint32_t *__restrict__ cnt,
-                                const uint32_t *__restrict__ aux, const uint32_t *__restrict__ bucket,
-                                const uint32_t *list, uint64_t cap, uint32_t (*s_col)[64]) {
-	constexpr uint32_t kWaves = kThreads / 64;
-	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-	uint64_t count = list[0];
-	if (count > cap)
-		count = cap;
-	for (uint64_t base = (uint64_t)blk * kWaves; base < count; base += (uint64_t)nblk * kWaves) {
-		const uint64_t item = base + wave;
-		if (item >= count)
-			break; // wave-uniform; no block barrier follows
-		const uint32_t j = list[3u + item];
-		const uint32_t n = cnt[j];
-		const uint32_t s = S == 1u ? 0u : seg_find(bbeg, S, j);
-		const LeafTarget t = leaf_target(segs[s], bbeg, s, j);
-		uint32_t key = lane < n ? bucket[aux[j] + lane] : kRawKey, slot = key >> 27u;
-		if (t.raw) { // wave-uniform
+// xor-shuffle by a power of two inside the wave: data-parallel moves where they reach, else LDS permutes.
+template <uint32_t kD> __device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+	if constexpr (kD == 1u)
+		return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true); // quad_perm 1 0 3 2
+	else if constexpr (kD == 2u)
+		return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, true); // quad_perm 2 3 0 1
+	else if constexpr (kD <= 16u)
+		return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, (int)(kD << 10 | 0x1fu)); // xor within 32 lanes
+	else
+		return (uint32_t)__shfl_xor((int)v, (int)kD, 64);
+}
+// Steps d = kD .. 1 of a bitonic merge: bit[b] is all ones in the lanes with bit b of their id set, dir
+// likewise in the lanes that sort downwards.  The median of (own, other, 0 or ~0) is their minimum or
+// maximum, so a step is an exclusive or, a move and a v_med3.
+template <uint32_t kB> __device__ __forceinline__ void wave_merge(uint32_t &key, const uint32_t (&bit)[6], uint32_t dir) {
+	const uint32_t other = lane_xor<1u << kB>(key), bound = dir ^ bit[kB];
+	key = umax32(umin32(key, other), umin32(umax32(key, other), bound));
+	if constexpr (kB > 0u)
+		wave_merge<kB - 1u>(key, bit, dir);
+}
+// Ascending bitonic sort of the keys of each half wave, or of the wave.
+template <bool kHalves> __device__ __forceinline__ void wave_sort(uint32_t &key, const uint32_t (&bit)[6]) {
+	wave_merge<0>(key, bit, bit[1]);
+	wave_merge<1>(key, bit, bit[2]);
+	wave_merge<2>(key, bit, bit[3]);
+	wave_merge<3>(key, bit, bit[4]);
+	wave_merge<4>(key, bit, kHalves ? 0u : bit[5]);
+	if constexpr (!kHalves)
+		wave_merge<5>(key, bit, 0u);
+}
+
+// Leaf blocks of 17..64 fragments: a wave takes 8 at a time (bins, n, at: numbers, sizes and bucket
+// positions, `count` of them), sorts one after another (two side by side up to 32 fragments) so that every
+// leaf's fragments are consecutive and ascending, and then folds the 64 leaves, one per lane.  A raw
+// scene's block sorts (slot, whole fragment) pairs.  col: 8 x 64 words of LDS; t: where leaf block
+// lane / 8 goes.  Bound by VALU: one block per wave, its runs folded by 8 lanes, and a step of the sort as
+// an LDS permute, a minimum, a maximum and a select took 520 us for the listed blocks of 32 mixed scenes
+// (100M fragments), this takes 150.
+__device__ __forceinline__ void fold_mid(const uint32_t *n, const uint32_t *at, uint32_t count, uint32_t *col,
+                                         const uint32_t *__restrict__ bucket, const LeafTarget &t) {
+	const uint32_t lane = threadIdx.x & 63u, leaf = lane & 7u, mine = lane >> 3;
+	const uint64_t raws = __ballot(t.raw != nullptr);
+	uint32_t bit[6];
+#pragma unroll
+	for (uint32_t b = 0; b < 6u; ++b)
+		bit[b] = 0u - (lane >> b & 1u);
+	uint32_t beg = 0u, len = 0u;
+	// the keys of one block are in the wave (sorted; lanes past its end: no slot): colours to LDS, run of
+	// each leaf to its lane
+	auto runs = [&](uint32_t item, uint32_t key, uint32_t slot) {
+		col[item * 64u + lane] = key & 0xffffffu;
+#pragma unroll
+		for (uint32_t u = 0; u < 8u; ++u) {
+			const uint64_t m = __ballot(slot == u);
+			if (mine == item && leaf == u) {
+				beg = m ? (uint32_t)__ffsll((unsigned long long)m) - 1u : 0u;
+				len = (uint32_t)__popcll(m);
+			}
+		}
+	};
+#pragma unroll 1
+	for (uint32_t i = 0; i < count; i += 2u) {
+		const bool two = i + 1u < count;
+		const uint32_t n0 = (uint32_t)__builtin_amdgcn_readfirstlane(n[i]),
+		               n1 = two ? (uint32_t)__builtin_amdgcn_readfirstlane(n[i + 1u]) : 0u;
+		const bool raw0 = raws >> (8u * i) & 1u, raw1 = two && (raws >> (8u * i + 8u) & 1u);
+		if (umax32(n0, n1) <= kPairBucket && !raw0 && !raw1) {
+			const uint32_t half = lane >> 5, l = lane & 31u, item = i + half;
+			const bool have = l < (half ? n1 : n0);
+			uint32_t key = have ? bucket[at[item] + l] : kRawKey;
+			wave_sort<true>(key, bit);
+			const uint32_t slot = key >> 27u;
+			col[(i + half) * 64u + l] = key & 0xffffffu;
+#pragma unroll
+			for (uint32_t u = 0; u < 8u; ++u) {
+				const uint64_t both = __ballot(slot == u);
+				const uint32_t m = (mine & 1u) ? (uint32_t)(both >> 32) : (uint32_t)both;
+				if ((mine & ~1u) == i && leaf == u) {
+					beg = m ? (uint32_t)__ffs((int)m) - 1u : 0u;
+					len = (uint32_t)__popc(m);
+				}
+			}
+			continue;
+		}
+#pragma unroll 1
+		for (uint32_t k = 0; k < (two ? 2u : 1u); ++k) {
+			const uint32_t item = i + k, ni = k ? n1 : n0;
+			uint32_t key = lane < ni ? bucket[at[item] + lane] : kRawKey;
+			if (!(k ? raw1 : raw0)) {
+				wave_sort<false>(key, bit);
+				runs(item, key, key >> 27u);
+				continue;
+			}
+			const uint32_t res = (uint32_t)__shfl((int)t.res, (int)(8u * item), 64);
+			const uint2 *frags = reinterpret_cast<const uint2 *>(
+			    __shfl((unsigned long long)reinterpret_cast<uintptr_t>(t.raw), (int)(8u * item), 64));
 			uint64_t whole = ~0ull;
-			slot = 8u;
-			if (lane < n) {
-				whole = frag_key(t.raw[key]);
-				slot = key_slot(whole, t.res);
+			uint32_t slot = 8u;
+			if (lane < ni) {
+				whole = frag_key(frags[key]);
+				slot = key_slot(whole, res);
 			}
 #pragma unroll 1
-			for (uint32_t k = 2; k <= 64u; k <<= 1)
+			for (uint32_t q = 2; q <= 64u; q <<= 1)
 #pragma unroll 1
-				for (uint32_t d = k >> 1; d > 0u; d >>= 1) {
+				for (uint32_t d = q >> 1; d > 0u; d >>= 1) {
 					const uint64_t ok = __shfl_xor(whole, (int)d, 64);
 					const uint32_t os = __shfl_xor(slot, (int)d, 64);
 					const bool other_less = os < slot || (os == slot && ok < whole);
-					const bool take_min = ((lane & k) == 0u) == ((lane & d) == 0u);
+					const bool take_min = ((lane & q) == 0u) == ((lane & d) == 0u);
 					const bool take_other = take_min == other_less;
 					whole = take_other ? ok : whole;
 					slot = take_other ? os : slot;
 				}
-			key = (uint32_t)whole;
-		} else {
-#pragma unroll
-			for (uint32_t k = 2; k <= 64u; k <<= 1)
-#pragma unroll
-				for (uint32_t d = k >> 1; d > 0u; d >>= 1) {
-					const uint32_t ok = __shfl_xor(key, (int)d, 64);
-					const bool take_min = ((lane & k) == 0u) == ((lane & d) == 0u);
-					key = take_min ? umin32(key, ok) : umax32(key, ok);
-				}
-			slot = key >> 27u;
+			runs(item, (uint32_t)whole, slot);
 		}
-		s_col[wave][lane] = key & 0xffffffu;
+	}
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+	if (mine < count)
+		t.oct[8u * t.block + leaf] = fold_run(beg, beg + len, [&](uint32_t i) { return col[mine * 64u + i]; });
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+}
+
+// Leaf blocks of 17..64 fragments from the list, 8 per wave and trip.  Blocks blk of nblk of the list
+// launch; s_col, s_item: 512 and 16 words of LDS per wave.
+__device__ void fold_mid_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__restrict__ segs,
+                                const uint64_t *__restrict__ bbeg, uint32_t S, const uint32_t *__restrict__ cnt,
+                                const uint32_t *__restrict__ aux, const uint32_t *__restrict__ bucket,
+                                const uint32_t *list, uint64_t cap, uint32_t *s_col, uint32_t *s_item) {
+	constexpr uint32_t kWaves = kThreads / 64;
+	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+	uint32_t *n = s_item + wave * 16u, *at = n + 8u;
+	uint64_t count = list[0];
+	if (count > cap)
+		count = cap;
+	for (uint64_t base = 8u * ((uint64_t)blk * kWaves + wave); base < count; base += 8u * (uint64_t)nblk * kWaves) {
+		const uint32_t m = (uint32_t)(count - base < 8u ? count - base : 8u), mine = lane >> 3;
+		const uint32_t j = list[3u + base + (mine < m ? mine : 0u)]; // of leaf block lane / 8
+		if (mine < m && (lane & 7u) == 0u) {
+			n[mine] = cnt[j];
+			at[mine] = aux[j];
+		}
 		__builtin_amdgcn_wave_barrier();
 		__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-		uint64_t run = 0;
-#pragma unroll
-		for (uint32_t u = 0; u < 8u; ++u) {
-			const uint64_t mu = __ballot(slot == u);
-			run = lane == u ? mu : run;
-		}
-		if (lane < 8u) {
-			const uint32_t beg = run ? (uint32_t)__ffsll((unsigned long long)run) - 1u : 0u;
-			t.oct[8u * t.block + lane] =
-			    fold_run(beg, beg + (uint32_t)__popcll(run), [&](uint32_t i) { return s_col[wave][i]; });
-		}
-		__builtin_amdgcn_wave_barrier();
+		const uint32_t s = S == 1u ? 0u : seg_find(bbeg, S, j);
+		fold_mid(n, at, m, s_col + wave * 512u, bucket, leaf_target(segs[s], bbeg, s, j));
 	}
 }
 
@@ -1252,10 +1339,10 @@ __global__ void __launch_bounds__(kThreads)
 	static_assert(kWaves * kWideBucket == kLdsBucket, "the wide and big roles share the key arrays");
 	__shared__ uint64_t s_keys[kLdsBucket];
 	__shared__ uint8_t s_slots[kLdsBucket];
-	__shared__ uint32_t s_beg[kWaves][8], s_end[kWaves][8];
+	__shared__ uint32_t s_beg[kWaves][8], s_end[kWaves][8], s_item[kWaves * 16];
 	if (blockIdx.x < g_mid)
 		fold_mid_blocks(blockIdx.x, g_mid, segs, bbeg, S, cnt, aux, bucket, list, cap,
-		                reinterpret_cast<uint32_t (*)[64]>(s_keys));
+		                reinterpret_cast<uint32_t *>(s_keys), s_item);
 	else if (blockIdx.x < g_mid + g_wide)
 		fold_wide_blocks(blockIdx.x - g_mid, g_wide, segs, bbeg, S, cnt, aux, bucket, list, cap, s_keys, s_slots, s_beg,
 		                 s_end);
@@ -1424,7 +1511,7 @@ int node_phase(svo_ctx *ctx, BuildBatch &bb, bool maybe_raw) {
 	// blocks (17, 65 and 513 fragments at least), a wave or a block each
 	constexpr uint64_t kWaves = kThreads / 64u;
 	const uint32_t cu = (uint32_t)ctx->cu_count;
-	const uint32_t g_mid = (uint32_t)std::min<uint64_t>(cu * 8u, bb.Ftot / (17u * kWaves) + 1u),
+	const uint32_t g_mid = (uint32_t)std::min<uint64_t>(cu * 8u, bb.Ftot / (17u * 8u * kWaves) + 1u),
 	               g_wide = (uint32_t)std::min<uint64_t>(cu * 8u, bb.Ftot / (65u * kWaves) + 1u),
 	               g_big = (uint32_t)std::min<uint64_t>(cu * 2u, bb.Ftot / 513u + 1u);
 	if ((e = launch(ctx, "build_fold_lists", build_fold_lists, dim3(g_mid + g_wide + g_big), dim3(kThreads), 0, segs,
