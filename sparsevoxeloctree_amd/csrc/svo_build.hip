@@ -74,6 +74,25 @@ __device__ __forceinline__ uint64_t spread3(uint32_t v) {
 	return x;
 }
 
+// Every third bit, for 10-bit inputs.
+__device__ __forceinline__ uint32_t spread3_10(uint32_t x) {
+	x = (x | x << 16) & 0x030000FFu;
+	x = (x | x << 8) & 0x0300F00Fu;
+	x = (x | x << 4) & 0x030C30C3u;
+	return (x | x << 2) & 0x09249249u;
+}
+
+// Inclusive sum over the lanes of a wave, by data-parallel moves (no LDS).
+__device__ __forceinline__ uint32_t wave_incl_sum(uint32_t v) {
+	v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true); // row_shr 1
+	v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true); // row_shr 2
+	v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true); // row_shr 4
+	v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true); // row_shr 8
+	v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false); // lane 15 of a row to rows 1, 3
+	v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false); // lane 31 to rows 2, 3
+	return v;
+}
+
 // Morton code of a leaf: the child slots (x | y << 1 | z << 2) of depths 1..L, depth 1 highest.
 __device__ __forceinline__ uint64_t morton(uint32_t x, uint32_t y, uint32_t z) {
 	return spread3(x) | (spread3(y) << 1) | (spread3(z) << 2);
@@ -126,13 +145,15 @@ __global__ void __launch_bounds__(kThreads) bm_zero(uint32_t *B, uint64_t n, uin
 // fragment indices (BuildSeg::raw), compared by the fragments they name.
 constexpr uint32_t kRawKey = 0xFFFFFFFFu;
 
-__device__ __forceinline__ uint32_t leaf_key(uint2 f, uint32_t res) {
-	const uint32_t x = f.x & 0xfffu, y = (f.x >> 12u) & 0xfffu, z = (f.x >> 24u) | ((f.y >> 28u) << 8u);
-	const uint32_t sx = x >= res ? 1u : 0u, sy = y >= res ? 1u : 0u, sz = z >= res ? 1u : 0u;
-	const uint32_t slot = ((x - sx) & 1u) | ((y - sy) & 1u) << 1u | ((z - sz) & 1u) << 2u;
-	const uint32_t fz = sz ^ (res >= 256u ? 1u : 0u);
-	const uint32_t key = slot << 27u | fz << 26u | sy << 25u | sx << 24u | (f.y & 0xffffffu);
-	return umax32(umax32(x, y), z) > res ? kRawKey : key;
+// x, y, z: the effective coordinates (decode_frag).  A raw coordinate exceeds its effective one by 1 where
+// it saturates at res, by more above res.
+__device__ __forceinline__ uint32_t leaf_key(uint2 f, uint32_t res, uint32_t x, uint32_t y, uint32_t z) {
+	const uint32_t dx = (f.x & 0xfffu) - x, dy = ((f.x >> 12u) & 0xfffu) - y,
+	               dz = ((f.x >> 24u) | ((f.y >> 28u) << 8u)) - z;
+	const uint32_t slot = (x & 1u) | (y & 1u) << 1u | (z & 1u) << 2u;
+	const uint32_t flags = dx | dy << 1u | (dz ^ (res >= 256u ? 1u : 0u)) << 2u;
+	const uint32_t key = slot << 27u | flags << 24u | (f.y & 0xffffffu);
+	return umax32(umax32(dx, dy), dz) > 1u ? kRawKey : key;
 }
 
 // ---- tiles and runs ------------------------------------------------------------------------------
@@ -162,8 +183,10 @@ static_assert(kLines == kThreads, "one thread per group in the scan");
 // group by group in Morton order inside (neighbouring lanes of tag_runs then count in one 64-byte
 // line).  A fragment that finds no group in kProbes probes becomes a run of its own at the tile's end
 // (random slivers at 2^12 touch 152 groups on average, 288 at most).  Each group marks its nodes with
-// one load and, only if bits are missing, one atomic.  Bound by VALU (0.6 busy) and the latency of its
-// phases, at 8 waves per SIMD: 193 us for 35M fragments in a room.  kIndex: a second pass that only rewrites the
+// one load and, only if bits are missing, one atomic.  Bound by VALU issue (0.9 busy in a room) and LDS
+// atomics, at 8 waves per SIMD.  35M fragments in a room / 180M with slivers at 2^12 / 100M of 32 mixed
+// scenes: 192 / 1436 / 587 us, -> 180 / 1388 / 548 with packed sums, 32-bit Morton codes and scans by
+// data-parallel moves, -> 173 / 1351 / 493 with the group read before the compare-and-swap.  kIndex: a second pass that only rewrites the
 // keys (and their order) of the raw scenes' tiles as fragment indices.
 template <bool kIndex>
 __global__ void __launch_bounds__(kThreads)
@@ -209,15 +232,17 @@ __global__ void __launch_bounds__(kThreads)
 		place[u] = 0u;
 		if (threadIdx.x + u * kThreads >= n)
 			continue;
-		key[u] = leaf_key(fr[u], res);
-		wide |= key[u] == kRawKey;
 		uint32_t x, y, z;
 		decode_frag(fr[u], res, x, y, z);
+		key[u] = leaf_key(fr[u], res, x, y, z);
+		wide |= key[u] == kRawKey;
 		const uint32_t line = (x >> 3u) | (y >> 2u) << 9u | (z >> 2u) << 19u;
 		const uint32_t sub = (x >> 1u & 1u) | (y & 2u) | (z << 1u & 4u) | (x << 1u & 8u);
 		uint32_t h = (line * 2654435761u) >> 24u;
 		for (uint32_t probe = 0; probe < kProbes; ++probe) {
-			const uint32_t old = atomicCAS(&s_line[h], kEmpty, line);
+			uint32_t old = __hip_atomic_load(&s_line[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+			if (old == kEmpty) // lanes of one group read in one go; atomics on one word go one after another
+				old = atomicCAS(&s_line[h], kEmpty, line);
 			if (old == kEmpty || old == line) {
 				at[u] = h * 16u + sub;
 				break;
@@ -232,18 +257,19 @@ __global__ void __launch_bounds__(kThreads)
 		atomicOr(&raw[sc], 1u);
 	__syncthreads();
 	// first keys of the groups' nodes (thread h owns group h), marking
-	uint32_t v[8], sum = 0u, mask = 0u;
+	uint32_t v[8], halves = 0u, mask = 0u;
 #pragma unroll
 	for (uint32_t c = 0; c < 8u; ++c) {
 		v[c] = s_n[threadIdx.x * kLineStride + c];
-		sum += (v[c] & 0xffffu) + (v[c] >> 16u);
-		mask |= (v[c] & 0xffffu ? 1u << (2u * c) : 0u) | (v[c] >> 16u ? 2u << (2u * c) : 0u);
+		halves += v[c]; // a half sums up to kTile at most
+		mask |= umin32(v[c] & 0xffffu, 1u) << (2u * c) | umin32(v[c] >> 16u, 1u) << (2u * c + 1u);
 	}
+	const uint32_t sum = (halves & 0xffffu) + (halves >> 16u);
 	if (mask) {
 		const uint32_t line = s_line[threadIdx.x];
-		// the group's Morton index: the node's bits above the 4 of its place in the group
-		const uint32_t gn = (uint32_t)(morton((line & 0x1ffu) << 2u, (line >> 9u & 0x3ffu) << 1u,
-		                                      (line >> 19u & 0x3ffu) << 1u) >> 4);
+		// the group's Morton index: the node's bits above the 4 of its place in the group (x0 y0 z0 x1)
+		const uint32_t gn = spread3_10(line >> 9u & 0x3ffu) | spread3_10(line >> 19u & 0x3ffu) << 1u |
+		                    spread3_10(line & 0x1ffu) << 2u;
 		s_node[threadIdx.x] = gn;
 		if (!kIndex && L > 1u) {
 			uint32_t *word = B + g.bm + g.off[L - 1u] + (gn >> 1u);
@@ -252,12 +278,7 @@ __global__ void __launch_bounds__(kThreads)
 				atomicOr(word, bits);
 		}
 	}
-	uint32_t incl = sum;
-#pragma unroll
-	for (uint32_t d = 1; d < 64u; d <<= 1) {
-		const uint32_t o = __shfl_up(incl, d, 64);
-		incl += (threadIdx.x & 63u) >= d ? o : 0u;
-	}
+	const uint32_t incl = wave_incl_sum(sum);
 	if ((threadIdx.x & 63u) == 63u)
 		s_wave[threadIdx.x >> 6] = incl;
 	__syncthreads();
@@ -295,12 +316,7 @@ __global__ void __launch_bounds__(kThreads)
 	__syncthreads();
 	if (threadIdx.x < 64u) { // run heads before each 32 keys
 		const uint32_t c = threadIdx.x < kTile / 32u ? (uint32_t)__popc(s_head[threadIdx.x]) : 0u;
-		uint32_t p = c;
-#pragma unroll
-		for (uint32_t d = 1; d < kTile / 32u; d <<= 1) {
-			const uint32_t o = __shfl_up(p, d, 64);
-			p += threadIdx.x >= d ? o : 0u;
-		}
+		const uint32_t p = wave_incl_sum(c);
 		if (threadIdx.x < kTile / 32u)
 			s_before[threadIdx.x] = p - c;
 		if (threadIdx.x == kTile / 32u - 1u)
