@@ -178,6 +178,16 @@ constexpr uint32_t kProbes = 32;
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;
 static_assert(kLines == kThreads, "one thread per group in the scan");
 
+// Home slot of a group in the tile's table: the low 3 bits of its Morton index (y0 z0 x0) under a hash of
+// the rest.  So the groups of a 2x2x2 cube are neighbours in the table and their runs in the tile, and
+// tag_runs counts them in common lines: room at 2^10 / slivers at 2^12 / 32 mixed scenes, tag_runs
+// 132 / 1340 / 276 -> 102 / 1078 / 213 us, while bm_group pays 173 / 1351 / 493 -> 182 / 1460 / 517.  5 or 6
+// Morton bits give tag_runs 3 us more and cost 8 here.
+__device__ __forceinline__ uint32_t group_slot(uint32_t line) {
+	const uint32_t rest = line & ~(1u | 1u << 9u | 1u << 19u);
+	return ((rest * 2654435761u) >> 24u & (kLines - 8u)) | (line >> 9u & 1u) | (line >> 18u & 2u) | (line << 2u & 4u);
+}
+
 // One block per tile.  Every fragment finds its group of 16 nodes in an LDS hash table and takes a
 // place in its node's counter; a scan over the counters turns them into offsets, so the runs come out
 // group by group in Morton order inside (neighbouring lanes of tag_runs then count in one 64-byte
@@ -186,7 +196,8 @@ static_assert(kLines == kThreads, "one thread per group in the scan");
 // one load and, only if bits are missing, one atomic.  Bound by VALU issue (0.9 busy in a room) and LDS
 // atomics, at 8 waves per SIMD.  35M fragments in a room / 180M with slivers at 2^12 / 100M of 32 mixed
 // scenes: 192 / 1436 / 587 us, -> 180 / 1388 / 548 with packed sums, 32-bit Morton codes and scans by
-// data-parallel moves, -> 173 / 1351 / 493 with the group read before the compare-and-swap.  kIndex: a second pass that only rewrites the
+// data-parallel moves, -> 173 / 1351 / 493 with the group read before the compare-and-swap
+// (and see group_slot).  kIndex: a second pass that only rewrites the
 // keys (and their order) of the raw scenes' tiles as fragment indices.
 template <bool kIndex>
 __global__ void __launch_bounds__(kThreads)
@@ -238,7 +249,7 @@ __global__ void __launch_bounds__(kThreads)
 		wide |= key[u] == kRawKey;
 		const uint32_t line = (x >> 3u) | (y >> 2u) << 9u | (z >> 2u) << 19u;
 		const uint32_t sub = (x >> 1u & 1u) | (y & 2u) | (z << 1u & 4u) | (x << 1u & 8u);
-		uint32_t h = (line * 2654435761u) >> 24u;
+		uint32_t h = group_slot(line);
 		for (uint32_t probe = 0; probe < kProbes; ++probe) {
 			uint32_t old = __hip_atomic_load(&s_line[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 			if (old == kEmpty) // lanes of one group read in one go; atomics on one word go one after another
@@ -663,7 +674,7 @@ __global__ void __launch_bounds__(kThreads)
 // the run's place in the bin's bucket, from per-bin counters.  A wave takes a tile's runs 64 at a time;
 // neighbouring lanes hold neighbouring nodes, so their counters share 64-byte lines and the L1 sends
 // one request per line (device-coherent atomics are done at the memory side, and each request stalls
-// the L2 for the reads behind it).  Bound by those requests: 2.7M in 134 us for the 9.4M runs of a room.
+// the L2 for the reads behind it).  Bound by those requests, 20 a nanosecond: 9.4M runs of a room in 102 us.
 __global__ void __launch_bounds__(kThreads)
     tag_runs(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ tbeg, uint32_t S,
              const uint32_t *__restrict__ B, const uint32_t *__restrict__ R, uint2 *__restrict__ runs,
@@ -715,7 +726,7 @@ __global__ void __launch_bounds__(kThreads)
 // Every key to its place in its bin's bucket (aux[j] = first slot of bin j), a wave per tile.  The wave
 // first turns the tile's runs into slots in LDS, with the keys already on their way, so a tile costs
 // three dependent loads; then lane i finds key i's run by the heads at or below it, and the lanes of a
-// run write neighbouring slots.  Bound by latency and part-line writes: 35M keys in 127 us (190 us with
+// run write neighbouring slots.  Bound by latency and part-line writes: 35M keys in 122 us (190 us with
 // every lane loading its key's run and bin offset itself).
 __global__ void __launch_bounds__(kThreads)
     scatter_runs(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ tbeg, uint32_t S,
