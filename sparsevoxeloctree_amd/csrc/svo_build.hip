@@ -579,63 +579,47 @@ __global__ void __launch_bounds__(kThreads)
 				store_parent_block(g.words, 0u, B[g.bm + g.off[1]] & 0xffu, g.fb[1], 0u);
 		}
 	}
-	uint32_t hint = 0;
-	for (uint64_t base = (uint64_t)blockIdx.x * kThreads; base < n; base += stride) {
-		const uint64_t i = base + threadIdx.x;
-		uint32_t k = kEmpty;
-		if (i < n)
-			with_seg<kThreads>(pw, M, hint, base, i, [&](uint32_t t) { k = t; });
-		const uint32_t k0 = __shfl(k, 0, 64);
-		if (k0 == kEmpty)
-			continue; // the wave is past the end (lane 0 holds its first item)
-		if (__all(k == k0 || k == kEmpty)) {
-			const uint32_t ku = __builtin_amdgcn_readfirstlane(k0);
-			const uint32_t d = 2u + ku / S;
-			const BuildSeg &g = segs[ku % S];
-			const uint64_t offp = g.bm + g.off[d - 1u], offc = g.bm + g.off[d]; // both start chunks
-			const uint64_t w0 = (i - lane) - pw[ku]; // lane 0's word
-			const uint32_t v = k != kEmpty ? B[offp + w0 + lane] : 0u, c = (uint32_t)__popc(v);
-			uint32_t incl = c;
-#pragma unroll
-			for (uint32_t dd = 1; dd < 64u; dd <<= 1) {
-				const uint32_t t = __shfl_up(incl, dd, 64);
-				incl += lane >= dd ? t : 0u;
-			}
-			const uint32_t excl = incl - c, T = __shfl(incl, 63, 64);
-			if (T == 0u)
-				continue;
-			uint32_t first = 0u; // rank of the wave's first parent among depth d-1
-			if (lane == 0u) {
-				uint32_t dummy;
-				first = bits_before(B, R, offp + w0, dummy) - R[offp >> 3];
-			}
-			const uint64_t blk0 = (uint64_t)g.fb[d - 1u] + __shfl(first, 0, 64);
-			const uint32_t fbd = g.fb[d];
-			// children of depth d before this word's 8-word chunk of B[d] (read only for occupied
-			// words: an empty padding word of a small B[d-1] may have no chunk)
-			const uint32_t rc = v != 0u ? R[(offc >> 3) + w0 + lane] - R[offc >> 3] : 0u;
-			for (uint32_t t0 = 0; t0 < T; t0 += 64u) {
-				const uint32_t j = t0 + lane; // the wave's j-th occupied parent
-				uint32_t o = 0u; // owner lane: the last with excl <= j
-#pragma unroll
-				for (uint32_t step = 32u; step >= 1u; step >>= 1) {
-					const uint32_t e = __shfl(excl, (int)(o + step), 64);
-					o = e <= j ? o + step : o;
-				}
-				const uint32_t vo = __shfl(v, (int)o, 64), eo = __shfl(excl, (int)o, 64), ro = __shfl(rc, (int)o, 64);
-				if (j < T) {
-					const uint32_t b = nth_bit(vo, j - eo); // the parent's bit in the owner's word
-					uint32_t cv; // the owner's chunk of B[d]: its word b / 4 holds the parent's byte
-					const uint32_t before = chunk_before(B + offc + 8u * (w0 + o), b >> 2u, cv);
-					const uint32_t sh = 8u * (b & 3u);
-					const uint32_t r = ro + before + (uint32_t)__popc(cv & ((1u << sh) - 1u));
-					store_parent_block(g.words, blk0 + j, (cv >> sh) & 0xffu, fbd, r);
-				}
-			}
-			continue;
+	// the 64 words from w0 on of segment ku, word w0 + lane being v
+	auto wave_words = [&](uint32_t ku, uint64_t w0, uint32_t v) {
+		const uint32_t d = 2u + ku / S;
+		const BuildSeg &g = segs[ku % S];
+		const uint64_t offp = g.bm + g.off[d - 1u], offc = g.bm + g.off[d]; // both start chunks
+		const uint32_t c = (uint32_t)__popc(v);
+		if (__ballot(v != 0u) == 0ull)
+			return; // most waves of a sparse level
+		const uint32_t incl = wave_incl_sum(c), excl = incl - c;
+		const uint32_t T = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+		uint32_t first = 0u; // rank of the wave's first parent among depth d-1
+		if (lane == 0u) {
+			uint32_t dummy;
+			first = bits_before(B, R, offp + w0, dummy) - R[offp >> 3];
 		}
-		if (k == kEmpty)
-			continue;
+		const uint64_t blk0 = (uint64_t)g.fb[d - 1u] + __shfl(first, 0, 64);
+		const uint32_t fbd = g.fb[d];
+		// children of depth d before this word's 8-word chunk of B[d] (read only for occupied
+		// words: an empty padding word of a small B[d-1] may have no chunk)
+		const uint32_t rc = v != 0u ? R[(offc >> 3) + w0 + lane] - R[offc >> 3] : 0u;
+		for (uint32_t t0 = 0; t0 < T; t0 += 64u) {
+			const uint32_t j = t0 + lane; // the wave's j-th occupied parent
+			uint32_t o = 0u; // owner lane: the last with excl <= j
+#pragma unroll
+			for (uint32_t step = 32u; step >= 1u; step >>= 1) {
+				const uint32_t e = __shfl(excl, (int)(o + step), 64);
+				o = e <= j ? o + step : o;
+			}
+			const uint32_t vo = __shfl(v, (int)o, 64), eo = __shfl(excl, (int)o, 64), ro = __shfl(rc, (int)o, 64);
+			if (j < T) {
+				const uint32_t b = nth_bit(vo, j - eo); // the parent's bit in the owner's word
+				uint32_t cv; // the owner's chunk of B[d]: its word b / 4 holds the parent's byte
+				const uint32_t before = chunk_before(B + offc + 8u * (w0 + o), b >> 2u, cv);
+				const uint32_t sh = 8u * (b & 3u);
+				const uint32_t r = ro + before + (uint32_t)__popc(cv & ((1u << sh) - 1u));
+				store_parent_block(g.words, blk0 + j, (cv >> sh) & 0xffu, fbd, r);
+			}
+		}
+	};
+	// word i of segment k
+	auto lane_word = [&](uint32_t k, uint64_t i) {
 		const uint32_t d = 2u + k / S;
 		const BuildSeg &g = segs[k % S];
 		const uint64_t w = i - pw[k];
@@ -643,7 +627,7 @@ __global__ void __launch_bounds__(kThreads)
 		uint32_t v;
 		const uint32_t rp = bits_before(B, R, offp + w, v);
 		if (v == 0u)
-			continue;
+			return;
 		const uint32_t fbd = g.fb[d];
 		uint64_t block = (uint64_t)g.fb[d - 1u] + (rp - R[offp >> 3]); // first parent's block
 		// the 32 parents' children bytes are the 8-word chunk offc + 8w; parents not in v have zero
@@ -666,6 +650,50 @@ __global__ void __launch_bounds__(kThreads)
 			store_parent_block(g.words, block, byte, fbd, r);
 			r += (uint32_t)__popc(byte);
 			++block;
+		}
+	};
+	// A wave takes 256 words at a time, four loads in flight, where the grid has that many for every wave:
+	// most words of a large batch or level are empty, and their waves only wait for the load (32 mixed
+	// scenes 296 -> 131 us, slivers at 2^12 758 -> 729).  Else 64, which spreads the occupied words (room at
+	// 2^10 34 us, 82 with 256).
+	constexpr uint32_t kV = 4;
+	const uint32_t per = n >= kV * stride ? kV : 1u;
+	uint32_t hint = 0;
+	for (uint64_t base = (uint64_t)blockIdx.x * kThreads * per; base < n; base += stride * per) {
+		const uint64_t i0 = base + (uint64_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * 64u * per;
+		if (i0 >= n)
+			continue; // wave-uniform
+		uint32_t k0 = 0u;
+		with_seg<kThreads * kV>(pw, M, hint, base, i0, [&](uint32_t t) { k0 = t; });
+		k0 = __builtin_amdgcn_readfirstlane(k0);
+		if (i0 + 64u * per <= pw[k0 + 1u]) {
+			const uint64_t w0 = i0 - pw[k0];
+			const uint32_t *words = B + segs[k0 % S].bm + segs[k0 % S].off[1u + k0 / S] + w0 + lane;
+			uint32_t v[kV] = {words[0], 0u, 0u, 0u};
+			if (per == kV) {
+#pragma unroll
+				for (uint32_t q = 1; q < kV; ++q)
+					v[q] = words[64u * q];
+			}
+#pragma unroll 1
+			for (uint32_t q = 0; q < per; ++q)
+				wave_words(k0, w0 + 64u * q, q == 0u ? v[0] : q == 1u ? v[1] : q == 2u ? v[2] : v[3]);
+			continue;
+		}
+#pragma unroll 1
+		for (uint32_t q = 0; q < per; ++q) { // a segment ends here
+			const uint64_t i = i0 + 64u * q + lane;
+			const uint32_t k = i < n ? seg_walk(pw, M, hint, i) : kEmpty;
+			const uint32_t first = __builtin_amdgcn_readfirstlane(k);
+			if (first == kEmpty)
+				break; // the wave is past the end (lane 0 holds its first item)
+			if (__all(k == first || k == kEmpty)) {
+				const uint64_t w0 = (i - lane) - pw[first];
+				const BuildSeg &g = segs[first % S];
+				wave_words(first, w0, k != kEmpty ? B[g.bm + g.off[1u + first / S] + w0 + lane] : 0u);
+			} else if (k != kEmpty) {
+				lane_word(k, i);
+			}
 		}
 	}
 }
