@@ -746,14 +746,12 @@ def bench_primary(args, cfg, cpu=True):
         "march_beam": 4 * nfetch_beam + bw * bh * 4,
         "vox_fill": 40 * T + 4 * T + 8 * F,
         "vox_count": 40 * T + 4 * T,
-        # occupancy marks: every fragment read once
-        "bm_mark": 8 * F,
-        # leaf-block index of every fragment: fragment read, 4-byte bin written
-        "build_tag_leaf": 12 * F,
-        # bin index and fragment read, fragment written into its bin's bucket
-        "build_scatter": 20 * F,
-        # the canonical colour fold: every bucketed fragment read once (leaf blocks written: not counted)
-        "build_fold": 8 * F,
+        # tiles grouped by leaf block: every fragment read once, its 4-byte key written
+        "bm_group": 12 * F,
+        # every key read and written into its bin's bucket
+        "scatter_runs": 8 * F,
+        # the canonical colour fold: every bucketed key read once (leaf blocks written: not counted)
+        "build_fold": 4 * F,
     }
     nb = None
     if cfg["bounce"]:

@@ -911,7 +911,7 @@ __device__ void fold_raw(const uint32_t *b, const uint2 *frags, uint32_t n, uint
 // threads first orders its 256 leaf blocks by size class in LDS, so that most waves run a single
 // network; the next 256 sizes and bucket positions are loaded a step ahead.  Bound by the latency of its
 // loads (7 waves per SIMD): 7.2M leaf blocks of a room at 2^10 279 -> 133 us, 62M with slivers at 2^12
-// 1578 -> 825 us, against whole fragments, 64-bit comparators, leaf words in registers and integer
+// 1578 -> 893 us, against whole fragments, 64-bit comparators, leaf words in registers and integer
 // division.  Staging the buckets in LDS instead of each thread reading its own: 192 and 1211 us.
 template <uint32_t kN> __device__ __forceinline__ void fold_small(const uint32_t *b, uint32_t n, uint32_t *w) {
 	uint32_t k[kN];

@@ -1247,7 +1247,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) pa
 		atomicOr(err_out, err);
 }
 
-// The same paths on a persistent grid (march_persist's refill scheme): a lane whose path ends writes
+// The same paths on a persistent grid, with refills as in march_pool: a lane whose path ends writes
 // its pixel and takes the next pixel of its wave's pool; a path that goes on starts its next ray
 // in place.  Pixels are numbered in 8x8 tiles and dealt to the waves in 64-pixel chunks.
 template <uint32_t kT>
