@@ -1210,8 +1210,11 @@ __device__ void fold_mid_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__r
 	uint64_t count = list[0];
 	if (count > cap)
 		count = cap;
-	for (uint64_t base = 8u * ((uint64_t)blk * kWaves + wave); base < count; base += 8u * (uint64_t)nblk * kWaves) {
-		const uint32_t m = (uint32_t)(count - base < 8u ? count - base : 8u), mine = lane >> 3;
+	// up to 8 per wave; fewer where the list is short, so that more waves share it
+	const uint64_t waves = (uint64_t)nblk * kWaves, share = (count + waves - 1u) / waves;
+	const uint32_t take = share >= 8u ? 8u : share > 2u ? (uint32_t)(share + 1u) & ~1u : 2u;
+	for (uint64_t base = take * ((uint64_t)blk * kWaves + wave); base < count; base += take * waves) {
+		const uint32_t m = (uint32_t)(count - base < take ? count - base : take), mine = lane >> 3;
 		const uint32_t j = list[3u + base + (mine < m ? mine : 0u)]; // of leaf block lane / 8
 		if (mine < m && (lane & 7u) == 0u) {
 			n[mine] = cnt[j];
@@ -1566,7 +1569,7 @@ int node_phase(svo_ctx *ctx, BuildBatch &bb, bool maybe_raw) {
 	// blocks (17, 65 and 513 fragments at least), a wave or a block each
 	constexpr uint64_t kWaves = kThreads / 64u;
 	const uint32_t cu = (uint32_t)ctx->cu_count;
-	const uint32_t g_mid = (uint32_t)std::min<uint64_t>(cu * 8u, bb.Ftot / (17u * 8u * kWaves) + 1u),
+	const uint32_t g_mid = (uint32_t)std::min<uint64_t>(cu * 8u, bb.Ftot / (17u * 2u * kWaves) + 1u),
 	               g_wide = (uint32_t)std::min<uint64_t>(cu * 8u, bb.Ftot / (65u * kWaves) + 1u),
 	               g_big = (uint32_t)std::min<uint64_t>(cu * 2u, bb.Ftot / 513u + 1u);
 	if ((e = launch(ctx, "build_fold_lists", build_fold_lists, dim3(g_mid + g_wide + g_big), dim3(kThreads), 0, segs,
