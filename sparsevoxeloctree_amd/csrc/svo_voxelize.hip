@@ -216,10 +216,11 @@ __device__ __forceinline__ double reciprocal(double a) {
 // integer in the low word.  C is exact in 64 bits (|x|, |y| < 2^30).  Where the bound lies within the
 // pixel grid, |M| < 2^45 is exact in double; what is rounded stays 1/(2 |A|) away from a tie, more than
 // the 2^-51 |M / |A|| by which the reciprocal can err, so the result is exact.  Further out it only has
-// to stay there: a line moves |B / A| pixels a row, so where the width times the height of the triangle
-// is below 2^29 bounds fit the word (`near`); else they are clamped.  A = 0 bounds the rows only, by
-// nothing that the snapped bounding box does not.  A triangle that is a segment or a point after
-// snapping gets its line's both sides.
+// to stay there: a line moves |B / A| pixels a row, at most the width in 1/256 pixels, and a side of a
+// row lies less than the height + 1 rows from the vertices.  So where the width times the height (its
+// whole rows + 2) is below 2^29 bounds fit the word (`near`); else they are clamped.  A = 0 bounds the
+// rows only, by nothing that the snapped bounding box does not.  A triangle that is a segment or a
+// point after snapping gets its line's both sides.
 // Doubles rather than 32- or 64-bit integers: v_fma_f64 runs at the rate of an integer add here.
 struct RowPlanes {
 	double iv[3], b[3], d[3];
@@ -279,7 +280,7 @@ struct RowPlanes {
 		}
 		ilo = mir ? -i1 : i0;
 		ihi = mir ? -i0 : i1;
-		near = (float)(xmx - xmn) * (float)((ymx - ymn) >> 8) < 536870912.0f;
+		near = (float)(xmx - xmn) * (float)(((ymx - ymn) >> 8) + 2) < 536870912.0f;
 #pragma unroll
 		for (int k = 0; k < 3; ++k) {
 			const int32_t A = y[(k + 1) % 3] - y[k], B = x[k] - x[(k + 1) % 3];

@@ -73,6 +73,25 @@ def test_far_vertices(ctx, no_device_errors, far):
     check(ctx, tri, 8, "far %g" % far)
 
 
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("level,height", [(8, 0.5), (8, 1.9), (8, 6.0), (12, 0.5), (12, 1.9)])
+def test_flat_and_far(ctx, no_device_errors, level, height, axis):
+    # triangles up to 2^23 pixels wide and a pixel or a few tall, across a row boundary: an edge moves
+    # 2^31 pixels and more from one row to the next
+    rng = np.random.default_rng([level, int(10 * height), axis])
+    T, res = 400, 1 << level
+    far = 4194303.0 - rng.integers(0, 65536, (T, 2)) * rng.choice([0.0, 1.0, 32.0], (T, 1))
+    px = np.stack([-far[:, 0], far[:, 1], rng.uniform(-1, 1, T) * far[:, 1]], 1)
+    py = rng.integers(1, res, (T, 1)) - height * rng.random((T, 1)) + height * rng.random((T, 3))
+    py[::2, 1] = py[::2, 0] + 1 / 256  # an edge that rises by one step of the snapping grid
+    p = np.stack([px, py], 2) * 2.0 / res - 1.0
+    tri = np.concatenate([p, np.full((T, 3, 1), 0.1)], 2)[:, rng.permutation(3)]
+    if (level, axis) == (8, 2):
+        tri[0] = [(-32768.796875, 0.761749267578125, 0.1), (32766.6484375, 0.76177978515625, 0.1),
+                  (32724.5078125, 0.769500732421875, 0.1)]
+    check(ctx, np.roll(tri, axis - 2, 2), level, "flat and far %g" % height)
+
+
 @pytest.mark.parametrize("T", [777, 1 << 18])
 def test_fill_units(ctx, no_device_errors, T):
     # the fill's units of work: triangles of 100 to 1500 fragments (a whole wave of them, and scattered)
