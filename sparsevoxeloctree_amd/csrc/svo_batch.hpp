@@ -110,7 +110,7 @@ struct BuildSeg {
 	uint64_t nbins;      // leaf blocks = nodes of depth L-1 (the root when L = 1)
 	uint32_t L;
 	uint32_t overflow;   // W > 2^30
-	uint32_t raw;        // keys are fragment indices: a raw coordinate above 2^L (structure phase)
+	uint32_t raw;        // keys are fragment indices: a fragment fits no leaf_key (structure phase)
 	uint32_t pad;
 	uint64_t off[14];    // word offset of B[d] relative to bm, d = 1..L; off[L] = the scene's bitmap words
 	uint32_t fb[16];     // first block of every depth: fb[0] = 0 (root block), fb[1] = 1

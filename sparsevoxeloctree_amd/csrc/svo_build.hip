@@ -141,8 +141,9 @@ __global__ void __launch_bounds__(kThreads) bm_zero(uint32_t *B, uint64_t n, uin
 // coordinates only where the descent saturates (res and above meet res - 1): at most one step above
 // for a voxelized scene, so a flag per axis orders them as the packed words do (z's low byte, y, x;
 // the low byte of res is below that of res - 1 from 2^8 on).  A raw coordinate above res (a list from
-// the host, or a scene reaching out of the cube) does not fit: kRawKey, and its scene's keys become
-// fragment indices (BuildSeg::raw), compared by the fragments they name.
+// the host, or a scene reaching out of the cube) does not fit, and neither do bits 24..27 of the second
+// word, which the packing leaves unused but a list from the host may hold and the order counts: kRawKey,
+// and its scene's keys become fragment indices (BuildSeg::raw), compared by the fragments they name.
 constexpr uint32_t kRawKey = 0xFFFFFFFFu;
 
 // x, y, z: the effective coordinates (decode_frag).  A raw coordinate exceeds its effective one by 1 where
@@ -153,7 +154,7 @@ __device__ __forceinline__ uint32_t leaf_key(uint2 f, uint32_t res, uint32_t x, 
 	const uint32_t slot = (x & 1u) | (y & 1u) << 1u | (z & 1u) << 2u;
 	const uint32_t flags = dx | dy << 1u | (dz ^ (res >= 256u ? 1u : 0u)) << 2u;
 	const uint32_t key = slot << 27u | flags << 24u | (f.y & 0xffffffu);
-	return umax32(umax32(dx, dy), dz) > 1u ? kRawKey : key;
+	return umax32(umax32(dx, dy), dz) > 1u || (f.y & 0x0f000000u) != 0u ? kRawKey : key;
 }
 
 // ---- tiles and runs ------------------------------------------------------------------------------

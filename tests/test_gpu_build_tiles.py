@@ -71,6 +71,24 @@ def test_fold_sizes_and_saturated_coordinates(ctx, level, sizes, over):
     check(ctx, np.ascontiguousarray(fr[rng.permutation(len(fr))]), level)
 
 
+@pytest.mark.parametrize("level", [1, 4, 8, 12])
+@pytest.mark.parametrize("sizes", [(2, 4, 5, 8, 9, 16), (17, 32, 33, 64), (65, 512, 513), (2048, 2049, 3000)])
+@pytest.mark.parametrize("some", [1.0, 0.5, 0.01])
+def test_bits_outside_the_packing(ctx, level, sizes, some):
+    # host lists may have bits 24..27 of the second word set (on `some` of the fragments): no part of the
+    # colour, but of the order in which a leaf's fragments are folded
+    rng = np.random.default_rng([level, int(100 * some), *sizes])
+    p = np.concatenate([np.tile(2 * rng.integers(0, (1 << level) // 2, 3), (n, 1)) for n in sizes])
+    p = p + (rng.random(p.shape) < 0.3)
+    fr = pack_frags(p[:, 0], p[:, 1], p[:, 2], rng.integers(0, 1 << 24, len(p)))
+    plain = oracle.build(fr, level)
+    fr[:, 1] |= np.where(rng.random(len(p)) < some, rng.integers(0, 16, len(p)), 0).astype(np.uint32) << 24
+    if some > 0.1:
+        assert not np.array_equal(oracle.build(fr, level), plain)
+    print("bits", level, sizes, some, flush=True)
+    check(ctx, np.ascontiguousarray(fr[rng.permutation(len(fr))]), level)
+
+
 def test_batch_mixes_key_forms(ctx):
     import sparsevoxeloctree_amd as S
 
