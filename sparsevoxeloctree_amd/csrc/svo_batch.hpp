@@ -143,7 +143,7 @@ struct BuildBatch {
 	uint64_t *index = nullptr;
 	uint32_t *bm = nullptr, *rk = nullptr; // bitmaps (TW words), ranks of 8-word chunks (TW / 8 + 1)
 	uint32_t *cnt = nullptr, *aux = nullptr; // per leaf block (nbins)
-	uint32_t *raw = nullptr;    // per scene: raw flag of the structure phase (after rk)
+	uint32_t *raw = nullptr;    // per scene: raw flag of the structure phase, then one for all (after rk)
 	// per fragment tile (tiles = h_index[S]), in one allocation at runs: runs, heads, keys, run counts
 	uint64_t tiles = 0;
 	uint2 *runs = nullptr;

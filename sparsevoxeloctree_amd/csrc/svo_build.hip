@@ -122,7 +122,7 @@ __device__ __forceinline__ uint32_t bits_before(const uint32_t *__restrict__ B, 
 	return R[w >> 3] + chunk_before(B + (w & ~7ull), (uint32_t)(w & 7u), word);
 }
 
-// Clears the bitmaps and the scenes' raw flags, and writes the batch's tables when they fit a kernel
+// Clears the bitmaps and the raw flags (one per scene, then one for all), and writes the batch's tables when they fit a kernel
 // argument (words = 0: they are there already).
 __global__ void __launch_bounds__(kThreads) bm_zero(uint32_t *B, uint64_t n, uint32_t *raw, uint32_t S, uint32_t *dst,
                                                     uint32_t words, SmallTable t) {
@@ -132,7 +132,7 @@ __global__ void __launch_bounds__(kThreads) bm_zero(uint32_t *B, uint64_t n, uin
 	for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride)
 		B[i] = 0u;
 	if (blockIdx.x == 0u)
-		for (uint32_t s = threadIdx.x; s < S; s += kThreads)
+		for (uint32_t s = threadIdx.x; s <= S; s += kThreads)
 			raw[s] = 0u;
 }
 
@@ -198,20 +198,19 @@ __device__ __forceinline__ uint32_t group_slot(uint32_t line) {
 // atomics, at 8 waves per SIMD.  35M fragments in a room / 180M with slivers at 2^12 / 100M of 32 mixed
 // scenes: 192 / 1436 / 587 us, -> 180 / 1388 / 548 with packed sums, 32-bit Morton codes and scans by
 // data-parallel moves, -> 173 / 1351 / 493 with the group read before the compare-and-swap
-// (and see group_slot).  kIndex: a second pass that only rewrites the
-// keys (and their order) of the raw scenes' tiles as fragment indices.
+// (and see group_slot).  kIndex: a second pass (blocks of bm_write_blocks) that only rewrites the keys
+// (and their order) of the raw scenes' tiles as fragment indices.
 template <bool kIndex>
-__global__ void __launch_bounds__(kThreads)
-    bm_group(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ tbeg, uint32_t S, uint32_t *B,
-             uint32_t *__restrict__ keys, uint64_t *__restrict__ heads, uint2 *__restrict__ runs,
-             uint32_t *__restrict__ nrun, uint32_t *raw) {
+__device__ __forceinline__ void group_tile(const uint64_t tile, const BuildSeg *__restrict__ segs,
+                                           const uint64_t *__restrict__ tbeg, uint32_t S, uint32_t *B,
+                                           uint32_t *__restrict__ keys, uint64_t *__restrict__ heads,
+                                           uint2 *__restrict__ runs, uint32_t *__restrict__ nrun, uint32_t *raw) {
 	__shared__ uint32_t s_line[kLines], s_node[kLines]; // group key, Morton index of the group
 	__shared__ uint32_t s_n[kLines * kLineStride];      // per node 16 bits: fragments, then the first key
 	__shared__ uint32_t s_key[kTile];
 	__shared__ uint32_t s_head[kTile / 32u], s_before[kTile / 32u];
 	__shared__ uint32_t s_wave[kThreads / 64u], s_over;
-	const uint64_t tile = blockIdx.x;
-	if (tile >= tbeg[S])
+	if (tile >= tbeg[S] || (kIndex && raw[S] == 0u))
 		return;
 	const uint32_t sc = S == 1u ? 0u : seg_find(tbeg, S, tile);
 	const BuildSeg &g = segs[sc];
@@ -265,8 +264,13 @@ __global__ void __launch_bounds__(kThreads)
 		place[u] = at[u] != kEmpty ? atomicAdd(&s_n[h * kLineStride + (sub >> 1u)], 1u << sh) >> sh & 0xffffu
 		                           : atomicAdd(&s_over, 1u);
 	}
-	if (!kIndex && __any(wide) && (threadIdx.x & 63u) == 0u)
+	// only until the flag is seen: atomics on one address go one after another, and a wave in two may hold
+	// such a fragment (3M fragments at 2^10, one in 100 raw: both passes 184 -> 80 us)
+	if (!kIndex && __any(wide) && (threadIdx.x & 63u) == 0u &&
+	    __hip_atomic_load(&raw[sc], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) {
 		atomicOr(&raw[sc], 1u);
+		atomicOr(&raw[S], 1u);
+	}
 	__syncthreads();
 	// first keys of the groups' nodes (thread h owns group h), marking
 	uint32_t v[8], halves = 0u, mask = 0u;
@@ -357,6 +361,13 @@ __global__ void __launch_bounds__(kThreads)
 		}
 		runs[tile * kTile + r] = make_uint2((uint32_t)P, (uint32_t)(P >> 32) << 31u | p);
 	}
+}
+
+__global__ void __launch_bounds__(kThreads)
+    bm_group(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ tbeg, uint32_t S, uint32_t *B,
+             uint32_t *__restrict__ keys, uint64_t *__restrict__ heads, uint2 *__restrict__ runs,
+             uint32_t *__restrict__ nrun, uint32_t *raw) {
+	group_tile<false>(blockIdx.x, segs, tbeg, S, B, keys, heads, runs, nrun, raw);
 }
 
 // Bit q of B[d] = OR of byte q of B[d+1] (node q occupied iff one of its 8 children is); items are
@@ -561,14 +572,23 @@ __device__ __forceinline__ uint32_t nth_bit(uint32_t v, uint32_t n) {
 // are contiguous.  A wave across a segment boundary walks each word's set bits in its own lane.
 // Block 0 also writes the root block of every scene with L > 1 (its 8 words point to the depth-1
 // blocks of the occupied children, the bits of B[1]).  The same launch clears the nb leaf-block
-// counters of tag_runs and the three counts of the fold's work lists.
+// counters of tag_runs and the three counts of the fold's work lists.  All that by the first `grid`
+// blocks; with kGroup (a scene may be raw) the others group the raw scenes' tiles again, which depends
+// on nothing here: as a launch of its own that costs every plan replay 2 us.
+template <bool kGroup>
 __global__ void __launch_bounds__(kThreads)
     bm_write_blocks(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ pw, uint32_t M, uint32_t S,
                     const uint32_t *__restrict__ B, const uint32_t *__restrict__ R, uint32_t *cnt,
-                    const uint64_t *__restrict__ nbp, uint32_t *list) {
+                    const uint64_t *__restrict__ nbp, uint32_t *list, uint32_t grid, const uint64_t *__restrict__ tbeg,
+                    uint32_t scenes, uint32_t *__restrict__ keys, uint64_t *__restrict__ heads,
+                    uint2 *__restrict__ runs, uint32_t *__restrict__ nrun, uint32_t *raw) {
+	if (kGroup && blockIdx.x >= grid) {
+		group_tile<true>(blockIdx.x - grid, segs, tbeg, scenes, nullptr, keys, heads, runs, nrun, raw);
+		return;
+	}
 	const uint64_t n = pw[M], nb = *nbp;
 	const uint32_t lane = threadIdx.x & 63u;
-	const uint64_t stride = (uint64_t)gridDim.x * kThreads;
+	const uint64_t stride = (uint64_t)grid * kThreads;
 	for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < nb; i += stride)
 		cnt[i] = 0u;
 	if (blockIdx.x == 0u) {
@@ -845,8 +865,14 @@ __device__ __forceinline__ LeafTarget leaf_target(const BuildSeg &g, const uint6
 	return LeafTarget{g.words, (uint64_t)(L == 1u ? 0u : g.fb[L - 1u]) + (j - bbeg[s]), 1u << L, g.raw ? g.frags : nullptr};
 }
 
-__device__ __forceinline__ void cmp_swap32(uint32_t &x, uint32_t &y) {
+__device__ __forceinline__ void cmp_swap(uint32_t &x, uint32_t &y) {
 	const uint32_t lo = umin32(x, y), hi = umax32(x, y);
+	x = lo;
+	y = hi;
+}
+__device__ __forceinline__ void cmp_swap(uint64_t &x, uint64_t &y) {
+	const bool less = y < x;
+	const uint64_t lo = less ? y : x, hi = less ? x : y;
 	x = lo;
 	y = hi;
 }
@@ -865,6 +891,12 @@ struct LeafMean {
 		b = __builtin_floorf(__builtin_fmaf(__builtin_fmaf(b, n, (float)(rgb >> 16u & 0xffu)), inv, half));
 		n = __builtin_fminf(w, 63.0f);
 	}
+	__device__ __forceinline__ void load(uint32_t word) { // a leaf's word, or 0
+		r = (float)(word & 0xffu);
+		g = (float)(word >> 8u & 0xffu);
+		b = (float)(word >> 16u & 0xffu);
+		n = (float)(word >> 24u & 0x3fu);
+	}
 	__device__ __forceinline__ uint32_t word() const {
 		uint32_t v = __builtin_amdgcn_cvt_pk_u8_f32(r, 0u, 0u);
 		v = __builtin_amdgcn_cvt_pk_u8_f32(g, 1u, v);
@@ -873,81 +905,78 @@ struct LeafMean {
 	}
 };
 
-// A leaf block of a raw scene (keys = fragment indices): leaf by leaf, by repeated minimum over the
-// whole fragments (equal fragments are folded together).  w: the block's leaf words, one per child
-// slot, stride kThreads.
-__device__ void fold_raw(const uint32_t *b, const uint2 *frags, uint32_t n, uint32_t res, uint32_t *w) {
-#pragma unroll 1
-	for (uint32_t slot = 0; slot < 8u; ++slot) {
-		LeafMean leaf;
-		leaf.clear();
-		uint64_t last = 0;
-		bool any = false;
-		for (;;) {
-			uint64_t best = ~0ull;
-			uint32_t same = 0u;
-#pragma unroll 1
-			for (uint32_t i = 0; i < n; ++i) {
-				const uint64_t k = frag_key(frags[b[i]]);
-				if (key_slot(k, res) != slot || (any && k <= last) || k > best)
-					continue;
-				same = k == best ? same + 1u : 1u;
-				best = k;
-			}
-			if (!same)
-				break;
-			for (uint32_t i = 0; i < same; ++i)
-				leaf.add((uint32_t)best);
-			last = best;
-			any = true;
-		}
-		if (any)
-			w[slot * kThreads] = leaf.word();
+// Ascending sort of 4, 8 or 16 keys in registers (5, 19 or 63 comparators).
+template <uint32_t kN, class Key> __device__ __forceinline__ void sort_small(Key (&k)[kN]) {
+	if (kN == 4) {
+		cmp_swap(k[0], k[1]), cmp_swap(k[2], k[3]), cmp_swap(k[0], k[2]), cmp_swap(k[1], k[3]);
+		cmp_swap(k[1], k[2]);
+	} else if (kN == 8) {
+		cmp_swap(k[0], k[1]), cmp_swap(k[2], k[3]), cmp_swap(k[4], k[5]), cmp_swap(k[6], k[7]);
+		cmp_swap(k[0], k[2]), cmp_swap(k[1], k[3]), cmp_swap(k[4], k[6]), cmp_swap(k[5], k[7]);
+		cmp_swap(k[1], k[2]), cmp_swap(k[5], k[6]), cmp_swap(k[0], k[4]), cmp_swap(k[3], k[7]);
+		cmp_swap(k[1], k[5]), cmp_swap(k[2], k[6]);
+		cmp_swap(k[1], k[4]), cmp_swap(k[3], k[6]);
+		cmp_swap(k[2], k[4]), cmp_swap(k[3], k[5]);
+		cmp_swap(k[3], k[4]);
+	} else { // Batcher odd-even merge sort of 16
+		cmp_swap(k[0], k[1]), cmp_swap(k[2], k[3]), cmp_swap(k[0], k[2]), cmp_swap(k[1], k[3]);
+		cmp_swap(k[1], k[2]), cmp_swap(k[4], k[5]), cmp_swap(k[6], k[7]), cmp_swap(k[4], k[6]);
+		cmp_swap(k[5], k[7]), cmp_swap(k[5], k[6]), cmp_swap(k[0], k[4]), cmp_swap(k[2], k[6]);
+		cmp_swap(k[2], k[4]), cmp_swap(k[1], k[5]), cmp_swap(k[3], k[7]), cmp_swap(k[3], k[5]);
+		cmp_swap(k[1], k[2]), cmp_swap(k[3], k[4]), cmp_swap(k[5], k[6]), cmp_swap(k[8], k[9]);
+		cmp_swap(k[10], k[11]), cmp_swap(k[8], k[10]), cmp_swap(k[9], k[11]), cmp_swap(k[9], k[10]);
+		cmp_swap(k[12], k[13]), cmp_swap(k[14], k[15]), cmp_swap(k[12], k[14]), cmp_swap(k[13], k[15]);
+		cmp_swap(k[13], k[14]), cmp_swap(k[8], k[12]), cmp_swap(k[10], k[14]), cmp_swap(k[10], k[12]);
+		cmp_swap(k[9], k[13]), cmp_swap(k[11], k[15]), cmp_swap(k[11], k[13]), cmp_swap(k[9], k[10]);
+		cmp_swap(k[11], k[12]), cmp_swap(k[13], k[14]), cmp_swap(k[0], k[8]), cmp_swap(k[4], k[12]);
+		cmp_swap(k[4], k[8]), cmp_swap(k[2], k[10]), cmp_swap(k[6], k[14]), cmp_swap(k[6], k[10]);
+		cmp_swap(k[2], k[4]), cmp_swap(k[6], k[8]), cmp_swap(k[10], k[12]), cmp_swap(k[1], k[9]);
+		cmp_swap(k[5], k[13]), cmp_swap(k[5], k[9]), cmp_swap(k[3], k[11]), cmp_swap(k[7], k[15]);
+		cmp_swap(k[7], k[11]), cmp_swap(k[3], k[5]), cmp_swap(k[7], k[9]), cmp_swap(k[11], k[13]);
+		cmp_swap(k[1], k[2]), cmp_swap(k[3], k[4]), cmp_swap(k[5], k[6]), cmp_swap(k[7], k[8]);
+		cmp_swap(k[9], k[10]), cmp_swap(k[11], k[12]), cmp_swap(k[13], k[14]);
 	}
+}
+
+// A leaf block of a raw scene (keys = fragment indices): whole fragments sorted in registers, each folded
+// into its leaf's word in w (one word per child slot, stride kThreads, 0 before).  Takes more registers
+// than the keys do, so build_fold<true> is a launch of its own, made when a scene may be raw.  Bound
+// by the gather of the fragments: 157,700 triangles of a room reaching half out of the cube at 2^10
+// 1245 -> 165 us for both launches, 3M fragments at 2^10 458 -> 48 us, 100,000 at 2^6 260 -> 21 us, against
+// repeated minima over the bucket in the one kernel, which fetch every fragment again for each.
+template <uint32_t kN>
+__device__ __forceinline__ void fold_whole(const uint32_t *b, const uint2 *frags, uint32_t n, uint32_t res, uint32_t *w) {
+	uint64_t k[kN];
+#pragma unroll
+	for (uint32_t a = 0; a < kN; ++a)
+		k[a] = a < n ? frag_key(frags[b[a]]) : ~0ull;
+	sort_small<kN>(k);
+#pragma unroll
+	for (uint32_t a = 0; a < kN; ++a)
+		if (a < n) {
+			uint32_t *leaf = w + key_slot(k[a], res) * kThreads;
+			LeafMean mean;
+			mean.load(*leaf);
+			mean.add((uint32_t)k[a]);
+			*leaf = mean.word();
+		}
 }
 
 // One thread per leaf block with at most 16 fragments: leaf_keys sorted in registers (5-, 19- or
 // 63-comparator networks of v_min / v_max, +inf padding), then folded in that order, each leaf's word
 // going to the thread's LDS column; the whole block is written, empty leaves as 0.  Each block of
 // threads first orders its 256 leaf blocks by size class in LDS, so that most waves run a single
-// network; the next 256 sizes and bucket positions are loaded a step ahead.  Bound by the latency of its
-// loads (7 waves per SIMD): 7.2M leaf blocks of a room at 2^10 279 -> 133 us, 62M with slivers at 2^12
-// 1578 -> 893 us, against whole fragments, 64-bit comparators, leaf words in registers and integer
-// division.  Staging the buckets in LDS instead of each thread reading its own: 192 and 1211 us.
+// network; the next 256 sizes and bucket positions are loaded a step ahead.  kRaw: the blocks of raw
+// scenes (fold_whole), else all others and the lists.  Bound by the latency of its loads (7 waves per
+// SIMD): 7.2M leaf blocks of a room at 2^10 279 -> 133 us, 62M with slivers at 2^12 1578 -> 893 us, against
+// whole fragments, 64-bit comparators, leaf words in registers and integer division.  Staging the
+// buckets in LDS instead of each thread reading its own: 192 and 1211 us.
 template <uint32_t kN> __device__ __forceinline__ void fold_small(const uint32_t *b, uint32_t n, uint32_t *w) {
 	uint32_t k[kN];
 #pragma unroll
 	for (uint32_t a = 0; a < kN; ++a)
 		k[a] = a < n ? b[a] : kRawKey;
-	if (kN == 4) {
-		cmp_swap32(k[0], k[1]), cmp_swap32(k[2], k[3]), cmp_swap32(k[0], k[2]), cmp_swap32(k[1], k[3]);
-		cmp_swap32(k[1], k[2]);
-	} else if (kN == 8) {
-		cmp_swap32(k[0], k[1]), cmp_swap32(k[2], k[3]), cmp_swap32(k[4], k[5]), cmp_swap32(k[6], k[7]);
-		cmp_swap32(k[0], k[2]), cmp_swap32(k[1], k[3]), cmp_swap32(k[4], k[6]), cmp_swap32(k[5], k[7]);
-		cmp_swap32(k[1], k[2]), cmp_swap32(k[5], k[6]), cmp_swap32(k[0], k[4]), cmp_swap32(k[3], k[7]);
-		cmp_swap32(k[1], k[5]), cmp_swap32(k[2], k[6]);
-		cmp_swap32(k[1], k[4]), cmp_swap32(k[3], k[6]);
-		cmp_swap32(k[2], k[4]), cmp_swap32(k[3], k[5]);
-		cmp_swap32(k[3], k[4]);
-	} else { // Batcher odd-even merge sort of 16
-		cmp_swap32(k[0], k[1]), cmp_swap32(k[2], k[3]), cmp_swap32(k[0], k[2]), cmp_swap32(k[1], k[3]);
-		cmp_swap32(k[1], k[2]), cmp_swap32(k[4], k[5]), cmp_swap32(k[6], k[7]), cmp_swap32(k[4], k[6]);
-		cmp_swap32(k[5], k[7]), cmp_swap32(k[5], k[6]), cmp_swap32(k[0], k[4]), cmp_swap32(k[2], k[6]);
-		cmp_swap32(k[2], k[4]), cmp_swap32(k[1], k[5]), cmp_swap32(k[3], k[7]), cmp_swap32(k[3], k[5]);
-		cmp_swap32(k[1], k[2]), cmp_swap32(k[3], k[4]), cmp_swap32(k[5], k[6]), cmp_swap32(k[8], k[9]);
-		cmp_swap32(k[10], k[11]), cmp_swap32(k[8], k[10]), cmp_swap32(k[9], k[11]), cmp_swap32(k[9], k[10]);
-		cmp_swap32(k[12], k[13]), cmp_swap32(k[14], k[15]), cmp_swap32(k[12], k[14]), cmp_swap32(k[13], k[15]);
-		cmp_swap32(k[13], k[14]), cmp_swap32(k[8], k[12]), cmp_swap32(k[10], k[14]), cmp_swap32(k[10], k[12]);
-		cmp_swap32(k[9], k[13]), cmp_swap32(k[11], k[15]), cmp_swap32(k[11], k[13]), cmp_swap32(k[9], k[10]);
-		cmp_swap32(k[11], k[12]), cmp_swap32(k[13], k[14]), cmp_swap32(k[0], k[8]), cmp_swap32(k[4], k[12]);
-		cmp_swap32(k[4], k[8]), cmp_swap32(k[2], k[10]), cmp_swap32(k[6], k[14]), cmp_swap32(k[6], k[10]);
-		cmp_swap32(k[2], k[4]), cmp_swap32(k[6], k[8]), cmp_swap32(k[10], k[12]), cmp_swap32(k[1], k[9]);
-		cmp_swap32(k[5], k[13]), cmp_swap32(k[5], k[9]), cmp_swap32(k[3], k[11]), cmp_swap32(k[7], k[15]);
-		cmp_swap32(k[7], k[11]), cmp_swap32(k[3], k[5]), cmp_swap32(k[7], k[9]), cmp_swap32(k[11], k[13]);
-		cmp_swap32(k[1], k[2]), cmp_swap32(k[3], k[4]), cmp_swap32(k[5], k[6]), cmp_swap32(k[7], k[8]);
-		cmp_swap32(k[9], k[10]), cmp_swap32(k[11], k[12]), cmp_swap32(k[13], k[14]);
-	}
+	sort_small<kN>(k);
 	LeafMean leaf;
 	leaf.clear();
 	uint32_t slot = 8u;
@@ -963,10 +992,13 @@ template <uint32_t kN> __device__ __forceinline__ void fold_small(const uint32_t
 		}
 }
 
-__global__ void __launch_bounds__(kThreads)
+template <bool kRaw>
+__global__ void __launch_bounds__(kThreads, kRaw ? 5 : 7)
     build_fold(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ bbeg, uint32_t S,
                const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ aux, const uint32_t *__restrict__ bucket,
-               uint32_t *list, uint64_t cap) {
+               const uint32_t *__restrict__ raw, uint32_t *list, uint64_t cap) {
+	if (kRaw && raw[S] == 0u)
+		return;
 	const uint64_t nbins = bbeg[S];
 	constexpr uint32_t kWaves = kThreads / 64;
 	__shared__ uint32_t s_bin[kThreads], s_n[kThreads];
@@ -993,8 +1025,10 @@ __global__ void __launch_bounds__(kThreads)
 		if (jj < nbins) {
 			cls = n <= 4u ? 0u : n <= 8u ? 1u : n <= kRegBucket ? 2u : n <= kPairBucket ? 3u : n <= kWaveBucket ? 4u : 5u;
 		}
-		const bool rest = jj < nbins && cls == 5u;
-		push_bins(list, cap, (uint32_t)jj, rest && n <= kWideBucket, rest && n > kWideBucket);
+		if constexpr (!kRaw) {
+			const bool rest = jj < nbins && cls == 5u;
+			push_bins(list, cap, (uint32_t)jj, rest && n <= kWideBucket, rest && n > kWideBucket);
+		}
 		uint64_t mine = 0u; // the wave's lanes of the same class
 #pragma unroll
 		for (uint32_t c = 0; c < 5u; ++c) {
@@ -1015,7 +1049,7 @@ __global__ void __launch_bounds__(kThreads)
 			}
 		pos += (uint32_t)__popcll(mine & below);
 		uint32_t first = 0u; // of the step's places in the mid list; used after the fold
-		if (threadIdx.x == 0u && mids)
+		if (!kRaw && threadIdx.x == 0u && mids)
 			first = atomicAdd(&list[0], mids);
 		if (cls < 3u) {
 			s_bin[pos] = (uint32_t)jj;
@@ -1027,29 +1061,29 @@ __global__ void __launch_bounds__(kThreads)
 			const uint32_t j = s_bin[threadIdx.x], nj = s_n[threadIdx.x];
 			LeafTarget t;
 			with_seg<kThreads>(bbeg, S, hint, base, j, [&](uint32_t s) { t = leaf_target(segs[s], bbeg, s, j); });
-			uint32_t *w = s_leaf + threadIdx.x;
+			if ((t.raw != nullptr) == kRaw) {
+				uint32_t *w = s_leaf + threadIdx.x;
 #pragma unroll
-			for (uint32_t c = 0; c < 8u; ++c)
-				w[c * kThreads] = 0u;
-			const uint32_t at = s_at[threadIdx.x];
-			if (t.raw)
-				fold_raw(bucket + at, t.raw, nj, t.res, w);
-			else if (nj <= 4u)
-				fold_small<4>(bucket + at, nj, w);
-			else if (nj <= 8u)
-				fold_small<8>(bucket + at, nj, w);
-			else
-				fold_small<16>(bucket + at, nj, w);
-			uint32_t words[8];
+				for (uint32_t c = 0; c < 8u; ++c)
+					w[c * kThreads] = 0u;
+				const uint32_t *b = bucket + s_at[threadIdx.x];
+				if (nj <= 4u)
+					kRaw ? fold_whole<4>(b, t.raw, nj, t.res, w) : fold_small<4>(b, nj, w);
+				else if (nj <= 8u)
+					kRaw ? fold_whole<8>(b, t.raw, nj, t.res, w) : fold_small<8>(b, nj, w);
+				else
+					kRaw ? fold_whole<16>(b, t.raw, nj, t.res, w) : fold_small<16>(b, nj, w);
+				uint32_t words[8];
 #pragma unroll
-			for (uint32_t c = 0; c < 8u; ++c)
-				words[c] = w[c * kThreads];
-			store_block(t.oct, t.block, words);
+				for (uint32_t c = 0; c < 8u; ++c)
+					words[c] = w[c * kThreads];
+				store_block(t.oct, t.block, words);
+			}
 		}
 		if (threadIdx.x == 0u)
 			s_mid = first;
 		__syncthreads();
-		if ((cls == 3u || cls == 4u) && s_mid + pos - total < cap)
+		if (!kRaw && (cls == 3u || cls == 4u) && s_mid + pos - total < cap)
 			list[3u + s_mid + pos - total] = (uint32_t)jj;
 	}
 }
@@ -1337,13 +1371,14 @@ __device__ void fold_wide_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__
 }
 
 // Leaf blocks of more than 512 fragments, one block each.  Up to kLdsBucket fragments: sorted in LDS.
-// Beyond (rare): the keys are sorted in place in the bucket and each of the 8 lanes walks all of them,
-// taking those of its slot.  Blocks blk of nblk of the list launch; s_keys / s_slots: kLdsBucket
-// entries for the block.
+// Beyond (rare): the keys are sorted in place in the bucket (a raw scene's whole fragments in spare,
+// 8 bytes per bucket entry) and each of the 8 lanes walks all of them, taking those of its slot.  Blocks
+// blk of nblk of the list launch; s_keys / s_slots: kLdsBucket entries for the block.
 __device__ void fold_big_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__restrict__ segs,
                                 const uint64_t *__restrict__ bbeg, uint32_t S, const uint32_t *__restrict__ cnt,
-                                const uint32_t *__restrict__ aux, uint32_t *bucket, const uint32_t *list, uint64_t cap,
-                                uint64_t *s_keys, uint8_t *s_slots, uint32_t *s_beg, uint32_t *s_end) {
+                                const uint32_t *__restrict__ aux, uint32_t *bucket, uint64_t *spare,
+                                const uint32_t *list, uint64_t cap, uint64_t *s_keys, uint8_t *s_slots,
+                                uint32_t *s_beg, uint32_t *s_end) {
 	uint64_t count = list[1];
 	if (count > cap)
 		count = cap;
@@ -1359,21 +1394,31 @@ __device__ void fold_big_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__r
 			uint32_t m = 1;
 			while (m < n)
 				m <<= 1;
-			// order of an entry: the whole fragment of a raw scene's index, else the key itself
-			auto order = [&](uint32_t e) { return t.raw ? frag_key(t.raw[e]) : (uint64_t)e; };
-			lds_bitonic<kThreads>(
-			    n, m, threadIdx.x, [&](uint32_t x, uint32_t y) { return order(b[x]) < order(b[y]); },
-			    [&](uint32_t x, uint32_t y) {
-				    const uint32_t e = b[x];
-				    b[x] = b[y], b[y] = e;
-			    },
-			    [] { __syncthreads(); });
+			uint64_t *whole = spare + aux[j]; // a raw scene's
+			if (t.raw) {
+				for (uint32_t i = threadIdx.x; i < n; i += kThreads)
+					whole[i] = frag_key(t.raw[b[i]]);
+				__syncthreads();
+			}
+			auto sort = [&](auto *k) {
+				lds_bitonic<kThreads>(
+				    n, m, threadIdx.x, [&](uint32_t x, uint32_t y) { return k[x] < k[y]; },
+				    [&](uint32_t x, uint32_t y) {
+					    const auto e = k[x];
+					    k[x] = k[y], k[y] = e;
+				    },
+				    [] { __syncthreads(); });
+			};
+			if (t.raw)
+				sort(whole);
+			else
+				sort(b);
 			if (threadIdx.x < 8u) {
 				LeafMean leaf;
 				leaf.clear();
 				bool any = false;
 				for (uint32_t i = 0; i < n; ++i) {
-					const uint64_t key = order(b[i]);
+					const uint64_t key = t.raw ? whole[i] : (uint64_t)b[i];
 					const uint32_t slot = t.raw ? key_slot(key, t.res) : (uint32_t)key >> 27u;
 					if (slot == threadIdx.x) {
 						leaf.add((uint32_t)key);
@@ -1393,7 +1438,7 @@ __device__ void fold_big_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__r
 __global__ void __launch_bounds__(kThreads)
     build_fold_lists(const BuildSeg *__restrict__ segs, const uint64_t *__restrict__ bbeg, uint32_t S,
                      const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ aux, uint32_t *bucket,
-                     const uint32_t *list, uint64_t cap, uint32_t g_mid, uint32_t g_wide) {
+                     uint64_t *spare, const uint32_t *list, uint64_t cap, uint32_t g_mid, uint32_t g_wide) {
 	constexpr uint32_t kWaves = kThreads / 64;
 	static_assert(kWaves * kWideBucket == kLdsBucket, "the wide and big roles share the key arrays");
 	__shared__ uint64_t s_keys[kLdsBucket];
@@ -1406,8 +1451,8 @@ __global__ void __launch_bounds__(kThreads)
 		fold_wide_blocks(blockIdx.x - g_mid, g_wide, segs, bbeg, S, cnt, aux, bucket, list, cap, s_keys, s_slots, s_beg,
 		                 s_end);
 	else
-		fold_big_blocks(blockIdx.x - g_mid - g_wide, gridDim.x - g_mid - g_wide, segs, bbeg, S, cnt, aux, bucket, list,
-		                cap, s_keys, s_slots, s_beg[0], s_end[0]);
+		fold_big_blocks(blockIdx.x - g_mid - g_wide, gridDim.x - g_mid - g_wide, segs, bbeg, S, cnt, aux, bucket,
+		                spare, list, cap, s_keys, s_slots, s_beg[0], s_end[0]);
 }
 
 // ---- scan plumbing for the bin offsets ---------------------------------------------------------
@@ -1450,12 +1495,6 @@ void levels_for(uint32_t L, uint64_t *off) {
 
 uint64_t big_capacity(uint64_t F) { return F / (kRegBucket + 1u) + 1u; }
 
-// Grouping of the fragment tiles; index: the pass that rewrites the raw scenes' keys as fragment indices.
-hipError_t group_tiles(svo_ctx *ctx, const BuildBatch &bb, bool index) {
-	return launch(ctx, "bm_group", index ? bm_group<true> : bm_group<false>, dim3((uint32_t)bb.tiles), dim3(kThreads), 0,
-	              (const BuildSeg *)bb.segs, bb.tbeg(), bb.S, bb.bm, bb.keys, bb.heads, bb.runs, bb.nrun, bb.raw);
-}
-
 // tiles: whole tiles of F fragments; the tile arrays of `tiles` tiles, one allocation.
 uint64_t tiles_of(uint64_t F) { return (F + kTile - 1u) / kTile; }
 hipError_t alloc_tiles(Pool *pool, BuildBatch &bb) {
@@ -1483,7 +1522,9 @@ int structure_phase(svo_ctx *ctx, BuildBatch &bb, const std::vector<uint8_t> *ta
 	                reinterpret_cast<uint32_t *>(bb.segs), small ? (uint32_t)(bytes / 4u) : 0u,
 	                small ? SmallTable(tables->data(), bytes) : SmallTable())) != hipSuccess)
 		return hip_check(ctx, e, "bm_zero");
-	if (bb.tiles > 0 && (e = group_tiles(ctx, bb, false)) != hipSuccess)
+	if (bb.tiles > 0 && (e = launch(ctx, "bm_group", bm_group, dim3((uint32_t)bb.tiles), dim3(kThreads), 0,
+	                                (const BuildSeg *)bb.segs, bb.tbeg(), S, bb.bm, bb.keys, bb.heads, bb.runs,
+	                                bb.nrun, bb.raw)) != hipSuccess)
 		return hip_check(ctx, e, "bm_group");
 	const Levels levels{bb.segs, S, bb.rk, bb.raw, 1ull << 30, out};
 	if (bb.TW > 0) {
@@ -1524,7 +1565,8 @@ int structure_phase(svo_ctx *ctx, BuildBatch &bb, const std::vector<uint8_t> *ta
 	return SVO_OK;
 }
 
-// maybe_raw: a scene may be raw (a plan's replay cannot know).
+// maybe_raw: a scene may be raw (a plan's replay cannot know): its tiles are grouped again, its leaf blocks
+// folded by a launch of their own.
 int node_phase(svo_ctx *ctx, BuildBatch &bb, bool maybe_raw) {
 	const uint32_t S = bb.S;
 	const BuildSeg *segs = bb.segs;
@@ -1533,13 +1575,14 @@ int node_phase(svo_ctx *ctx, BuildBatch &bb, bool maybe_raw) {
 		// with maxL == 1 there are no parent words and no root blocks to write (the bitmaps are empty)
 		const uint32_t M = bb.pw_segs();
 		const uint64_t n = bb.maxL > 1u ? bb.h_index[bb.pw_at() + M] : 0u; // parent words of all depths >= 2
-		if ((e = launch(ctx, "bm_write_blocks", bm_write_blocks, dim3(grid_for(std::max(n, bb.nbins), ctx)),
-		                dim3(kThreads), 0, segs, bb.pw(), M, bb.maxL > 1u ? S : 0u, (const uint32_t *)bb.bm,
-		                (const uint32_t *)bb.rk, bb.cnt, bb.bbeg() + S, bb.list)) != hipSuccess)
+		const uint32_t grid = grid_for(std::max(n, bb.nbins), ctx);
+		if ((e = launch(ctx, "bm_write_blocks", maybe_raw ? bm_write_blocks<true> : bm_write_blocks<false>,
+		                dim3(grid + (maybe_raw ? (uint32_t)bb.tiles : 0u)), dim3(kThreads), 0, segs, bb.pw(), M,
+		                bb.maxL > 1u ? S : 0u, (const uint32_t *)bb.bm, (const uint32_t *)bb.rk, bb.cnt,
+		                bb.bbeg() + S, bb.list, grid, bb.tbeg(), S, bb.keys, bb.heads, bb.runs, bb.nrun,
+		                bb.raw)) != hipSuccess)
 			return hip_check(ctx, e, "bm_write_blocks");
 	}
-	if (maybe_raw && bb.tiles > 0 && (e = group_tiles(ctx, bb, true)) != hipSuccess)
-		return hip_check(ctx, e, "bm_group");
 	const uint32_t gT = div_up(bb.tiles, kThreads / 64u);
 	if (bb.tiles > 0 && (e = launch(ctx, "tag_runs", tag_runs, dim3(gT), dim3(kThreads), 0, segs, bb.tbeg(), S,
 	                                (const uint32_t *)bb.bm, (const uint32_t *)bb.rk, bb.runs,
@@ -1562,10 +1605,11 @@ int node_phase(svo_ctx *ctx, BuildBatch &bb, bool maybe_raw) {
 	                                (const uint32_t *)bb.nrun, (const uint32_t *)bb.aux, bb.bucket)) != hipSuccess)
 		return hip_check(ctx, e, "scatter_runs");
 	const uint64_t cap = big_capacity(bb.Ftot);
-	if ((e = launch(ctx, "build_fold", build_fold, dim3(grid_for(bb.nbins, ctx)), dim3(kThreads), 0, segs, bb.bbeg(),
-	                S, (const uint32_t *)bb.cnt, (const uint32_t *)bb.aux, (const uint32_t *)bb.bucket, bb.list, cap)) !=
-	    hipSuccess)
-		return hip_check(ctx, e, "build_fold");
+	for (int raw = 0; raw <= (maybe_raw ? 1 : 0); ++raw)
+		if ((e = launch(ctx, "build_fold", raw ? build_fold<true> : build_fold<false>, dim3(grid_for(bb.nbins, ctx)),
+		                dim3(kThreads), 0, segs, bb.bbeg(), S, (const uint32_t *)bb.cnt, (const uint32_t *)bb.aux,
+		                (const uint32_t *)bb.bucket, (const uint32_t *)bb.raw, bb.list, cap)) != hipSuccess)
+			return hip_check(ctx, e, "build_fold");
 	// the roles' loops take any number of blocks: no more than the fragments can fill with listed leaf
 	// blocks (17, 65 and 513 fragments at least), a wave or a block each
 	constexpr uint64_t kWaves = kThreads / 64u;
@@ -1574,8 +1618,8 @@ int node_phase(svo_ctx *ctx, BuildBatch &bb, bool maybe_raw) {
 	               g_wide = (uint32_t)std::min<uint64_t>(cu * 8u, bb.Ftot / (65u * kWaves) + 1u),
 	               g_big = (uint32_t)std::min<uint64_t>(cu * 2u, bb.Ftot / 513u + 1u);
 	if ((e = launch(ctx, "build_fold_lists", build_fold_lists, dim3(g_mid + g_wide + g_big), dim3(kThreads), 0, segs,
-	                bb.bbeg(), S, (const uint32_t *)bb.cnt, (const uint32_t *)bb.aux, bb.bucket, (const uint32_t *)bb.list,
-	                cap, g_mid, g_wide)) != hipSuccess)
+	                bb.bbeg(), S, (const uint32_t *)bb.cnt, (const uint32_t *)bb.aux, bb.bucket,
+	                reinterpret_cast<uint64_t *>(bb.runs), (const uint32_t *)bb.list, cap, g_mid, g_wide)) != hipSuccess)
 		return hip_check(ctx, e, "build_fold_lists");
 	return SVO_OK;
 }
@@ -1698,7 +1742,7 @@ int build_batch(svo_ctx *ctx, svo_octree *const *octs, uint32_t S) {
 	const size_t seg_bytes = seg_table_bytes(S), idx_bytes = sizeof(uint64_t) * bb.h_index.size();
 	if (pool->alloc((void **)&bb.segs, seg_bytes + idx_bytes) != hipSuccess ||
 	    pool->alloc((void **)&bb.bm, sizeof(uint32_t) * (bb.TW ? bb.TW : 1)) != hipSuccess ||
-	    pool->alloc((void **)&bb.rk, sizeof(uint32_t) * (bb.TW / 8u + 1 + S)) != hipSuccess ||
+	    pool->alloc((void **)&bb.rk, sizeof(uint32_t) * (bb.TW / 8u + 2 + S)) != hipSuccess ||
 	    alloc_tiles(pool, bb) != hipSuccess || pool->alloc((void **)&bb.bucket, sizeof(uint32_t) * Fa) != hipSuccess ||
 	    pool->alloc((void **)&bb.list, sizeof(uint32_t) * (3 + 3 * cap)) != hipSuccess)
 		rc = set_error(ctx, SVO_ERR_OUT_OF_MEMORY, "octree build allocation failed");
@@ -1923,7 +1967,7 @@ int build_plan_init(svo_ctx *ctx, BuildPlan *p, const svo_scene *const *scenes, 
 	const size_t seg_bytes = seg_table_bytes(S), idx_bytes = sizeof(uint64_t) * bb.h_index.size();
 	if (pool->alloc((void **)&bb.segs, seg_bytes + idx_bytes) != hipSuccess ||
 	    pool->alloc((void **)&bb.bm, sizeof(uint32_t) * (bb.TW ? bb.TW : 1)) != hipSuccess ||
-	    pool->alloc((void **)&bb.rk, sizeof(uint32_t) * (bb.TW / 8u + 1 + S)) != hipSuccess ||
+	    pool->alloc((void **)&bb.rk, sizeof(uint32_t) * (bb.TW / 8u + 2 + S)) != hipSuccess ||
 	    alloc_tiles(pool, bb) != hipSuccess ||
 	    pool->alloc((void **)&bb.bucket, sizeof(uint32_t) * Fcap) != hipSuccess ||
 	    pool->alloc((void **)&bb.list, sizeof(uint32_t) * (3 + 3 * big_capacity(Fcap))) != hipSuccess ||
