@@ -1262,20 +1262,26 @@ __device__ void fold_mid_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__r
 	}
 }
 
-// Bitonic sort of n (<= m = 2^p) keys in LDS by kStep lanes (one wave, or the block); sync() separates
-// the stages.
-template <uint32_t kStep, class Less, class Swap, class Sync>
-__device__ __forceinline__ void lds_bitonic(uint32_t n, uint32_t m, uint32_t lane, Less less, Swap swap, Sync sync) {
+// Bitonic sort of n (<= m = 2^p) keys by kStep lanes (one wave, or the block); step(a, b) leaves the
+// smaller of keys a and b at a, sync() separates the stages.
+template <uint32_t kStep, class Step, class Sync>
+__device__ __forceinline__ void bitonic(uint32_t n, uint32_t m, uint32_t lane, Step step, Sync sync) {
 	for (uint32_t k = 2; k <= m; k <<= 1)
 		for (uint32_t jj = k >> 1; jj > 0; jj >>= 1) {
 			for (uint32_t q = lane; q < m / 2u; q += kStep) {
 				uint32_t a, b;
 				bitonic_pair(q, k, jj, a, b);
-				if (b < n && less(b, a))
-					swap(a, b);
+				if (b < n)
+					step(a, b);
 			}
 			sync();
 		}
+}
+
+template <class Key> __device__ __forceinline__ void order_keys(Key *keys, uint32_t x, uint32_t y) {
+	const Key kx = keys[x], ky = keys[y];
+	if (ky < kx)
+		keys[x] = ky, keys[y] = kx;
 }
 
 // Sorts the n keys of one leaf block in LDS and finds the runs of its 8 leaves: s_beg / s_end[slot].
@@ -1298,33 +1304,22 @@ __device__ __forceinline__ void sort_leaves(uint32_t n, uint32_t lane, const Lea
 			slots[i] = (uint8_t)key_slot(key, t.res);
 		}
 		sync();
-		lds_bitonic<kStep>(
+		bitonic<kStep>(
 		    n, m, lane,
-		    [&](uint32_t x, uint32_t y) { return slots[x] < slots[y] || (slots[x] == slots[y] && keys64[x] < keys64[y]); },
 		    [&](uint32_t x, uint32_t y) {
-			    const uint64_t kx = keys64[x];
-			    const uint8_t sx = slots[x];
-			    keys64[x] = keys64[y], keys64[y] = kx;
-			    slots[x] = slots[y], slots[y] = sx;
+			    const uint64_t kx = keys64[x], ky = keys64[y];
+			    const uint8_t sx = slots[x], sy = slots[y];
+			    if (sy < sx || (sy == sx && ky < kx)) {
+				    keys64[x] = ky, keys64[y] = kx;
+				    slots[x] = sy, slots[y] = sx;
+			    }
 		    },
 		    sync);
 	} else {
 		for (uint32_t i = lane; i < n; i += kStep)
 			keys32[i] = b[i];
 		sync();
-		for (uint32_t k = 2; k <= m; k <<= 1)
-			for (uint32_t jj = k >> 1; jj > 0; jj >>= 1) {
-				for (uint32_t q = lane; q < m / 2u; q += kStep) {
-					uint32_t x, y;
-					bitonic_pair(q, k, jj, x, y);
-					if (y < n) {
-						const uint32_t kx = keys32[x], ky = keys32[y];
-						if (ky < kx)
-							keys32[x] = ky, keys32[y] = kx;
-					}
-				}
-				sync();
-			}
+		bitonic<kStep>(n, m, lane, [&](uint32_t x, uint32_t y) { order_keys(keys32, x, y); }, sync);
 	}
 	auto slot_of = [&](uint32_t i) { return t.raw ? (uint32_t)slots[i] : keys32[i] >> 27u; };
 	for (uint32_t i = lane; i < n; i += kStep) {
@@ -1371,9 +1366,10 @@ __device__ void fold_wide_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__
 }
 
 // Leaf blocks of more than 512 fragments, one block each.  Up to kLdsBucket fragments: sorted in LDS.
-// Beyond (rare): the keys are sorted in place in the bucket (a raw scene's whole fragments in spare,
-// 8 bytes per bucket entry) and each of the 8 lanes walks all of them, taking those of its slot.  Blocks
-// blk of nblk of the list launch; s_keys / s_slots: kLdsBucket entries for the block.
+// Beyond (rare): the keys are sorted in place in the bucket and each of 8 lanes folds its slot's run;
+// a raw scene's whole fragments are sorted in spare (8 bytes per bucket entry), and each lane walks all
+// of them, taking those of its slot.  Blocks blk of nblk of the list launch; s_keys / s_slots:
+// kLdsBucket entries for the block.
 __device__ void fold_big_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__restrict__ segs,
                                 const uint64_t *__restrict__ bbeg, uint32_t S, const uint32_t *__restrict__ cnt,
                                 const uint32_t *__restrict__ aux, uint32_t *bucket, uint64_t *spare,
@@ -1400,27 +1396,31 @@ __device__ void fold_big_blocks(uint32_t blk, uint32_t nblk, const BuildSeg *__r
 					whole[i] = frag_key(t.raw[b[i]]);
 				__syncthreads();
 			}
-			auto sort = [&](auto *k) {
-				lds_bitonic<kThreads>(
-				    n, m, threadIdx.x, [&](uint32_t x, uint32_t y) { return k[x] < k[y]; },
-				    [&](uint32_t x, uint32_t y) {
-					    const auto e = k[x];
-					    k[x] = k[y], k[y] = e;
-				    },
-				    [] { __syncthreads(); });
-			};
 			if (t.raw)
-				sort(whole);
+				bitonic<kThreads>(
+				    n, m, threadIdx.x, [&](uint32_t x, uint32_t y) { order_keys(whole, x, y); }, [] { __syncthreads(); });
 			else
-				sort(b);
-			if (threadIdx.x < 8u) {
+				bitonic<kThreads>(
+				    n, m, threadIdx.x, [&](uint32_t x, uint32_t y) { order_keys(b, x, y); }, [] { __syncthreads(); });
+			if (threadIdx.x < 8u && !t.raw) {
+				auto first = [&](uint32_t key) { // index of the first key not below
+					uint32_t lo = 0u, hi = n;
+					while (lo < hi) {
+						const uint32_t mid = lo + (hi - lo) / 2u;
+						lo = b[mid] < key ? mid + 1u : lo;
+						hi = b[mid] < key ? hi : mid;
+					}
+					return lo;
+				};
+				const uint32_t beg = first(threadIdx.x << 27u), end = first((threadIdx.x + 1u) << 27u);
+				t.oct[8u * t.block + threadIdx.x] = fold_run(beg, end, [&](uint32_t i) { return b[i]; });
+			} else if (threadIdx.x < 8u) {
 				LeafMean leaf;
 				leaf.clear();
 				bool any = false;
 				for (uint32_t i = 0; i < n; ++i) {
-					const uint64_t key = t.raw ? whole[i] : (uint64_t)b[i];
-					const uint32_t slot = t.raw ? key_slot(key, t.res) : (uint32_t)key >> 27u;
-					if (slot == threadIdx.x) {
+					const uint64_t key = whole[i];
+					if (key_slot(key, t.res) == threadIdx.x) {
 						leaf.add((uint32_t)key);
 						any = true;
 					}
