@@ -403,22 +403,36 @@ __global__ void __launch_bounds__(kThreads)
 	if (!again)
 		return;
 	for (uint64_t base = first; base < T; base += stride) {
-		for (uint64_t t = base; t < T && t < base + per; ++t) {
+		// those that cannot cover a pixel are done here
+		bool covers = false;
+		if (lane < per && base + lane < T) {
+			const uint64_t t = base + lane;
 			const uint32_t sg = S == 1u ? 0u : seg_find(tbeg, S, t);
 			const uint32_t res = 1u << segs[sg].level;
 			TriBase tri;
 			tri_base(segs[sg].xyz, t - tbeg[sg], res, tri);
-			if (pixels_ok(tri) || tri.degenerate)
-				continue;
+			if (!pixels_ok(tri) && !tri.degenerate) {
+				Setup s;
+				tri_setup(tri, res, s);
+				covers = !s.empty;
+				if (s.empty)
+					counts[t] = 0u;
+			}
+		}
+		for (uint64_t m = __ballot(covers); m; m &= m - 1u) {
+			const uint64_t t = base + (uint32_t)__ffsll((unsigned long long)m) - 1u;
+			const uint32_t sg = S == 1u ? 0u : seg_find(tbeg, S, t);
+			const uint32_t res = 1u << segs[sg].level;
+			TriBase tri;
+			tri_base(segs[sg].xyz, t - tbeg[sg], res, tri);
 			Setup s;
 			tri_setup(tri, res, s);
 			uint32_t c = 0;
-			if (!s.empty)
-				for (int32_t j = s.jlo + (int32_t)lane; j <= s.jhi; j += 64) {
-					int32_t i0, i1;
-					row_span(s, j, i0, i1);
-					c += (uint32_t)(i1 - i0 + 1);
-				}
+			for (int32_t j = s.jlo + (int32_t)lane; j <= s.jhi; j += 64) {
+				int32_t i0, i1;
+				row_span(s, j, i0, i1);
+				c += (uint32_t)(i1 - i0 + 1);
+			}
 			c = wave_sum(c);
 			if (lane == 0u) {
 				counts[t] = c;

@@ -73,6 +73,20 @@ def test_far_vertices(ctx, no_device_errors, far):
     check(ctx, tri, 8, "far %g" % far)
 
 
+@pytest.mark.parametrize("T", [63, 64, 65, 3000])
+@pytest.mark.parametrize("share", [0.02, 0.5, 1.0])
+def test_many_far_triangles(ctx, no_device_errors, T, share):
+    # `share` of the triangles in the 64-bit form: most of those cover no pixel, some cross the volume
+    rng = np.random.default_rng([T, int(100 * share)])
+    tri = rng.uniform(-1, 1, (T, 3, 3))
+    far = np.nonzero(rng.random(T) < share)[0]
+    tri[far] = rng.uniform(-1, 1, (len(far), 1, 3)) * 60000 + rng.normal(size=(len(far), 3, 3)) * 1000
+    cross = far[::7]
+    tri[cross] = np.stack([rng.uniform(-1, 1, (len(cross), 3)), rng.uniform(-60000, 60000, (len(cross), 3)),
+                           rng.uniform(-60000, 60000, (len(cross), 3))], 1)
+    check(ctx, tri, 7, "many far %g" % share)
+
+
 @pytest.mark.parametrize("axis", [0, 1, 2])
 @pytest.mark.parametrize("level,height", [(8, 0.5), (8, 1.9), (8, 6.0), (12, 0.5), (12, 1.9)])
 def test_flat_and_far(ctx, no_device_errors, level, height, axis):
