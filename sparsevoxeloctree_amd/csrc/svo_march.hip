@@ -263,7 +263,8 @@ __device__ __forceinline__ bool march_trip(const uint32_t *__restrict__ oct, uin
 //    pos * t_coef - t_bias is monotone in pos;
 //  - no value is NaN, so the selects of gmin are v_min3 (a zero's sign changes no record), and at
 //    least one axis steps in every advance, so the loop ends;
-//  - half * t_coef is exact (a power of two times a normal number), so t_center is one fma;
+//  - half * t_coef is exact (|t_coef| >= 2^-112, half >= 2^-13: its last bit is a denormal's at least), so
+//    t_center is one fma;
 //  - a word is loaded in every trip (an empty cell's word is 0), so iter counts the loads too;
 //  - the child slot is bit `scale` of the three coordinates, and the advance pops exactly when the
 //    highest bit it changes lies above `scale`.
@@ -271,7 +272,8 @@ __device__ __forceinline__ bool march_trip(const uint32_t *__restrict__ oct, uin
 // non-empty word: internal with its 8 children below W (limit = lean_limit) against leaf, or a
 // pointer out of range, or a word without the non-empty bit.  lean_odd recognises the last two, and a
 // descent below the stack's last slot; such a ray is marched again by march_step, which raises the
-// error bits.  102 -> 60 VALU instructions over the loop's paths; march_step alone against this loop:
+// error bits.  A ray that is not lean goes on with march_step from its set-up: most of them miss the
+// cube and need few trips (2560x1440 with the room far away 112 us when set up twice, 104 so).  102 -> 60 VALU instructions over the loop's paths; march_step alone against this loop:
 // room at 1920x1080 march 177 -> 130 us and beam 82 -> 68 us, 2M bounce rays 360 -> 283 us, a path
 // tracer sample at 1283x719 1175 -> 860 us.
 struct LeanOctree {
@@ -285,7 +287,7 @@ __device__ __forceinline__ LeanOctree lean_octree(const uint32_t *oct, uint64_t 
 	return LeanOctree{oct, (int32_t)(0x80000000u + (W32 - 8u)), (W32 - 8u) << 2u, W32 >= 8u};
 }
 __device__ __forceinline__ bool lean_axis(float t_coef, float t_bias) {
-	return fabsf(t_coef) >= 0x1p-60f && fabsf(t_bias) < __builtin_inff(); // false for NaN
+	return fabsf(t_coef) >= 0x1p-112f && fabsf(t_bias) < __builtin_inff(); // false for NaN
 }
 __device__ __forceinline__ bool lean_ray(const LeanOctree &t, const March &m) {
 	return t.ok && m.t_min <= m.t_max && lean_axis(m.t_coef.x, m.t_bias.x) && lean_axis(m.t_coef.y, m.t_bias.y) &&
@@ -374,15 +376,22 @@ __device__ __forceinline__ void march_leaf(const uint32_t *__restrict__ oct, uin
 	uint32_t nfetch = 0u, iter = 0u;
 	march_init<kVariant != 0>(o, d, m);
 	const LeanOctree t = lean_octree(oct, W);
-	bool general = !lean_ray(t, m);
-	if (!general) {
+	bool lean = lean_ray(t, m);
+	if (lean) {
 		while (lean_trip<false, kStride>(t, m, stk, iter, 0.0f, 0.0f)) {
 		}
-		general = lean_odd(t, m, iter);
 		nfetch = iter;
+		if (__builtin_expect(lean_odd(t, m, iter), 0)) {
+			march_init<kVariant != 0>(o, d, m);
+			iter = nfetch = 0u;
+			lean = false;
+		}
 	}
-	if (__builtin_expect(general, 0))
-		march_general<kVariant != 0, kStride>(oct, W, o, d, m, stk, iter, nfetch, err);
+	if (!lean) {
+#pragma unroll 1
+		while (march_trip<kStride>(oct, W, m, stk, iter, nfetch, err)) {
+		}
+	}
 	march_finish<kVariant>(m, o, d, iter, nfetch, out0, out1);
 }
 
@@ -437,17 +446,18 @@ __device__ __forceinline__ float beam_cell(const uint32_t *__restrict__ oct, uin
 	march_init<false>(o, d, m);
 	const LeanOctree t = lean_octree(oct, W);
 	uint32_t iter = 0u;
-	bool general = !lean_ray(t, m);
-	if (!general) {
+	bool lean = lean_ray(t, m);
+	if (lean) {
 		while (lean_trip<true, kStride>(t, m, stk, iter, orig_sz, dir_sz)) {
 		}
-		general = lean_odd(t, m, iter);
 		nfetch = iter;
+		if (__builtin_expect(lean_odd(t, m, iter), 0)) {
+			march_init<false>(o, d, m);
+			iter = nfetch = 0u;
+			lean = false;
+		}
 	}
-	if (__builtin_expect(general, 0)) {
-		iter = nfetch = 0u;
-		march_init<false>(o, d, m);
-#pragma unroll 1
+	if (!lean) {
 		for (;;) {
 			if (m.scale >= kStackSize) // after a push below the stack's last slot
 				break;

@@ -202,3 +202,23 @@ def test_ray_pool_sizes_match_oracle(ctx, no_device_errors, R):
     for k, got in enumerate(march_all(ctx, octree, rays, 0)):
         ok, msg = hits_equal(got, ref)
         assert ok, "form %d: %s" % (k, msg)
+
+
+@pytest.mark.parametrize("power", [60, 61, 100, 111, 112, 113, 120, -112, -149])
+@pytest.mark.parametrize("variant", [0, 1, 2])
+def test_direction_lengths_match_oracle(ctx, no_device_errors, power, variant):
+    # directions of length 2^power: from 2^112 on the reciprocals are too small for the fast loop
+    import sparsevoxeloctree_amd as S
+
+    words = scene_words(ctx)
+    octree = S.Octree.FromWords(ctx, words, 6)
+    rng = np.random.default_rng(200 + power)
+    o = rng.uniform(0.5, 2.5, (2000, 3))
+    d = rng.normal(size=(2000, 3))
+    d *= 2.0 ** (power + rng.integers(0, 2, (2000, 1))) / np.linalg.norm(d, axis=1, keepdims=True)
+    rays = np.concatenate([o, d], axis=1).astype(np.float32)
+    ref = oracle.march_rays(words, 6, rays, variant)
+    print("direction lengths", power, variant, flush=True)
+    for k, got in enumerate(march_all(ctx, octree, rays, variant)):
+        ok, msg = hits_equal(got, ref)
+        assert ok, "form %d: %s" % (k, msg)
