@@ -651,8 +651,10 @@ __global__ void __launch_bounds__(kBlock)
 // arithmetic as the one-ray-per-lane kernels, so the records are identical.
 // 2M bounce rays in the room at 2^10: 250 us, against 380 one ray per lane and 283 with a grid that just
 // fills the GPU and a fixed share of the rays per wave (80 VGPRs); pools of 512 / 2048 rays 302 / 278,
-// 8 / 32 trips 265 / 280, 8 / 32 idle lanes 252 / 264.  Frames gain nothing from refills (a bigger pool
-// only lowers the number of waves): 256 rays, i.e. a 16x16 tile, 1920x1080 150 us.
+// 8 / 32 trips 265 / 280, 8 / 32 idle lanes 252 / 264.  Fewer rays make smaller pools, so that there are 4
+// blocks per CU: random rays over slivers at 2^10, 20,000: 512 us in pools of 1024, 260 in pools of 256;
+// 400,000: 508 / 418 / 397 in pools of 1024 / 512 / 256; 1M: 708 / 768 / 794.  Frames gain nothing from
+// refills (a bigger pool only lowers the number of waves): 256 rays, i.e. a 16x16 tile, 1920x1080 150 us.
 constexpr uint32_t kRefill = 16; // idle lanes that trigger a refill
 
 // Ray sources: ray(k, ...) sets up ray k (false: no ray, e.g. a pixel outside the frame), out(k) is
@@ -728,18 +730,19 @@ struct SegmentRays { // rays [rbeg[s], rbeg[s+1]) against octree s, per-segment 
 };
 
 template <int kVariant, uint32_t kT, class Src>
-__global__ void __launch_bounds__(kT) march_pool(Src src, uint64_t n, uint32_t *err_out) {
+__global__ void __launch_bounds__(kT) march_pool(Src src, uint64_t n, uint32_t pool, uint32_t *err_out) {
 	constexpr uint32_t kPool = Src::kPool;
 	__shared__ uint32_t s_stack[kStackSlots * kT];
 	__shared__ float s_ray[6 * kT]; // origin and direction of the lane's ray, for its record
 	__shared__ uint32_t s_general[kPool / 32u];
+	static_assert(kPool <= 6u * kT, "the list of the general rays");
 	__shared__ uint32_t s_next;
 	uint32_t *stk = s_stack + threadIdx.x;
 	float *park = s_ray + threadIdx.x;
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint64_t below = (1ull << lane) - 1ull;
-	const uint64_t base = (uint64_t)xcd_stripes<8>(blockIdx.x, gridDim.x) * kPool;
-	const uint32_t total = (uint32_t)(n - base < kPool ? n - base : kPool);
+	const uint64_t base = (uint64_t)xcd_stripes<8>(blockIdx.x, gridDim.x) * pool;
+	const uint32_t total = (uint32_t)(n - base < pool ? n - base : pool);
 	for (uint32_t i = threadIdx.x; i < kPool / 32u; i += kT)
 		s_general[i] = 0u;
 	if (threadIdx.x == 0u)
@@ -809,11 +812,19 @@ __global__ void __launch_bounds__(kT) march_pool(Src src, uint64_t n, uint32_t *
 			}
 		}
 	}
-	// the block's other rays, one per lane
+	// the block's other rays, one per lane, listed where the pool's were parked
 	__syncthreads();
-	for (uint32_t q = threadIdx.x; q < total; q += kT) {
-		if (!(s_general[q >> 5] >> (q & 31u) & 1u))
-			continue;
+	uint32_t *list = reinterpret_cast<uint32_t *>(s_ray);
+	if (threadIdx.x == 0u)
+		s_next = 0u;
+	__syncthreads();
+	for (uint32_t q = threadIdx.x; q < total; q += kT)
+		if (s_general[q >> 5] >> (q & 31u) & 1u)
+			list[atomicAdd(&s_next, 1u)] = q;
+	__syncthreads();
+	const uint32_t others = s_next;
+	for (uint32_t i = threadIdx.x; i < others; i += kT) {
+		const uint32_t q = list[i];
 		f3 o, d;
 		const uint32_t *oct;
 		uint64_t W;
@@ -1617,7 +1628,11 @@ const char *const kScheduleName[4] = {"one-ray-per-lane", "refill", "one-ray-per
 // Refill march of n rays from src; name is the profiler's name of the march.
 template <int kVariant, class Src>
 hipError_t launch_pool(svo_ctx *ctx, const char *name, const Src &src, uint64_t n) {
-	return launch(ctx, name, march_pool<kVariant, kBlock, Src>, dim3(div_up(n, Src::kPool)), dim3(kBlock), 0, src, n,
+	const uint64_t fill = (uint64_t)ctx->cu_count * 4u;
+	uint32_t pool = kBlock;
+	while (pool < Src::kPool && pool * fill < n)
+		pool += kBlock;
+	return launch(ctx, name, march_pool<kVariant, kBlock, Src>, dim3(div_up(n, pool)), dim3(kBlock), 0, src, n, pool,
 	              ctx->d_err);
 }
 

@@ -222,3 +222,19 @@ def test_direction_lengths_match_oracle(ctx, no_device_errors, power, variant):
     for k, got in enumerate(march_all(ctx, octree, rays, variant)):
         ok, msg = hits_equal(got, ref)
         assert ok, "form %d: %s" % (k, msg)
+
+
+@pytest.mark.parametrize("R", [262144, 262145, 600001, 1000003])
+def test_ray_pool_grows_with_the_rays(ctx, no_device_errors, R):
+    # pools of 256 rays up to 4 blocks per CU, then of 512, 768 and 1024: against one ray per lane, with
+    # rays for the general loop among them
+    import sparsevoxeloctree_amd as S
+
+    octree = S.Octree.FromWords(ctx, scene_words(ctx), 6)
+    some = odd_rays(R, 8192)
+    rays = np.ascontiguousarray(some[np.random.default_rng(R).integers(0, len(some), R)])
+    print("ray pool growth", R, flush=True)
+    one, one_batch, pool, pool_batch = march_all(ctx, octree, rays, 0)
+    for got in (one_batch, pool, pool_batch):
+        ok, msg = hits_equal(got, one)
+        assert ok, msg
