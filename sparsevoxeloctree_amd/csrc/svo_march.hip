@@ -269,7 +269,7 @@ __device__ __forceinline__ bool march_trip(const uint32_t *__restrict__ oct, uin
 //  - the child slot is bit `scale` of the three coordinates, and the advance pops exactly when the
 //    highest bit it changes lies above `scale`.
 // m.parent is a byte offset here: cur << 2 drops the two flag bits.  One signed compare splits a
-// non-empty word: internal with its 8 children below W (limit = lean_limit) against leaf, or a
+// non-empty word: internal with its 8 children below W (LeanOctree::limit) against leaf, or a
 // pointer out of range, or a word without the non-empty bit.  lean_odd recognises the last two, and a
 // descent below the stack's last slot; such a ray is marched again by march_step, which raises the
 // error bits.  A ray that is not lean goes on with march_step from its set-up: most of them miss the
@@ -413,9 +413,11 @@ template <uint32_t kGroup> __device__ __forceinline__ uint32_t xcd_stripes(uint3
 	return (k / kGroup * 8u + (b & 7u)) * kGroup + k % kGroup;
 }
 // The same with one contiguous band of the range per XCD: less of the octree is read by two XCDs, but
-// XCDs with a cheap band idle.  8x8-tile marches, bands -> stripes of 64 tiles: 3840x2160 over slivers at
-// 2^12 3950 -> 2890 us, 1920x1080 over spheres at 2^10 157 -> 133 us, 2560x1440 in the room at 2^11
-// 196 -> 111 us, but 1920x1080 in the room at 2^10 127 -> 137 us (stripes of 1..64 tiles within 3%).
+// XCDs with a cheap band idle.  Which one wins depends on the view, so bands are a candidate of the
+// autotuner only: of 54 views of the room at 2^9 to 2^11 they were the fastest schedule in 17, all of
+// 1920x1080 or less, by up to 15% (1920x1080 at 2^10: 142 us, 166 in stripes), and in others slower by up
+// to 21%.  From 2560x1440 on and over scattered small geometry stripes win (3840x2160 over slivers at
+// 2^12 2890 us against 3950; stripes of 1..64 tiles within 3%).
 __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nblocks) {
 	const uint32_t per = (nblocks + 7u) / 8u;
 	const uint32_t full = nblocks - (per - 1u) * 8u; // XCDs that get `per` blocks
@@ -1671,7 +1673,7 @@ namespace {
 
 // The primary march of a frame (and its beam pre-pass when beam_img is not null, written there).
 // may_tune: the autotuner may time the candidate schedules of a new shape class; without it the
-// schedule is the context's fixed one, or one ray per lane in 16x16 tiles.  timed: bracket the
+// schedule is the context's fixed one, or one ray per lane in one-wave 8x8 tiles.  timed: bracket the
 // passes with the context's stage timers.
 int march_frame_into(svo_ctx *ctx, const svo_octree *oct, const svo_camera *cam, uint32_t w, uint32_t h,
                      float *beam_img, svo_hit *hits, bool may_tune, bool timed = true) {
@@ -1960,7 +1962,7 @@ constexpr int kFrameShapes = 4;
 const char *const kFrameShapeName[kFrameShapes] = {"16x16", "8x8", "16x8", "32x8"};
 constexpr uint32_t kShapeWX[kFrameShapes] = {2, 1, 2, 4};
 constexpr uint32_t kShapeWY[kFrameShapes] = {2, 1, 1, 1};
-// ray-batch schedules: one ray per lane in blocks of 256 / 128 / 64 threads, or persistent refill
+// ray-batch schedules: one ray per lane in blocks of 256 / 128 / 64 threads, or refill
 constexpr int kRayShapes = 4;
 constexpr uint32_t kRayBlock[3] = {256, 128, 64};
 
@@ -2146,7 +2148,7 @@ int march_rays_segments(svo_ctx *ctx, const svo_octree *const *octs, const float
 		return bs == 256 ? SVO_RAYS(2, 256) : bs == 128 ? SVO_RAYS(2, 128) : SVO_RAYS(2, 64);
 #undef SVO_RAYS
 	};
-	// an explicit schedule (svo_march_mode 1: persistent; 0, 2: one ray per lane in blocks of 256),
+	// an explicit schedule (svo_march_mode 1: refill; 0, 2: one ray per lane in blocks of 256),
 	// else the autotuner's choice among the four
 	int shape = ctx->march_mode == 1 ? 3 : 0;
 	if (!rc && ctx->march_mode < 0 && ctx->autotune) {
@@ -2155,7 +2157,7 @@ int march_rays_segments(svo_ctx *ctx, const svo_octree *const *octs, const float
 			++lg;
 		char key[96];
 		std::snprintf(key, sizeof key, "march_rays_batch variant=%d R~2^%u", variant, lg);
-		static const char *const names[kRayShapes] = {"block256", "block128", "block64", "persistent-refill"};
+		static const char *const names[kRayShapes] = {"block256", "block128", "block64", "refill"};
 		rc = tune(ctx, key, kRayShapes, names, run, shape);
 	}
 	if (!rc) {

@@ -227,10 +227,12 @@ void svo_server::ray_loop() {
 }
 
 // Voxelize + build of a batch of build requests.  The batch is voxelized once; it is then built in
-// consecutive groups whose transient build scratch (20 B per fragment plus bitmaps and ranks) fits
-// the byte budget after evicting idle octrees: a group that does not fit is halved, and a single
-// scene that does not fit even alone is rejected (SVO_ERR_OUT_OF_MEMORY).  A voxelize failure of
-// the whole batch retries each request alone, so that one bad scene cannot fail the others.
+// consecutive groups whose transient build scratch fits the byte budget after evicting idle octrees:
+// a group that does not fit is halved, and a single scene that does not fit even alone is rejected
+// (SVO_ERR_OUT_OF_MEMORY).  The scratch is estimated at 20 B per fragment (tiles and runs take 12.1,
+// buckets 4, lists 0.7, counters 8 per leaf block; a scene's last, partial tile, 12 KB at most, is
+// left out) plus bitmaps and ranks.  A voxelize failure of the whole batch retries each request
+// alone, so that one bad scene cannot fail the others.
 void svo_server::build_batch_requests(std::vector<Request *> &batch) {
 	const uint32_t n = (uint32_t)batch.size();
 	std::vector<const svo_scene *> scenes(n);

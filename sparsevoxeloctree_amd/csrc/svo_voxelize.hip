@@ -344,8 +344,8 @@ __device__ __forceinline__ void wave_sync() {
 __global__ void vox_zero_counter(uint32_t *c) { c[0] = 0u; }
 
 // Count pass: a lane walks its triangle's rows.  A few tall triangles in a wave of flat ones are
-// instead taken by the whole wave, a row per lane; so are those in the general form, after the others
-// (in a loop of its own: it needs the registers).  `general` lists the latter, [0] is their number.
+// instead taken by the whole wave, a row per lane; so are those in the general form that can cover a
+// pixel, after the others (in a loop of its own: it needs the registers).  `general` lists the latter, [0] is their number.
 // Bound by VALU issue (1.0 busy, a third of it the triangles' setup): 990,800 triangles of a room at
 // 2^10 65 -> 22 us, 8.0M with slivers at 2^12 465 -> 108 us, against 64-bit integers with a division
 // per edge side; 870 triangles of 500 rows 56 -> 7 us by the wave-wide walk.
