@@ -666,6 +666,35 @@ def copy_calibration(mib):
                           "avg_ms": ms / cnt, "gbs": 2 * n / (ms / cnt * 1e-3) / 1e9}))
 
 
+def kernel_of(label, report):
+    """The kernel behind a launch label of the profiler, as rocprofv3 names it.  A march has one per
+    schedule: the tuner's report (lines "key: trials -> choice") says which ran, else the defaults."""
+    key = {"march_rays6": "march_rays variant=0 ", "march_rays5": "march_rays variant=1 ",
+           "march_occlude": "march_rays variant=2 ", "march_frame": "march_frame "}.get(label)
+    if key is None:
+        return {"bounce": "bounce_kernel", "march_beam": "march_beam_kernel",
+                "build_fold": "build_fold<false>"}.get(label, label)
+    choice = [line.rpartition(" -> ")[2] for line in report if line.startswith(key)]
+    if label == "march_frame":
+        return {"one-ray-per-lane": "march_frame_kernel<2u,2u,false>", "refill": "march_pool<0,256u,FrameRays>",
+                "one-ray-per-lane-8x8": "march_frame_kernel<1u,1u,false>",
+                "one-ray-per-lane-8x8-bands": "march_frame_kernel<1u,1u,true>"}[(choice or ["one-ray-per-lane-8x8"])[-1]]
+    variant = key.split("=")[1].strip()
+    refill = bool(choice) and choice[-1] == "refill"
+    return ("march_pool<%s,256u,ExplicitRays>" if refill else "march_rays_kernel<%s>") % variant
+
+
+def counter(kind, label, cid, kernel, field):
+    """A recorded hardware counter of a launch label in workload c<cid>; None unless it was recorded
+    for the kernel that runs under that label now."""
+    path = os.path.join(ROOT, "profiles", "%s_%s_c%d.json" % (kind, label, cid))
+    if not os.path.exists(path):
+        return None
+    with open(path) as f:
+        rec = json.load(f)
+    return rec.get(field) if rec.get("rocprof_name") == kernel else None
+
+
 def bench_primary(args, cfg, cpu=True):
     """One single-scene configuration (c1, c2 or c3): args.warmup untimed and args.steps timed steps
     of voxelize + build + march (+ the bounce for c2); returns the result line."""
@@ -675,7 +704,7 @@ def bench_primary(args, cfg, cpu=True):
     T = rgb.shape[0]
     cam = make_camera(S, cfg, xyz)
     ctx = S.Context(0)
-    # launch schedules (one ray per lane / persistent refill) picked per shape class by the
+    # launch schedules (one ray per lane / refill) picked per shape class by the
     # library's autotuner during the warm-up steps
     S.autotune(ctx, True)
     scene = S.Scene.Create(ctx, xyz, rgb, normalize=True)
@@ -771,18 +800,12 @@ def bench_primary(args, cfg, cpu=True):
     roofline = None
     if dominant in alg:
         achieved = alg[dominant] / (kernel_ms[dominant] * 1e-3) / 1e9
-        traffic = valu_busy = None
         cid = next(k for k, v in CONFIGS.items() if v is cfg)
-        tpath = os.path.join(ROOT, "profiles", "traffic_%s_c%d.json" % (dominant, cid))
-        if os.path.exists(tpath):
-            with open(tpath) as f:
-                traffic = json.load(f).get("bytes_per_launch")
+        kernel = kernel_of(dominant, S.autotune(ctx, True).strip().splitlines())
+        traffic = counter("traffic", dominant, cid, kernel, "bytes_per_launch")
         # VALU busy of the same kernel from the SQ counter pass (a march is bound by VALU issue,
         # so its HBM fraction alone says little)
-        vpath = os.path.join(ROOT, "profiles", "valu_%s_c%d.json" % (dominant, cid))
-        if os.path.exists(vpath):
-            with open(vpath) as f:
-                valu_busy = json.load(f).get("valu_busy")
+        valu_busy = counter("valu", dominant, cid, kernel, "valu_busy")
         roofline = {
             "kernel": dominant,
             "bound": "hbm",
