@@ -346,9 +346,9 @@ __global__ void vox_zero_counter(uint32_t *c) { c[0] = 0u; }
 // Count pass: a lane walks its triangle's rows.  A few tall triangles in a wave of flat ones are
 // instead taken by the whole wave, a row per lane; so are those in the general form that can cover a
 // pixel, after the others (in a loop of its own: it needs the registers).  `general` lists the latter, [0] is their number.
-// Bound by VALU issue (1.0 busy, a third of it the triangles' setup): 990,800 triangles of a room at
-// 2^10 65 -> 22 us, 8.0M with slivers at 2^12 465 -> 108 us, against 64-bit integers with a division
-// per edge side; 870 triangles of 500 rows 56 -> 7 us by the wave-wide walk.
+// Bound by VALU issue (1.0 busy with slivers, a third of it the triangles' setup): 990,800 triangles
+// of a room at 2^10 65 -> 22 us, 8.0M with slivers at 2^12 465 -> 108 us, against 64-bit integers with
+// a division per edge side; 870 triangles of 500 rows 56 -> 7 us by the wave-wide walk.
 constexpr int32_t kTallRows = 32;
 
 __global__ void __launch_bounds__(kThreads)
@@ -488,8 +488,8 @@ using FragOut = __attribute__((address_space(1))) uint64_t;
 // its place and its triangle's parameters in LDS, and writes: even work and whole lines, whatever the
 // triangles' shapes.  Rows are walked a triangle per lane, or, where a window holds few triangles (tall
 // ones, or of many fragments), a row per lane.
-// Bound by VALU issue (0.9 busy; per 64 fragments 46 instructions, and 25 per row of the tallest
-// triangle of a window): 35M fragments of a room at 2^10 245 -> 116 us, 173M with slivers at 2^12
+// Bound by VALU issue (0.7 busy in a room, 1.0 with slivers; per 64 fragments 46 instructions, and 25
+// per row of the tallest triangle of a window): 35M fragments of a room at 2^10 245 -> 116 us, 173M with slivers at 2^12
 // 1472 -> 560 us, 32 mixed scenes 990 -> 396 us, against a triangle per lane writing its own fragments
 // and a block per triangle above 128 of them; where few triangles hold most (room of 220,848 at 2^11,
 // 54M fragments) 659 -> 153 us.  Windows of 512 / 1024: 598 / 576 us with slivers, 404 / 415 the batch.
